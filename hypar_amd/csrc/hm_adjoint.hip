@@ -65,15 +65,6 @@ __device__ __forceinline__ LineSlot line_slot(size_t item, int n, size_t nlines)
   return s;
 }
 
-// 1/d, d > 0 and normal: hardware estimate and two Newton-Raphson steps
-__device__ __forceinline__ double vjp_rcp(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  double e = __builtin_fma(-d, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-d, r, 1.0);
-  return __builtin_fma(r, e, r);
-}
-
 // one side of a WENO5 interpolation from its smoothness indicators beta_k
 // and candidate values f_k: the interpolated value, the weights, ob times
 // d out/d beta_k (g1..g3) and, for the YC weights, ob times d out/d tau (gt)
@@ -112,7 +103,7 @@ __device__ __forceinline__ W5Side w5_side(double b1, double b2, double b3, doubl
   } else if (W == WENO_JS) {
     const double a1 = 0.1 * (s2 * s3), a2 = 0.6 * (s1 * s3), a3 = 0.3 * (s1 * s2);
     const double A = a1 + a2 + a3, e23 = e2 * e3, P = e1 * e23;
-    const double q = vjp_rcp(A * P);
+    const double q = nr_rcp(A * P);
     const double inv = q * P, k = -2.0 * ob * (q * A);
     r.w1 = a1 * inv;
     r.w2 = a2 * inv;
@@ -126,7 +117,7 @@ __device__ __forceinline__ W5Side w5_side(double b1, double b2, double b3, doubl
     const double p1 = s2 * s3, p2 = s1 * s3, p3 = s1 * s2;  // products of the other two s_k
     const double a1 = 0.1 * (s1 + t2) * p1, a2 = 0.6 * (s2 + t2) * p2, a3 = 0.3 * (s3 + t2) * p3;
     const double A = a1 + a2 + a3, e23 = e2 * e3, P = e1 * e23;
-    const double q = vjp_rcp(A * P);
+    const double q = nr_rcp(A * P);
     const double inv = q * P;
     r.w1 = a1 * inv;
     r.w2 = a2 * inv;
@@ -151,7 +142,7 @@ __device__ __forceinline__ W5Side w5_side(double b1, double b2, double b3, doubl
     const double c1 = 0.1, c2 = 0.6, c3 = 0.3;
     const double at1 = c1 * (s2 * s3), at2 = c2 * (s1 * s3), at3 = c3 * (s1 * s2);
     const double At = at1 + at2 + at3, e23 = e2 * e3, P = e1 * e23;
-    const double q = vjp_rcp(At * P);
+    const double q = nr_rcp(At * P);
     const double it = q * P;
     const double u1 = at1 * it, u2 = at2 * it, u3 = at3 * it;  // JS weights
     const double N1 = c1 + c1 * c1 - 3 * c1 * u1 + u1 * u1, D1 = c1 * c1 + u1 * (1.0 - 2.0 * c1);
@@ -159,7 +150,7 @@ __device__ __forceinline__ W5Side w5_side(double b1, double b2, double b3, doubl
     const double N3 = c3 + c3 * c3 - 3 * c3 * u3 + u3 * u3, D3 = c3 * c3 + u3 * (1.0 - 2.0 * c3);
     const double o1 = D2 * D3, o2 = D1 * D3, o3 = D1 * D2, DD = D1 * o1;
     const double B1 = u1 * N1 * o1, B2 = u2 * N2 * o2, B3 = u3 * N3 * o3, B = B1 + B2 + B3;
-    const double qm = vjp_rcp(B * DD);
+    const double qm = nr_rcp(B * DD);
     const double im = qm * DD;
     r.w1 = B1 * im;
     r.w2 = B2 * im;
@@ -1453,12 +1444,11 @@ __global__ void __launch_bounds__(256) k_ens_vjp_prims(EnsVjp a, size_t ncell) {
     double s[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) s[v] = a.u[5 * M.off + (size_t)v * M.ncell + c];
-    const Prim q = flowvar(s, a.gamma);
+    double q[4];
+    visc_prims(s, a.gamma, q);
     double *Q = a.work + 20 * M.off;
-    Q[c] = q.vx;
-    Q[M.ncell + c] = q.vy;
-    Q[2 * M.ncell + c] = q.vz;
-    Q[3 * M.ncell + c] = a.gamma * q.P / q.rho;
+#pragma unroll
+    for (int v = 0; v < 4; v++) Q[(size_t)v * M.ncell + c] = q[v];
   });
 }
 

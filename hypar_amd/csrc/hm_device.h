@@ -41,6 +41,47 @@ __device__ __forceinline__ Prim flowvar(const double *u, double gamma) {
   return q;
 }
 
+// 1/d, d > 0 and normal: hardware estimate refined by two Newton-Raphson
+// steps, each of which squares the relative error.
+__device__ __forceinline__ double nr_rcp(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  double e = __builtin_fma(-d, r, 1.0);
+  r = __builtin_fma(r, e, r);
+  e = __builtin_fma(-d, r, 1.0);
+  return __builtin_fma(r, e, r);
+}
+
+// 1/sqrt(d), d > 0 and normal: hardware estimate r, then r + r e (1/2 + 3/8 e)
+// with e = 1 - d r^2, which leaves an error of the order e^3, and once more
+// r + r e / 2 for the last bits.
+__device__ __forceinline__ double nr_rsq(double d) {
+  double r = __builtin_amdgcn_rsq(d);
+  double e = __builtin_fma(-d * r, r, 1.0);
+  r = __builtin_fma(r * e, __builtin_fma(0.375, e, 0.5), r);
+  e = __builtin_fma(-d * r, r, 1.0);
+  return __builtin_fma(0.5 * r, e, r);
+}
+
+// sqrt(d) from r = nr_rsq(d): d r with one correction by the residual d - s^2
+__device__ __forceinline__ double sqrt_of(double d, double r) {
+  const double s = d * r;
+  const double t = __builtin_fma(__builtin_fma(-s, s, d), 0.5 * r, s);
+  return d == 0.0 ? 0.0 : t;
+}
+__device__ __forceinline__ double nr_sqrt(double d) { return sqrt_of(d, nr_rsq(d)); }
+
+// primitive variables u, v, w, T = gamma P / rho of the viscous term
+// (NavierStokes3DParabolicFunction.c:85-108)
+__device__ __forceinline__ void visc_prims(const double *u, double gamma, double q[4]) {
+  const double ir = nr_rcp(u[0]);
+  const double iv = u[0] == 0.0 ? 0.0 : ir;
+  q[0] = u[1] * iv;
+  q[1] = u[2] * iv;
+  q[2] = u[3] * iv;
+  const double P = (u[4] - 0.5 * u[0] * (q[0] * q[0] + q[1] * q[1] + q[2] * q[2])) * (gamma - 1.0);
+  q[3] = gamma * P * ir;
+}
+
 template <int DIR> __device__ __forceinline__ double vel(const Prim &q) {
   return DIR == 0 ? q.vx : (DIR == 1 ? q.vy : q.vz);
 }

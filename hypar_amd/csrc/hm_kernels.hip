@@ -448,11 +448,10 @@ __global__ void __launch_bounds__(256) k_ens_prims(const EnsMember *__restrict__
   double s[NV];
 #pragma unroll
   for (int v = 0; v < NV; v++) s[v] = um[(size_t)v * M.ncell + c];
-  const Prim q = flowvar(s, gamma);
-  M.q[c] = q.vx;
-  M.q[M.ncell + c] = q.vy;
-  M.q[2 * M.ncell + c] = q.vz;
-  M.q[3 * M.ncell + c] = gamma * q.P / q.rho;
+  double q[4];
+  visc_prims(s, gamma, q);
+#pragma unroll
+  for (int v = 0; v < 4; v++) M.q[(size_t)v * M.ncell + c] = q[v];
 }
 
 // ---------------------------------------------------------------------------

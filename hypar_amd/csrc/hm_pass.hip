@@ -29,23 +29,37 @@
 //
 // Restatements relative to the reference arithmetic (equal in exact
 // arithmetic; rounding-level differences only):
-//  * 1/rho, the Jiang-Shu normalisation and the Roe-average weights use a
-//    Newton-Raphson-refined reciprocal (two steps r <- r + r(1 - d r) from
-//    the hardware estimate); velocities are m * (1/rho).
+//  * 1/rho, the weights' normalisation, the Roe-average weights and the
+//    square roots use hardware estimates refined to full precision (nr_rcp,
+//    nr_rsq); velocities are m * (1/rho).
 //  * The mass flux of a cell is its momentum m_d (the reference forms
 //    rho * (m_d / rho)).
-//  * The smoothness indicators are evaluated as 4*beta with 4*eps, which
-//    scales every (beta_k + eps)^2 by 16 and leaves the weights unchanged;
-//    the second differences shared by the left- and right-biased
-//    indicators of an interface are formed once.
+//  * An interpolated value is the value of the cell next to the interface
+//    plus a correction formed from first differences (weno5_lr).
+//  * The values the solution's interpolant takes are u itself: the modified
+//    solution P/(gamma-1) + rho |v|^2/2 that the reference interpolates
+//    (NavierStokes3DModifiedSolution.c:31-70, gravity 0) is u's energy.
+//  * What depends on one cell alone (the factors of the Roe average, the
+//    Rusanov speed) is formed once per cell; s H = (e + P)/s with s = sqrt(rho).
 //  * The characteristic projections use the structure of the left
 //    eigenvectors (navierstokes3d.h:288-374): with
 //    w = v.x_{1..3} - x_4, rows 0, d and 4 are
-//      L00 x0 + (g-1)/a^2 w,  Ld0 x0 - (g-1)/(2a^2) w -/+ a/(2a^2) x_d,
+//      L00 x0 + (g-1)/a^2 w,  Ld0 x0 - (g-1)/(2a^2) w -/+ 1/(2a) x_d,
 //    and the two shear rows have two non-zero entries; the product with the
 //    right eigenvectors (navierstokes3d.h:384-470) is expanded the same
 //    way.  The speed of sound of the Roe state is sqrt((g-1)(H - |v|^2/2)),
 //    the reference's sqrt(g P / rho) with P from H.
+//  * Only differences between cells are projected; the mean of the two
+//    cells' fluxes passes L and R unchanged (L R = I).
+//
+// FP64 issue bounds these passes: a wave64 FP64 instruction takes a SIMD 4
+// cycles, and two waves per SIMD hide the rest to about 60%.  The forms above
+// take 946 FP64 (1050 VALU) instructions per interface of the characteristic
+// JS/Roe x pass and 744 (843) of the component-wise JS/Rusanov one, where
+// weights from second and one-sided differences, projected values and
+// Roe averages formed at each interface took 1356 (1474) and 1072 (1188):
+// 256^3 RK4 step 15.55 -> 13.54 ms, 201^3 SSPRK3/YC step 5.20 -> 4.18 ms,
+// 64-member Euler ensemble 18.7 -> 15.2 ms per step.
 #include <hip/hip_runtime.h>
 
 #include "hm_device.h"
@@ -55,23 +69,16 @@ namespace hm {
 
 namespace {
 
-constexpr int NQ = 10;  // per-cell LDS data: U0..U4, F1..F4 (F0 = U_d), modified energy
-
-
-// 1/d, d > 0 and normal: hardware estimate refined by two Newton-Raphson
-// steps, each of which squares the relative error.
-__device__ __forceinline__ double nr_rcp(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  double e = __builtin_fma(-d, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-d, r, 1.0);
-  return __builtin_fma(r, e, r);
-}
+// per-cell LDS record: U0..U4, F1..F4 (F0 = U_d), 1/sqrt(rho), sqrt(rho) H
+// and, for Rusanov upwinding, the cell's speed c + |v_d|.  What an interface
+// needs of one cell alone (the factors of the Roe average, the speed) is so
+// formed once per cell and not at both of its interfaces.
+constexpr int nq(int upw) { return upw == UPWIND_RUSANOV ? 12 : 11; }
 
 struct PassConst {
   int n[3];
   size_t ncell;
-  double gamma, gm1, inv_gm1, eps4;
+  double gamma, gm1, inv_gm1, eps34;  // eps34 = 3/4 of the WENO epsilon
   const double *dxg;  // ghosted dxinv x|y|z
 };
 
@@ -102,12 +109,11 @@ struct SspIO {
   int nout;  // outputs stored: O1, then O2 (nout >= 2), then O3 (nout = 3)
 };
 
-// per-cell data of the pass direction (NavierStokes3DFlux.c:23-57 and
-// NavierStokes3DModifiedSolution.c:31-70)
-template <int DIR>
-__device__ __forceinline__ void cell_data(const double u[NV], const PassConst &k, double c[NQ]) {
+// per-cell record of the pass direction (NavierStokes3DFlux.c:23-57)
+template <int DIR, int UPW>
+__device__ __forceinline__ void cell_data(const double u[NV], const PassConst &k, double c[nq(UPW)]) {
   const double rho = u[0];
-  const double ir = rho == 0.0 ? 0.0 : nr_rcp(rho);
+  const double ir = rho == 0.0 ? 0.0 : nr_rcp(rho), is = rho == 0.0 ? 0.0 : nr_rsq(rho);
   const double vx = u[1] * ir, vy = u[2] * ir, vz = u[3] * ir;
   const double vsq = vx * vx + vy * vy + vz * vz;
   const double P = (u[4] - 0.5 * rho * vsq) * k.gm1;
@@ -119,52 +125,53 @@ __device__ __forceinline__ void cell_data(const double u[NV], const PassConst &k
   c[6] = m * vy + (DIR == 1 ? P : 0.0);
   c[7] = m * vz + (DIR == 2 ? P : 0.0);
   c[8] = (u[4] + P) * vn;
-  c[9] = (P * k.inv_gm1) + (0.5 * rho * vsq);
+  c[9] = is;
+  c[10] = (u[4] + P) * is;
+  if (UPW == UPWIND_RUSANOV) c[11] = nr_sqrt(k.gamma * P * ir) + fabs(vn);
 }
 
-// WENO5 on both sides of one interface.  b[0..5] are the values of cells
-// I-3..I+2 the smoothness indicators use, g[0..5] the values that are
-// interpolated (include/interpolation.h:265-500,
-// Interp1PrimFifthOrderWENO.c:146-158; the right-biased stencil is the
-// mirror image, WENOFifthOrderCalculateWeights.c:166-177).  The indicators
-// arrive scaled by 4 (l1..l3 = 4 beta_k) together with eps4 = 4 eps; W
-// selects the weights:
+// A constant held in scalar registers: without it the compiler folds the
+// constant into the two-address fused multiply-add and copies the addend
+// first (one extra instruction each time).
+__device__ __forceinline__ double scalar(double c) {
+  asm("" : "+s"(c));
+  return c;
+}
+
+// One side of WENO5 at an interface: twice the difference between the
+// interpolated value and the value of the upwind cell next to the interface
+// (include/interpolation.h:265-500, Interp1PrimFifthOrderWENO.c:146-158).
+// l1..l3 = 3/4 (beta_k + eps); p1..p3 = the candidates' differences from that
+// cell's value times 2, 12, 6 (the ratios 1, 6, 3 of the optimal weights);
+// d4 the stencil's 4th difference (YC).  W selects the weights:
 //  * WENO_JS:     a_k = c_k / (beta_k + eps)^2
 //  * WENO_Z:      a_k = c_k (1 + (tau / (beta_k + eps))^2), tau = |beta_1 - beta_3|
-//  * WENO_YC:     the same with tau = (m3 - 4 m2 + 6 m1 - 4 p1 + p2)^2
+//  * WENO_YC:     the same with tau = d4^2
 //  * WENO_MAPPED: the JS weights w mapped by
 //                 w (c + c^2 - 3 c w + w^2) / (c^2 + w (1 - 2c)) and renormalised
-// All are applied in ratio form with one reciprocal (two for the mapped).
+//  * WENO_OPTIMAL: the constant weights of no_limiting
+//    (WENOFifthOrderInitializeWeights.c:33-228, HyperbolicFunction.c:62)
+// The a_k are multiplied through by the product of all (beta_k + eps)^2 and
+// applied with one reciprocal (two for the mapped weights).
 template <int W>
-__device__ __forceinline__ double weno_combine(double l1, double l2, double l3, double d4, double g3, double g2,
-                                               double g1, double q1, double q2, double eps4) {
-  const double s6 = 1.0 / 6.0;
-  const double s1 = (l1 + eps4) * (l1 + eps4);
-  const double s2 = (l2 + eps4) * (l2 + eps4);
-  const double s3 = (l3 + eps4) * (l3 + eps4);
-  const double f1 = (2 * s6) * g3 + (-7 * s6) * g2 + (11 * s6) * g1;
-  const double f2 = (-s6) * g2 + (5 * s6) * g1 + (2 * s6) * q1;
-  const double f3 = (2 * s6) * g1 + (5 * s6) * q1 + (-s6) * q2;
-  // no_limiting: the weights stay at their optimal initial values
-  // (WENOFifthOrderInitializeWeights.c:33-228, HyperbolicFunction.c:62)
-  if (W == WENO_OPTIMAL) return 0.1 * f1 + 0.6 * f2 + 0.3 * f3;
-  double a1, a2, a3;
+__device__ __forceinline__ double weno_side(double l1, double l2, double l3, double p1, double p2, double p3,
+                                            double d4) {
+  if (W == WENO_OPTIMAL) return 0.1 * (p1 + p2 + p3);
+  const double q1 = l2 * l3, q2 = l1 * l3, q3 = l1 * l2;
+  double a1 = q1 * q1, a2 = q2 * q2, a3 = q3 * q3;
   if (W == WENO_Z || W == WENO_YC) {
-    // tau scales like beta for WENO-Z; the YC tau does not, hence 4 tau
-    const double tau = W == WENO_Z ? fabs(l3 - l1) : 4.0 * (d4 * d4);
+    // tau in the scale of l; the YC tau is formed from the data itself
+    const double tau = W == WENO_Z ? l3 - l1 : 0.75 * (d4 * d4);
     const double t2 = tau * tau;
-    a1 = 0.1 * ((s1 + t2) * (s2 * s3));
-    a2 = 0.6 * ((s2 + t2) * (s1 * s3));
-    a3 = 0.3 * ((s3 + t2) * (s1 * s2));
-  } else {
-    a1 = 0.1 * (s2 * s3);
-    a2 = 0.6 * (s1 * s3);
-    a3 = 0.3 * (s1 * s2);
+    a1 *= l1 * l1 + t2;
+    a2 *= l2 * l2 + t2;
+    a3 *= l3 * l3 + t2;
   }
+  const double k3 = scalar(3.0);
   if (W == WENO_MAPPED) {
     const double c1 = 0.1, c2 = 0.6, c3 = 0.3;
-    const double in = nr_rcp(a1 + a2 + a3);
-    const double w1 = a1 * in, w2 = a2 * in, w3 = a3 * in;
+    const double in = nr_rcp(a1 + k3 * (2.0 * a2 + a3));
+    const double w1 = a1 * in, w2 = a2 * (6.0 * in), w3 = a3 * (3.0 * in);
     const double n1 = w1 * (c1 + c1 * c1 - 3 * c1 * w1 + w1 * w1), e1 = c1 * c1 + w1 * (1.0 - 2.0 * c1);
     const double n2 = w2 * (c2 + c2 * c2 - 3 * c2 * w2 + w2 * w2), e2 = c2 * c2 + w2 * (1.0 - 2.0 * c2);
     const double n3 = w3 * (c3 + c3 * c3 - 3 * c3 * w3 + w3 * w3), e3 = c3 * c3 + w3 * (1.0 - 2.0 * c3);
@@ -172,35 +179,34 @@ __device__ __forceinline__ double weno_combine(double l1, double l2, double l3, 
     a1 = n1 * (e2 * e3);
     a2 = n2 * (e1 * e3);
     a3 = n3 * (e1 * e2);
+    return (a1 * p1 + a2 * ((1.0 / 6.0) * p2) + a3 * ((1.0 / 3.0) * p3)) * nr_rcp(a1 + a2 + a3);
   }
-  return (a1 * f1 + a2 * f2 + a3 * f3) * nr_rcp(a1 + a2 + a3);
+  return (a1 * p1 + a2 * p2 + a3 * p3) * nr_rcp(a1 + k3 * (2.0 * a2 + a3));
 }
 
+// WENO5 on both sides of one interface from the five first differences
+// D_s = b_{s+1} - b_s of cells I-3..I+2: the left-biased value is
+// b_2 + cl/2, the right-biased one (the mirror image,
+// WENOFifthOrderCalculateWeights.c:166-177) b_3 + cr/2.  With e the second
+// difference of a candidate stencil and x its first difference nearest the
+// interface, the smoothness indicators are
+//   3/4 beta = e^2 + 3/4 x (x + e)       (outer stencils; e towards x)
+//   3/4 beta = e^2 + 3/4 x y             (middle stencil, differences x, y),
+// equal to 13/16 e^2 + 3/16 (..)^2 of the textbook form: 21 operations for
+// all six with eps, where that form takes 38.
 template <int W>
-__device__ __forceinline__ void weno5_lr(const double (&b)[6], const double (&g)[6], double eps4, double &vl,
-                                         double &vr) {
-  const double c13 = 13.0 / 3.0;  // 4 * 13/12
-  const double d1 = b[0] - 2 * b[1] + b[2], d2 = b[1] - 2 * b[2] + b[3];
-  const double d3 = b[2] - 2 * b[3] + b[4], d4 = b[3] - 2 * b[4] + b[5];
-  const double q2 = c13 * (d2 * d2), q3 = c13 * (d3 * d3);
-  double e;
-  e = b[0] - 4 * b[1] + 3 * b[2];
-  const double l1 = c13 * (d1 * d1) + e * e;
-  e = b[1] - b[3];
-  const double l2 = q2 + e * e;
-  e = 3 * b[2] - 4 * b[3] + b[4];
-  const double l3 = q3 + e * e;
-  e = b[5] - 4 * b[4] + 3 * b[3];
-  const double r1 = c13 * (d4 * d4) + e * e;
-  e = b[4] - b[2];
-  const double r2 = q3 + e * e;
-  e = 3 * b[3] - 4 * b[2] + b[1];
-  const double r3 = q2 + e * e;
-  // 4th undivided differences of the two stencils (YC weights only)
-  const double tl = W == WENO_YC ? b[0] - 4 * b[1] + 6 * b[2] - 4 * b[3] + b[4] : 0.0;
-  const double tr = W == WENO_YC ? b[5] - 4 * b[4] + 6 * b[3] - 4 * b[2] + b[1] : 0.0;
-  vl = weno_combine<W>(l1, l2, l3, tl, g[0], g[1], g[2], g[3], g[4], eps4);
-  vr = weno_combine<W>(r1, r2, r3, tr, g[5], g[4], g[3], g[2], g[1], eps4);
+__device__ __forceinline__ void weno5_lr(const double (&D)[5], double eps34, double &cl, double &cr) {
+  const double k34 = scalar(0.75), k23 = scalar(2.0 / 3.0);
+  const double e0 = D[1] - D[0], e1 = D[2] - D[1], e2 = D[3] - D[2], e3 = D[4] - D[3];
+  const double s0 = e0 * e0 + eps34, s1 = e1 * e1 + eps34, s2 = e2 * e2 + eps34, s3 = e3 * e3 + eps34;
+  const double x1 = k34 * D[1], x2 = k34 * D[2], x3 = k34 * D[3];
+  const double l1 = x1 * (D[1] + e0) + s0, l2 = x1 * D[2] + s1, l3 = x2 * (D[2] - e2) + s2;
+  const double r1 = x3 * (D[3] - e3) + s3, r2 = x3 * D[2] + s2, r3 = x2 * (D[2] + e1) + s1;
+  const double F = 4.0 * D[2];
+  const double tl = W == WENO_YC ? (e0 + e2) - 2.0 * e1 : 0.0;
+  const double tr = W == WENO_YC ? (e1 + e3) - 2.0 * e2 : 0.0;
+  cl = weno_side<W>(l1, l2, l3, k23 * e0 + D[1], 2.0 * D[1] + F, F - D[3], tl);
+  cr = -weno_side<W>(r1, r2, r3, D[3] - k23 * e3, 2.0 * D[3] + F, F - D[1], tr);
 }
 
 // Roe-averaged state of two cells (navierstokes3d.h:144-169) and the
@@ -208,43 +214,33 @@ __device__ __forceinline__ void weno5_lr(const double (&b)[6], const double (&g)
 struct RoeState {
   double vx, vy, vz, vn, a, ek, h0;
   double L00, Lm0, L40, k0, kh, aih;  // left-eigenvector entries (see top)
-  double cL, cR;                      // sound speeds + |v_d| of the two cells
 };
 
-template <int DIR>
-__device__ __forceinline__ RoeState roe_state(const double uL[NV], const double uR[NV], const PassConst &k) {
+// L(q), R(q): quantity q of the records of the cells left and right of the
+// interface.  With s = sqrt(rho) of each cell, the averages are
+// (s_L x_L + s_R x_R) / (s_L + s_R), s v = m / s and s H = (e + P) / s.
+template <int DIR, class LQ, class RQ>
+__device__ __forceinline__ RoeState roe_state(const LQ &L, const RQ &R, const PassConst &k) {
   RoeState s;
-  const double rL = uL[0], rR = uR[0];
-  const double iL = rL == 0.0 ? 0.0 : nr_rcp(rL), iR = rR == 0.0 ? 0.0 : nr_rcp(rR);
-  const double vxL = uL[1] * iL, vyL = uL[2] * iL, vzL = uL[3] * iL;
-  const double vxR = uR[1] * iR, vyR = uR[2] * iR, vzR = uR[3] * iR;
-  const double qL = vxL * vxL + vyL * vyL + vzL * vzL, qR = vxR * vxR + vyR * vyR + vzR * vzR;
-  const double PL = (uL[4] - 0.5 * rL * qL) * k.gm1, PR = (uR[4] - 0.5 * rR * qR) * k.gm1;
-  const double c2L = k.gamma * PL * iL, c2R = k.gamma * PR * iR;
-  const double HL = 0.5 * qL + c2L * k.inv_gm1, HR = 0.5 * qR + c2R * k.inv_gm1;
-  const double tL = sqrt(rL), tR = sqrt(rR);
-  const double inv = nr_rcp(tL + tR);
-  s.vx = (tL * vxL + tR * vxR) * inv;
-  s.vy = (tL * vyL + tR * vyR) * inv;
-  s.vz = (tL * vzL + tR * vzR) * inv;
-  const double H = (tL * HL + tR * HR) * inv;
+  const double iL = L(9), iR = R(9);
+  const double inv = nr_rcp(L(0) * iL + R(0) * iR);
+  s.vx = (L(1) * iL + R(1) * iR) * inv;
+  s.vy = (L(2) * iL + R(2) * iR) * inv;
+  s.vz = (L(3) * iL + R(3) * iR) * inv;
+  const double H = (L(10) + R(10)) * inv;
   s.ek = 0.5 * (s.vx * s.vx + s.vy * s.vy + s.vz * s.vz);
   const double a2 = (H - s.ek) * k.gm1;
-  s.a = sqrt(a2);
+  const double ra = nr_rsq(a2);  // 1/a
+  s.a = sqrt_of(a2, ra);
   s.vn = DIR == 0 ? s.vx : (DIR == 1 ? s.vy : s.vz);
-  s.h0 = a2 * k.inv_gm1 + s.ek;
-  const double ia2 = nr_rcp(a2), ih2 = 0.5 * ia2;
-  const double gek = k.gm1 * s.ek, avn = s.a * s.vn;
-  s.L00 = (a2 - gek) * ia2;
-  s.Lm0 = (gek + avn) * ih2;
-  s.L40 = (gek - avn) * ih2;
-  s.k0 = k.gm1 * ia2;
-  s.kh = k.gm1 * ih2;
-  s.aih = s.a * ih2;
-  const double vnL = DIR == 0 ? vxL : (DIR == 1 ? vyL : vzL);
-  const double vnR = DIR == 0 ? vxR : (DIR == 1 ? vyR : vzR);
-  s.cL = sqrt(c2L) + fabs(vnL);
-  s.cR = sqrt(c2R) + fabs(vnR);
+  s.h0 = H;
+  s.aih = 0.5 * ra;
+  s.k0 = k.gm1 * (ra * ra);
+  s.kh = 0.5 * s.k0;
+  const double gek = s.kh * s.ek, avn = s.aih * s.vn;
+  s.L00 = 1.0 - 2.0 * gek;
+  s.Lm0 = gek + avn;
+  s.L40 = gek - avn;
   return s;
 }
 
@@ -312,92 +308,86 @@ __device__ __forceinline__ void right_mult(const RoeState &s, double g0, double 
   f[4] = e;
 }
 
-// Interface flux at I-1/2 from the LDS data of cells I-3..I+2;
-// ld(s, q) returns quantity q of cell I-3+s.
+// Interface flux at I-1/2 from the LDS records of cells I-3..I+2;
+// ld(s, q) returns quantity q of cell I-3+s.  The flux is written as the mean
+// of the two cells' fluxes plus a correction from the differences between
+// neighbouring cells.  In the characteristic scheme only the differences are
+// projected: L R = I, so the mean passes through L and R unchanged.
 template <int DIR, int INTERP, int UPW, int W, class LD>
 __device__ __forceinline__ void iface(const LD &ld, const PassConst &k, double fI[NV]) {
-  double uL[NV], uR[NV];
-#pragma unroll
-  for (int q = 0; q < NV; q++) {
-    uL[q] = ld(2, q);
-    uR[q] = ld(3, q);
+  const RoeState s = roe_state<DIR>([&](int q) { return ld(2, q); }, [&](int q) { return ld(3, q); }, k);
+  double alpha = 0.0;
+  if (UPW == UPWIND_RUSANOV) {  // NavierStokes3DUpwind.c:349-420
+    const double cL = ld(2, 11), cR = ld(3, 11), aA = s.a + fabs(s.vn);
+    alpha = fmax(fmax(cL, cR), fmax(cR, aA));
   }
-  const RoeState s = roe_state<DIR>(uL, uR, k);
-  const double aA = s.a + fabs(s.vn);
-  const double alpha = fmax(fmax(s.cL, s.cR), fmax(s.cR, aA));  // NavierStokes3DUpwind.c:349-420
+  // half of |lambda|
+  const double l0 = 0.5 * (UPW == UPWIND_ROE ? harten(s.vn) : alpha);
+  const double lm = UPW == UPWIND_ROE ? 0.5 * harten(s.vn - s.a) : l0;
+  const double l4 = UPW == UPWIND_ROE ? 0.5 * harten(s.vn + s.a) : l0;
+  double cl, cr;
 
   if (INTERP == INTERP_CHAR) {
-    // rows 0, d, 4 (WENOFifthOrderCalculateWeightsChar, Interp1PrimFifthOrderWENOChar.c:86-198)
-    double f0[6], fm[6], f4[6], u0[6], um[6], u4[6], c0[6], cm[6], c4[6];
+    // fluxes, then states: projected differences of the five fields (rows 0,
+    // d, 4, then the two shear rows; WENOFifthOrderCalculateWeightsChar,
+    // Interp1PrimFifthOrderWENOChar.c:86-198)
+    double g[5];
 #pragma unroll
-    for (int p = 0; p < 6; p++) {
-      const double x0 = ld(p, 0), x1 = ld(p, 1), x2 = ld(p, 2), x3 = ld(p, 3), x4 = ld(p, 4);
-      const double F0 = ld(p, DIR + 1), F1 = ld(p, 5), F2 = ld(p, 6), F3 = ld(p, 7), F4 = ld(p, 8);
-      const double dC = ld(p, 9) - x4;
-      proj_acoustic<DIR>(s, F0, F1, F2, F3, F4, f0[p], fm[p], f4[p]);
-      proj_acoustic<DIR>(s, x0, x1, x2, x3, x4, u0[p], um[p], u4[p]);
-      c0[p] = u0[p] - s.k0 * dC;
-      cm[p] = um[p] + s.kh * dC;
-      c4[p] = u4[p] + s.kh * dC;
-    }
-    double fl, fr, ul, ur;
-    const double l0 = UPW == UPWIND_ROE ? harten(s.vn) : alpha;
-    const double lm = UPW == UPWIND_ROE ? harten(s.vn - s.a) : alpha;
-    const double l4 = UPW == UPWIND_ROE ? harten(s.vn + s.a) : alpha;
-    weno5_lr<W>(f0, f0, k.eps4, fl, fr);
-    weno5_lr<W>(u0, c0, k.eps4, ul, ur);
-    const double g0 = 0.5 * (fl + fr) - l0 * (0.5 * (ur - ul));
-    weno5_lr<W>(fm, fm, k.eps4, fl, fr);
-    weno5_lr<W>(um, cm, k.eps4, ul, ur);
-    const double gm = 0.5 * (fl + fr) - lm * (0.5 * (ur - ul));
-    weno5_lr<W>(f4, f4, k.eps4, fl, fr);
-    weno5_lr<W>(u4, c4, k.eps4, ul, ur);
-    const double g4 = 0.5 * (fl + fr) - l4 * (0.5 * (ur - ul));
-    // shear rows: the modified energy does not enter them (L[row][4] = 0)
-    double fa[6], fb[6], ua[6], ub[6];
+    for (int part = 0; part < 2; part++) {
+      double d[5][5];
 #pragma unroll
-    for (int p = 0; p < 6; p++) {
-      proj_shear<DIR>(s, ld(p, DIR + 1), ld(p, 5), ld(p, 6), ld(p, 7), fa[p], fb[p]);
-      proj_shear<DIR>(s, ld(p, 0), ld(p, 1), ld(p, 2), ld(p, 3), ua[p], ub[p]);
+      for (int p = 0; p < 5; p++) {
+        double x[NV];
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+          const int q = part == 1 ? v : (v == 0 ? DIR + 1 : 4 + v);
+          x[v] = ld(p + 1, q) - ld(p, q);
+        }
+        proj_acoustic<DIR>(s, x[0], x[1], x[2], x[3], x[4], d[0][p], d[1][p], d[2][p]);
+        proj_shear<DIR>(s, x[0], x[1], x[2], x[3], d[3][p], d[4][p]);
+      }
+#pragma unroll
+      for (int f = 0; f < 5; f++) {
+        weno5_lr<W>(d[f], k.eps34, cl, cr);
+        if (part == 0) g[f] = 0.25 * (cl + cr);
+        else g[f] -= (f == 1 ? lm : (f == 2 ? l4 : l0)) * (d[f][2] + 0.5 * (cr - cl));
+      }
     }
-    const double ls = UPW == UPWIND_ROE ? harten(s.vn) : alpha;
-    weno5_lr<W>(fa, fa, k.eps4, fl, fr);
-    weno5_lr<W>(ua, ua, k.eps4, ul, ur);
-    const double ga = 0.5 * (fl + fr) - ls * (0.5 * (ur - ul));
-    weno5_lr<W>(fb, fb, k.eps4, fl, fr);
-    weno5_lr<W>(ub, ub, k.eps4, ul, ur);
-    const double gb = 0.5 * (fl + fr) - ls * (0.5 * (ur - ul));
-    right_mult<DIR>(s, g0, gm, g4, ga, gb, fI);
+    right_mult<DIR>(s, g[0], g[1], g[2], g[3], g[4], fI);
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      const int q = v == 0 ? DIR + 1 : 4 + v;
+      fI[v] += 0.5 * (ld(2, q) + ld(3, q));
+    }
   } else {
     // component-wise (Interp1PrimFifthOrderWENO.c:74-168)
     double fh[NV], du[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      double b[6], g[6];
+      double b[6], D[5];
 #pragma unroll
       for (int p = 0; p < 6; p++) b[p] = ld(p, v == 0 ? DIR + 1 : 4 + v);
-      double fl, fr, ul, ur;
-      weno5_lr<W>(b, b, k.eps4, fl, fr);
 #pragma unroll
-      for (int p = 0; p < 6; p++) {
-        b[p] = ld(p, v);
-        g[p] = v == 4 ? ld(p, 9) : b[p];
-      }
-      weno5_lr<W>(b, g, k.eps4, ul, ur);
-      fh[v] = 0.5 * (fl + fr);
-      du[v] = 0.5 * (ur - ul);
+      for (int p = 0; p < 5; p++) D[p] = b[p + 1] - b[p];
+      weno5_lr<W>(D, k.eps34, cl, cr);
+      fh[v] = 0.5 * ((b[2] + b[3]) + 0.5 * (cl + cr));
+#pragma unroll
+      for (int p = 0; p < 6; p++) b[p] = ld(p, v);
+#pragma unroll
+      for (int p = 0; p < 5; p++) D[p] = b[p + 1] - b[p];
+      weno5_lr<W>(D, k.eps34, cl, cr);
+      du[v] = D[2] + 0.5 * (cr - cl);
     }
     if (UPW == UPWIND_RUSANOV) {
 #pragma unroll
-      for (int v = 0; v < NV; v++) fI[v] = fh[v] - alpha * du[v];
+      for (int v = 0; v < NV; v++) fI[v] = fh[v] - l0 * du[v];
     } else {
-      // R |Lambda| L (uR - uL)/2 (NavierStokes3DUpwind.c:40-124)
+      // R |Lambda|/2 L (uR - uL) (NavierStokes3DUpwind.c:40-124)
       double p0, pm, p4, pa, pb;
       proj_acoustic<DIR>(s, du[0], du[1], du[2], du[3], du[4], p0, pm, p4);
       proj_shear<DIR>(s, du[0], du[1], du[2], du[3], pa, pb);
-      const double hs = harten(s.vn);
       double d[NV];
-      right_mult<DIR>(s, hs * p0, harten(s.vn - s.a) * pm, harten(s.vn + s.a) * p4, hs * pa, hs * pb, d);
+      right_mult<DIR>(s, l0 * p0, lm * pm, l4 * p4, l0 * pa, l0 * pb, d);
 #pragma unroll
       for (int v = 0; v < NV; v++) fI[v] = fh[v] - d[v];
     }
@@ -525,11 +515,10 @@ __device__ __forceinline__ void emit_store(const PassConst &k, const PassIO &io,
   if (io.visc) {
     // primitive variables (u, v, w, T) of the new state for the next
     // viscous-term evaluation (NavierStokes3DParabolicFunction.c:85-108)
-    const Prim q = flowvar(nu, k.gamma);
-    io.Q[idx] = q.vx;
-    io.Q[k.ncell + idx] = q.vy;
-    io.Q[2 * k.ncell + idx] = q.vz;
-    io.Q[3 * k.ncell + idx] = k.gamma * q.P / q.rho;
+    double q[4];
+    visc_prims(nu, k.gamma, q);
+#pragma unroll
+    for (int c = 0; c < 4; c++) io.Q[(size_t)c * k.ncell + idx] = q[c];
   }
 }
 
@@ -547,9 +536,9 @@ constexpr int XCH = 64;        // interfaces per chunk
 constexpr int XNC = XCH + 6;   // cells per chunk
 constexpr int XPAD = 72;
 
-template <int LPB>
+template <int LPB, int UPW>
 struct XShared {
-  double sC[LPB][NQ][XPAD];
+  double sC[LPB][nq(UPW)][XPAD];
   double sF[LPB][NV][XCH + 1];  // slot 0: fI[x0-1]; slot 1+l: fI[x0+l]
   double sF0[LPB][NV];          // fI[0] of the line
 };
@@ -557,7 +546,7 @@ struct XShared {
 // lines LPB*group .. LPB*group + LPB-1 of the grid (line = j + ny*k)
 template <int INTERP, int UPW, int LPB, int W, bool COH = false>
 __device__ __forceinline__ void pass_x_body(const PassConst &k, const PassIO &io, size_t group,
-                                            XShared<LPB> &sh) {
+                                            XShared<LPB, UPW> &sh) {
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nx = k.n[0];
@@ -574,12 +563,12 @@ __device__ __forceinline__ void pass_x_body(const PassConst &k, const PassIO &io
     const int ncells = min(XNC, nx + 6 - x0);
     for (int c = lane; c < ncells; c += 64) {
       const size_t cell = base + wrap(x0 - 3 + c, nx);
-      double u[NV], cd[NQ];
+      double u[NV], cd[nq(UPW)];
 #pragma unroll
       for (int v = 0; v < NV; v++) u[v] = io.U[(size_t)v * k.ncell + cell];
-      cell_data<0>(u, k, cd);
+      cell_data<0, UPW>(u, k, cd);
 #pragma unroll
-      for (int q = 0; q < NQ; q++) sh.sC[w][q][c] = cd[q];
+      for (int q = 0; q < nq(UPW); q++) sh.sC[w][q][c] = cd[q];
     }
     __syncthreads();
     if (active && x0 + lane < nx) {
@@ -623,11 +612,11 @@ __device__ __forceinline__ void pass_x_body(const PassConst &k, const PassIO &io
 // ---------------------------------------------------------------------------
 constexpr int MW = 64;  // columns
 
-template <int MR>
+template <int MR, int UPW>
 struct MShared {
   static constexpr int NRING = MR + 5;  // cell rows t0-3 .. t0+MR+1
   static constexpr int NFR = MR + 1;    // interface rows t0-1 .. t0+MR-1
-  double sC[NQ][NRING][MW];
+  double sC[nq(UPW)][NRING][MW];
   double sF[NV][NFR][MW];
   double sF0[NV][MW];
 };
@@ -635,8 +624,8 @@ struct MShared {
 // columns MW*group .. MW*group + MW-1 of the plane across DIR
 template <int DIR, int INTERP, int UPW, int MR, int W, int RK = RK_CLASSIC, bool COH = false>
 __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io, size_t group,
-                                            MShared<MR> &sh, const SspIO &sp = SspIO{}) {
-  constexpr int NRING = MShared<MR>::NRING, NFR = MShared<MR>::NFR;
+                                            MShared<MR, UPW> &sh, const SspIO &sp = SspIO{}) {
+  constexpr int NRING = MShared<MR, UPW>::NRING, NFR = MShared<MR, UPW>::NFR;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nx = k.n[0], ny = k.n[1];
@@ -653,13 +642,13 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
 
   auto load_row = [&](int r) {  // r in [-3, MR+1]
     const size_t cell = cbase + (size_t)wrap(r, n) * stride;
-    double u[NV], cd[NQ];
+    double u[NV], cd[nq(UPW)];
 #pragma unroll
     for (int v = 0; v < NV; v++) u[v] = io.U[(size_t)v * k.ncell + cell];
-    cell_data<DIR>(u, k, cd);
+    cell_data<DIR, UPW>(u, k, cd);
     const int slot = (r + NRING) % NRING;
 #pragma unroll
-    for (int q = 0; q < NQ; q++) sh.sC[q][slot][lane] = cd[q];
+    for (int q = 0; q < nq(UPW); q++) sh.sC[q][slot][lane] = cd[q];
   };
 
   // ring row r's state, loaded one march step ahead in the same block as
@@ -670,11 +659,11 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
     for (int v = 0; v < NV; v++) u[v] = io.U[(size_t)v * k.ncell + cell];
   };
   auto stage_row = [&](int r, const double (&u)[NV]) {
-    double cd[NQ];
-    cell_data<DIR>(u, k, cd);
+    double cd[nq(UPW)];
+    cell_data<DIR, UPW>(u, k, cd);
     const int slot = (r + NRING) % NRING;
 #pragma unroll
-    for (int q = 0; q < NQ; q++) sh.sC[q][slot][lane] = cd[q];
+    for (int q = 0; q < nq(UPW); q++) sh.sC[q][slot][lane] = cd[q];
   };
 
   // rows -3..MR+1
@@ -738,7 +727,7 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
 
 template <int INTERP, int UPW, int W>
 __global__ void __launch_bounds__(256) k_pass_x(PassConst k, PassIO io) {
-  __shared__ XShared<4> sh;
+  __shared__ XShared<4, UPW> sh;
   pass_x_body<INTERP, UPW, 4, W>(k, io, blockIdx.x, sh);
 }
 
@@ -746,7 +735,7 @@ __global__ void __launch_bounds__(256) k_pass_x(PassConst k, PassIO io) {
 // at the limit, and one register more would halve the occupancy)
 template <int DIR, int INTERP, int UPW, int W>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_pass_m(PassConst k, PassIO io) {
-  __shared__ MShared<4> sh;
+  __shared__ MShared<4, UPW> sh;
   pass_m_body<DIR, INTERP, UPW, 4, W>(k, io, blockIdx.x, sh);
 }
 
@@ -754,7 +743,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
 template <int INTERP, int UPW, int W>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_pass_z_affine(PassConst k, PassIO io,
                                                                                              SspIO sp) {
-  __shared__ MShared<4> sh;
+  __shared__ MShared<4, UPW> sh;
   pass_m_body<2, INTERP, UPW, 4, W, RK_AFFINE>(k, io, blockIdx.x, sh, sp);
 }
 
@@ -766,7 +755,7 @@ struct EnsArgs {
   int nmem;
   const unsigned *item0;   // first work item of each member, nmem + 1 entries
   unsigned nitems;
-  double gamma, gm1, inv_gm1, eps4;
+  double gamma, gm1, inv_gm1, eps34;  // eps34 = 3/4 of the WENO epsilon
   const double *U;         // stage states of all members (member m at 5*off)
   double *R, *u, *S, *acc;
   int mode, stage, visc;
@@ -790,7 +779,7 @@ __device__ __forceinline__ void ens_setup(const EnsArgs &a, int m, int dir, Pass
   k.gamma = a.gamma;
   k.gm1 = a.gm1;
   k.inv_gm1 = a.inv_gm1;
-  k.eps4 = a.eps4;
+  k.eps34 = a.eps34;
   k.dxg = M.dxg;
   const size_t o = 5 * M.off;
   io.U = a.U + o;
@@ -811,7 +800,7 @@ __device__ __forceinline__ void ens_setup(const EnsArgs &a, int m, int dir, Pass
 
 template <int INTERP, int UPW, int LPB, int W>
 __global__ void __launch_bounds__(64 * LPB) k_ens_x(EnsArgs a) {
-  __shared__ XShared<LPB> sh;
+  __shared__ XShared<LPB, UPW> sh;
   for (unsigned item = blockIdx.x; item < a.nitems; item += gridDim.x) {
     const int m = ens_member(a, item);
     PassConst k;
@@ -824,7 +813,7 @@ __global__ void __launch_bounds__(64 * LPB) k_ens_x(EnsArgs a) {
 
 template <int DIR, int INTERP, int UPW, int MR, int W>
 __global__ void __launch_bounds__(64 * MR) __attribute__((amdgpu_waves_per_eu(2))) k_ens_m(EnsArgs a) {
-  __shared__ MShared<MR> sh;
+  __shared__ MShared<MR, UPW> sh;
   for (unsigned item = blockIdx.x; item < a.nitems; item += gridDim.x) {
     const int m = ens_member(a, item);
     PassConst k;
@@ -860,10 +849,10 @@ struct EnsStageArgs {
   unsigned spin_limit;
 };
 
-template <int SH>
+template <int SH, int UPW>
 union StageShared {
-  XShared<SH> x;
-  MShared<SH> m;
+  XShared<SH, UPW> x;
+  MShared<SH, UPW> m;
 };
 
 // the member of item `item` of a direction whose first items are item0
@@ -924,7 +913,7 @@ __device__ __forceinline__ void stage_signal(unsigned *c) {
 
 template <int INTERP, int UPW, int SH, int W>
 __global__ void __launch_bounds__(64 * SH) __attribute__((amdgpu_waves_per_eu(2))) k_ens_stage(EnsStageArgs s) {
-  __shared__ StageShared<SH> sh;
+  __shared__ StageShared<SH, UPW> sh;
   __shared__ unsigned s_ticket, s_last;
   const int nmem = s.a.nmem;
   unsigned *const done_x = s.ctr + 4, *const done_y = s.ctr + 4 + nmem;
@@ -992,11 +981,10 @@ __global__ void __launch_bounds__(256) k_prims(const double *__restrict__ u, dou
   double s[NV];
 #pragma unroll
   for (int v = 0; v < NV; v++) s[v] = u[(size_t)v * ncell + idx];
-  const Prim q = flowvar(s, gamma);
-  Q[idx] = q.vx;
-  Q[ncell + idx] = q.vy;
-  Q[2 * ncell + idx] = q.vz;
-  Q[3 * ncell + idx] = gamma * q.P / q.rho;
+  double q[4];
+  visc_prims(s, gamma, q);
+#pragma unroll
+  for (int c = 0; c < 4; c++) Q[(size_t)c * ncell + idx] = q[c];
 }
 
 template <int DIR, int INTERP, int UPW, int W>
@@ -1040,7 +1028,7 @@ void pass_args(const Grid &g, const Scheme &sc, const PassBuffers &b, int dir, i
   k.gamma = sc.gamma;
   k.gm1 = sc.gamma - 1.0;
   k.inv_gm1 = 1.0 / (sc.gamma - 1.0);
-  k.eps4 = 4.0 * sc.eps;
+  k.eps34 = 0.75 * sc.eps;
   k.dxg = dxg;
   io.U = b.U;
   io.R = b.R;
@@ -1147,7 +1135,7 @@ void launch_ens_pass(const Scheme &sc, int dir, int shape, const EnsMember *mem,
   a.gamma = sc.gamma;
   a.gm1 = sc.gamma - 1.0;
   a.inv_gm1 = 1.0 / (sc.gamma - 1.0);
-  a.eps4 = 4.0 * sc.eps;
+  a.eps34 = 0.75 * sc.eps;
   a.U = U;
   a.R = R;
   a.u = u;
@@ -1212,7 +1200,7 @@ void launch_ens_stage(const Scheme &sc, int rows, const EnsMember *mem, int nmem
   a.gamma = sc.gamma;
   a.gm1 = sc.gamma - 1.0;
   a.inv_gm1 = 1.0 / (sc.gamma - 1.0);
-  a.eps4 = 4.0 * sc.eps;
+  a.eps34 = 0.75 * sc.eps;
   a.U = U;
   a.R = R;
   a.u = u;
