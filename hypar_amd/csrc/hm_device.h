@@ -41,25 +41,24 @@ __device__ __forceinline__ Prim flowvar(const double *u, double gamma) {
   return q;
 }
 
-// 1/d, d > 0 and normal: hardware estimate refined by two Newton-Raphson
-// steps, each of which squares the relative error.
+// 1/d, d > 0 and normal, from the hardware estimate r: with e = 1 - d r,
+// r + r (e + e^2) leaves an error of e^3.  The estimate's e is at most 4.7e-8
+// (measured over 4 million arguments, mantissas over the whole range), so
+// the result is exact to rounding; two Newton-Raphson steps take one
+// operation more.
 __device__ __forceinline__ double nr_rcp(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  double e = __builtin_fma(-d, r, 1.0);
-  r = __builtin_fma(r, e, r);
-  e = __builtin_fma(-d, r, 1.0);
-  return __builtin_fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = __builtin_fma(-d, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
-// 1/sqrt(d), d > 0 and normal: hardware estimate r, then r + r e (1/2 + 3/8 e)
-// with e = 1 - d r^2, which leaves an error of the order e^3, and once more
-// r + r e / 2 for the last bits.
+// 1/sqrt(d), d > 0 and normal, from the hardware estimate r: with
+// e = 1 - d r^2 (at most 1.1e-7, measured), r + r e (1/2 + 3/8 e) leaves an
+// error of 5/16 e^3.
 __device__ __forceinline__ double nr_rsq(double d) {
-  double r = __builtin_amdgcn_rsq(d);
-  double e = __builtin_fma(-d * r, r, 1.0);
-  r = __builtin_fma(r * e, __builtin_fma(0.375, e, 0.5), r);
-  e = __builtin_fma(-d * r, r, 1.0);
-  return __builtin_fma(0.5 * r, e, r);
+  const double r = __builtin_amdgcn_rsq(d);
+  const double e = __builtin_fma(-d * r, r, 1.0);
+  return __builtin_fma(r * e, __builtin_fma(0.375, e, 0.5), r);
 }
 
 // sqrt(d) from r = nr_rsq(d): d r with one correction by the residual d - s^2
