@@ -292,6 +292,8 @@ hm_status hm_create(const hm_config *cfg, hm_solver **out) {
   hm_solver *s = new hm_solver();
   for (int d = 0; d < 3; d++) s->g.n[d] = cfg->dim[d];
   s->g.ncell = (size_t)cfg->dim[0] * cfg->dim[1] * cfg->dim[2];
+  s->g.seg[0] = s->g.n[0];
+  for (int d = 1; d < 3; d++) hm::march_segments(1, &s->g.n, d, &s->g.seg[d]);
   s->sc.interp = cfg->interp == HM_INTERP_CHARACTERISTIC ? hm::INTERP_CHAR : hm::INTERP_COMP;
   s->sc.upwind = cfg->upwind == HM_UPWIND_ROE ? hm::UPWIND_ROE : hm::UPWIND_RUSANOV;
   s->sc.gamma = cfg->gamma;
@@ -1226,6 +1228,14 @@ hm_status hm_ensemble_create(const hm_config *members, int nmembers, hm_ensemble
       }
     }
   }
+  {
+    std::vector<int> dims(3 * (size_t)nmembers), seg(nmembers);
+    for (int m = 0; m < nmembers; m++) std::copy(e->mem[m].n, e->mem[m].n + 3, dims.data() + 3 * (size_t)m);
+    for (int d = 0; d < 3; d++) {
+      if (d > 0) hm::march_segments(nmembers, (const int(*)[3])dims.data(), d, seg.data());
+      for (int m = 0; m < nmembers; m++) e->mem[m].seg[d] = d == 0 ? e->mem[m].n[0] : seg[m];
+    }
+  }
   const size_t n5 = 5 * e->ncell;
   if (hipGetDevice(&e->device) != hipSuccess) {
     st = fail(HM_ERR_HIP, "hm_ensemble_create: no HIP device");
@@ -1279,7 +1289,7 @@ hm_status hm_ensemble_create(const hm_config *members, int nmembers, hm_ensemble
   for (int sh = 0; sh < 2; sh++) {
     for (int d = 0; d < 3; d++) {
       std::vector<unsigned> pre(nmembers + 1, 0);
-      for (int m = 0; m < nmembers; m++) pre[m + 1] = pre[m] + hm::ens_items_per_member(d, sh, e->mem[m].n);
+      for (int m = 0; m < nmembers; m++) pre[m + 1] = pre[m] + hm::ens_items_per_member(d, sh, e->mem[m].n, e->mem[m].seg);
       e->nitems[sh][d] = pre[nmembers];
       if (hipMalloc((void **)&e->item0[sh][d], pre.size() * sizeof(unsigned)) != hipSuccess ||
           hipMemcpy(e->item0[sh][d], pre.data(), pre.size() * sizeof(unsigned), hipMemcpyHostToDevice) !=
@@ -1290,7 +1300,7 @@ hm_status hm_ensemble_create(const hm_config *members, int nmembers, hm_ensemble
     }
     std::vector<unsigned> pre(nmembers + 1, 0);
     for (int m = 0; m < nmembers; m++) {
-      const unsigned groups = hm::ens_items_per_member(0, sh, e->mem[m].n);
+      const unsigned groups = hm::ens_items_per_member(0, sh, e->mem[m].n, e->mem[m].seg);
       pre[m + 1] = pre[m] + (groups + hm::ENS_STAGE_XG - 1) / hm::ENS_STAGE_XG;
     }
     e->nxitems[sh] = pre[nmembers];

@@ -22,6 +22,7 @@ enum { WENO_JS = 0, WENO_MAPPED = 1, WENO_Z = 2, WENO_YC = 3, WENO_OPTIMAL = 4 }
 struct Grid {
   int n[3];
   size_t ncell;
+  int seg[3];  // cells per march segment of the y and z passes (march_segments)
 };
 
 struct Scheme {
@@ -157,6 +158,7 @@ inline int visc_pks(int nx, int ny, int nz) {
 // batched ensemble passes (hm_pass.hip): members of one scheme
 struct EnsMember {
   int n[3];
+  int seg[3];         // cells per march segment of the y and z passes
   size_t ncell;
   size_t off;         // first cell of the member; its state is u[5*off .. 5*(off+ncell))
   const double *dxg;  // ghosted dxinv x|y|z of the member (device)
@@ -167,7 +169,10 @@ struct EnsMember {
 };
 // work items of one member in pass dir with tile shape `shape` (0: 4
 // wavefronts per block, 1: 2 wavefronts per block)
-unsigned ens_items_per_member(int dir, int shape, const int n[3]);
+unsigned ens_items_per_member(int dir, int shape, const int n[3], const int seg[3]);
+// cells per march segment of the pass along dir (1 or 2) of `count` grids that
+// run together, into seg[count]
+void march_segments(int count, const int (*n)[3], int dir, int *seg);
 // one pass of RK stage `stage` over all members; grid = number of
 // persistent blocks (0: one block per work item)
 void launch_ens_pass(const Scheme &sc, int dir, int shape, const EnsMember *mem, int nmem, const unsigned *item0,

@@ -62,6 +62,8 @@
 // 64-member Euler ensemble 18.7 -> 15.2 ms per step.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "hm_device.h"
 #include "hm_internal.h"
 
@@ -77,6 +79,7 @@ constexpr int nq(int upw) { return upw == UPWIND_RUSANOV ? 12 : 11; }
 
 struct PassConst {
   int n[3];
+  int seg;    // cells per march segment along the pass direction (y, z passes)
   size_t ncell;
   double gamma, gm1, inv_gm1, eps34;  // eps34 = 3/4 of the WENO epsilon
   const double *dxg;  // ghosted dxinv x|y|z
@@ -621,9 +624,13 @@ struct MShared {
   double sF0[NV][MW];
 };
 
-// columns MW*group .. MW*group + MW-1 of the plane across DIR
+// item = group + groups * segment: columns MW*group .. MW*group + MW-1 of the
+// plane across DIR, and the cells c0 .. c1-1 of the segment along DIR.  A
+// segment that is a whole line keeps the flux of interface 0 for its last
+// cell; any other evaluates interfaces c0 .. c1, one more than its cells,
+// and starts on six rows of its neighbour.
 template <int DIR, int INTERP, int UPW, int MR, int W, int RK = RK_CLASSIC, bool COH = false>
-__device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io, size_t group,
+__device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io, size_t item,
                                             MShared<MR, UPW> &sh, const SspIO &sp = SspIO{}) {
   constexpr int NRING = MShared<MR, UPW>::NRING, NFR = MShared<MR, UPW>::NFR;
   const int lane = threadIdx.x & 63;
@@ -633,14 +640,20 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
   // the 64 lanes take 64 consecutive columns c = i + nx*o of the plane
   // across DIR (o = z index in the y pass, y index in the z pass)
   const size_t ncol = k.ncell / n;
-  const size_t c = group * MW + lane;
+  const unsigned groups = (unsigned)((ncol + MW - 1) / MW);
+  const bool whole = k.seg >= n;
+  const unsigned sg = whole ? 0u : (unsigned)item / groups;
+  const int c0 = (int)sg * k.seg, c1 = min(c0 + k.seg, n);
+  const int tend = whole ? n : c1 + 1;        // interfaces c0 .. tend-1
+  const int elast = whole ? n - 2 : c1 - 1;   // last cell the march emits
+  const size_t c = ((unsigned)item - sg * groups) * (size_t)MW + lane;
   const bool col = c < ncol;
   const size_t line = col ? c : ncol - 1;
   const size_t o = line / nx;
   const size_t stride = DIR == 1 ? (size_t)nx : (size_t)nx * ny;
   const size_t cbase = DIR == 1 ? o * nx * ny + (line - o * nx) : line;  // cell at position 0
 
-  auto load_row = [&](int r) {  // r in [-3, MR+1]
+  auto load_row = [&](int r) {  // r in [c0-3, c0+MR+1]
     const size_t cell = cbase + (size_t)wrap(r, n) * stride;
     double u[NV], cd[nq(UPW)];
 #pragma unroll
@@ -653,7 +666,7 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
 
   // ring row r's state, loaded one march step ahead in the same block as
   // the output's operands, so that their latencies overlap
-  auto fetch_row = [&](int r, double (&u)[NV]) {  // r in [-3, n+MR]
+  auto fetch_row = [&](int r, double (&u)[NV]) {  // r in [-3, n+MR+1]
     const size_t cell = cbase + (size_t)wrap(r, n) * stride;
 #pragma unroll
     for (int v = 0; v < NV; v++) u[v] = io.U[(size_t)v * k.ncell + cell];
@@ -666,12 +679,12 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
     for (int q = 0; q < nq(UPW); q++) sh.sC[q][slot][lane] = cd[q];
   };
 
-  // rows -3..MR+1
-  for (int r = w; r < MR + 5; r += MR) load_row(r - 3);
-  for (int t0 = 0; t0 < n; t0 += MR) {
+  // rows c0-3..c0+MR+1
+  for (int r = w; r < MR + 5; r += MR) load_row(c0 + r - 3);
+  for (int t0 = c0; t0 < tend; t0 += MR) {
     __syncthreads();
     const int t = t0 + w;
-    if (t < n) {
+    if (t < tend) {
       const int sl0 = (t - 3 + NRING) % NRING;
       auto ld = [&](int s, int q) {
         int sl = sl0 + s;
@@ -688,17 +701,17 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
         for (int v = 0; v < NV; v++) sh.sF0[v][lane] = f[v];
     }
     const int e = t0 - 1 + w;  // row emitted by this wavefront
-    const bool emits = col && e >= 0 && e <= n - 2;
+    const bool emits = col && e >= c0 && e <= elast;
     __syncthreads();
     // the next step's ring row (its slot held row t0-3+w, which no later
     // step reads) and the output's operands, loaded by every lane (a stand-in
     // row 0 after the last step, output rows clamped into the line) so that
     // no divergent branch separates the loads
-    const bool more = t0 + MR < n;
-    const int rn = more ? t0 + MR + 2 + w : 0;  // at most n+MR
+    const bool more = t0 + MR < tend;
+    const int rn = more ? t0 + MR + 2 + w : 0;  // at most n+MR (n+MR+1 in a segment)
     double un[NV];
     fetch_row(rn, un);
-    const int ec = e < 0 ? 0 : (e > n - 2 ? n - 2 : e);
+    const int ec = e < 0 ? 0 : (e > elast ? elast : e);
     const EmitIn in = emit_load<DIR, RK, COH>(k, io, cbase + (size_t)ec * stride, ec, sp);
     if (more) stage_row(rn, un);
     if (emits) {
@@ -712,8 +725,8 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
       emit_store<DIR, RK, COH>(k, io, cbase + (size_t)e * stride, in, fm, fp, sp);
     }
   }
-  // last row: fI[n-1] and fI[n] = fI[0]
-  if (w == 0 && col) {
+  // last row of a whole line: fI[n-1] and fI[n] = fI[0]
+  if (whole && w == 0 && col) {
     double fm[NV], fp[NV];
     const int a = (n - 1) % NFR;
 #pragma unroll
@@ -775,6 +788,7 @@ __device__ __forceinline__ int ens_member(const EnsArgs &a, unsigned item) {
 __device__ __forceinline__ void ens_setup(const EnsArgs &a, int m, int dir, PassConst &k, PassIO &io) {
   const EnsMember M = a.mem[m];
   for (int d = 0; d < 3; d++) k.n[d] = M.n[d];
+  k.seg = M.seg[dir];
   k.ncell = M.ncell;
   k.gamma = a.gamma;
   k.gm1 = a.gm1;
@@ -987,13 +1001,18 @@ __global__ void __launch_bounds__(256) k_prims(const double *__restrict__ u, dou
   for (int c = 0; c < 4; c++) Q[(size_t)c * ncell + idx] = q[c];
 }
 
+// work items of a y or z pass: groups of MW columns times segments
+size_t march_items(size_t ncol, int n, int seg) {
+  return ((ncol + MW - 1) / MW) * (size_t)(seg >= n ? 1 : (n + seg - 1) / seg);
+}
+
 template <int DIR, int INTERP, int UPW, int W>
 void launch_t(const Grid &g, const PassConst &k, const PassIO &io, hipStream_t st) {
   if (DIR == 0) {
     const size_t nlines = (size_t)g.n[1] * g.n[2];
     hipLaunchKernelGGL((k_pass_x<INTERP, UPW, W>), dim3((unsigned)((nlines + 3) / 4)), dim3(256), 0, st, k, io);
   } else {
-    const size_t nb = (g.ncell / g.n[DIR] + MW - 1) / MW;
+    const size_t nb = march_items(g.ncell / g.n[DIR], g.n[DIR], k.seg);
     hipLaunchKernelGGL((k_pass_m<DIR == 0 ? 1 : DIR, INTERP, UPW, W>), dim3((unsigned)nb), dim3(256), 0, st, k, io);
   }
 }
@@ -1043,12 +1062,12 @@ void pass_args(const Grid &g, const Scheme &sc, const PassBuffers &b, int dir, i
   io.stage = stage;
   io.ca = ca;
   io.cb = cb;
-  (void)dir;
+  k.seg = dir == 0 ? 0 : g.seg[dir];
 }
 
 template <int INTERP, int UPW, int W>
 void launch_ssp_t(const Grid &g, const PassConst &k, const PassIO &io, const SspIO &sp, hipStream_t st) {
-  const size_t nb = (g.ncell / g.n[2] + MW - 1) / MW;
+  const size_t nb = march_items(g.ncell / g.n[2], g.n[2], k.seg);
   hipLaunchKernelGGL((k_pass_z_affine<INTERP, UPW, W>), dim3((unsigned)nb), dim3(256), 0, st, k, io, sp);
 }
 
@@ -1115,13 +1134,13 @@ void ens_launch_t(int weno, int dir, int shape, const EnsArgs &a, unsigned grid,
 }
 }  // namespace
 
-unsigned ens_items_per_member(int dir, int shape, const int n[3]) {
+unsigned ens_items_per_member(int dir, int shape, const int n[3], const int seg[3]) {
   const size_t ncell = (size_t)n[0] * n[1] * n[2];
   if (dir == 0) {
     const size_t lpb = shape == 0 ? 4 : 2;
     return (unsigned)(((size_t)n[1] * n[2] + lpb - 1) / lpb);
   }
-  return (unsigned)((ncell / n[dir] + MW - 1) / MW);
+  return (unsigned)march_items(ncell / n[dir], n[dir], seg[dir]);
 }
 
 void launch_ens_pass(const Scheme &sc, int dir, int shape, const EnsMember *mem, int nmem, const unsigned *item0,
@@ -1224,6 +1243,50 @@ void launch_ens_stage(const Scheme &sc, int rows, const EnsMember *mem, int nmem
     if (sc.upwind == UPWIND_ROE) stage_launch_t<INTERP_COMP, UPWIND_ROE>(sc.weno, rows, s, grid, cus, st);
     else stage_launch_t<INTERP_COMP, UPWIND_RUSANOV>(sc.weno, rows, s, grid, cus, st);
   }
+}
+
+// Segments of the y (z) march.  A block marches 64 columns; a grid (or an
+// ensemble) with few columns leaves CUs idle and ends on a long tail, so its
+// lines are cut into segments, each of which evaluates one interface more
+// than its cells and stages six rows of its neighbour again.  The length is
+// the one with the least estimated time
+//   max(0.9 work/256 + longest/2, 1.1 longest)
+// in march steps of MR rows, a segment costing its steps plus 2 for its
+// start (work: all segments' steps; 256 CUs of two blocks each); a shorter
+// one has to win 3%, and lines under 8 cells stay whole (the row indices of
+// a segment reach n + 5).  Measured, y / z pass, whole lines -> segments: 64^3
+// component-wise 45 / 60 -> 17 / 20 us, 128^3 106 / 159 -> 86 / 125 us, 201^3
+// 403 / 539 -> 340 / 456 us; 256^3 stays whole (666 / 866 us, 656-672 / 866-900
+// in segments of 47 to 127 cells).
+void march_segments(int count, const int (*n)[3], int dir, int *seg) {
+  constexpr int MR = 4, CUS = 256;
+  int nmax = 0;
+  for (int m = 0; m < count; m++) nmax = std::max(nmax, n[m][dir]);
+  auto cut = [](int N, int len) {  // cells per segment: equal parts of at most len cells
+    if (N < 8 || len >= N) return N;
+    const int parts = (N + len - 1) / len;
+    return (N + parts - 1) / parts;
+  };
+  int best = nmax;
+  double tbest = 0.0;
+  for (int parts = 1; parts <= std::max(1, nmax / 3); parts++) {
+    const int len = (nmax + parts - 1) / parts;
+    if (parts > 1 && len == (nmax + parts - 2) / (parts - 1)) continue;
+    double work = 0.0;
+    int longest = 0;
+    for (int m = 0; m < count; m++) {
+      const int N = n[m][dir], c = cut(N, len);
+      const int steps = 2 + ((c < N ? c + 1 : N) + MR - 1) / MR;
+      work += (double)march_items((size_t)n[m][0] * n[m][1] * n[m][2] / N, N, c) * steps;
+      longest = std::max(longest, steps);
+    }
+    const double t = std::max(0.9 * work / CUS + 0.5 * longest, 1.1 * longest);
+    if (parts == 1 || t < 0.97 * tbest) {
+      tbest = t;
+      best = len;
+    }
+  }
+  for (int m = 0; m < count; m++) seg[m] = cut(n[m][dir], best);
 }
 
 void launch_prims(const Grid &g, const Scheme &sc, const double *u, double *Q, hipStream_t st) {
