@@ -294,6 +294,7 @@ hm_status hm_create(const hm_config *cfg, hm_solver **out) {
   s->g.ncell = (size_t)cfg->dim[0] * cfg->dim[1] * cfg->dim[2];
   s->g.seg[0] = s->g.n[0];
   for (int d = 1; d < 3; d++) hm::march_segments(1, &s->g.n, d, &s->g.seg[d]);
+  s->g.pks = hm::visc_segment(1, &s->g.n);
   s->sc.interp = cfg->interp == HM_INTERP_CHARACTERISTIC ? hm::INTERP_CHAR : hm::INTERP_COMP;
   s->sc.upwind = cfg->upwind == HM_UPWIND_ROE ? hm::UPWIND_ROE : hm::UPWIND_RUSANOV;
   s->sc.gamma = cfg->gamma;
@@ -1022,6 +1023,7 @@ struct hm_ensemble {
   double *par = nullptr, *Q = nullptr;
   unsigned *ptiles0 = nullptr, *tiles0 = nullptr;
   unsigned nptiles = 0, ntiles = 0;
+  int pks = 1;  // planes per z segment of the viscous-term launch
   unsigned *item0[2][3] = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
   unsigned nitems[2][3] = {{0, 0, 0}, {0, 0, 0}};
   // x items of the one-launch-per-stage kernel (ENS_STAGE_XG line groups each)
@@ -1073,7 +1075,7 @@ void ens_drop_graph(hm_ensemble *e) {
 // primitive variables in Q), then the three direction passes, as three
 // launches (shapes 0, 1) or one (shapes 2, 3)
 void ens_stage_launches(hm_ensemble *e, int stage, const double *U, double *u, double *Sn, hipStream_t st) {
-  if (e->sc.Re > 0) hm::launch_ens_visc(e->sc, e->mem_dev, e->nmem, e->ptiles0, e->nptiles, st);
+  if (e->sc.Re > 0) hm::launch_ens_visc(e->sc, e->mem_dev, e->nmem, e->ptiles0, e->nptiles, e->pks, st);
   const int ts = e->shape & 1;  // 0: 4 wavefronts per block, 1: 2
   if (e->shape >= 2) {
     const unsigned *const item0[3] = {e->xitem0[ts], e->item0[ts][1], e->item0[ts][2]};
@@ -1235,6 +1237,7 @@ hm_status hm_ensemble_create(const hm_config *members, int nmembers, hm_ensemble
       if (d > 0) hm::march_segments(nmembers, (const int(*)[3])dims.data(), d, seg.data());
       for (int m = 0; m < nmembers; m++) e->mem[m].seg[d] = d == 0 ? e->mem[m].n[0] : seg[m];
     }
+    e->pks = hm::visc_segment(nmembers, (const int(*)[3])dims.data());
   }
   const size_t n5 = 5 * e->ncell;
   if (hipGetDevice(&e->device) != hipSuccess) {
@@ -1259,7 +1262,7 @@ hm_status hm_ensemble_create(const hm_config *members, int nmembers, hm_ensemble
       hm::EnsMember &M = e->mem[m];
       M.par = e->par + 4 * M.off;
       M.q = e->Q + 4 * M.off;
-      pre[m + 1] = pre[m] + hm::par_tiles(M.n[0], M.n[1], M.n[2]);
+      pre[m + 1] = pre[m] + hm::par_tiles(M.n[0], M.n[1], M.n[2], e->pks);
     }
     e->nptiles = pre[nmembers];
     if (hipMalloc((void **)&e->ptiles0, pre.size() * sizeof(unsigned)) != hipSuccess ||

@@ -23,6 +23,7 @@ struct Grid {
   int n[3];
   size_t ncell;
   int seg[3];  // cells per march segment of the y and z passes (march_segments)
+  int pks;     // planes per segment of the viscous-term kernel (visc_segment)
 };
 
 struct Scheme {
@@ -127,33 +128,13 @@ __host__ __device__ inline unsigned visc_tiles(int nx, int ny, int nz) {
 }
 
 // tiles of the viscous-term kernel (hm_kernels.hip): a block owns PTX x PTY
-// (x, y) columns and marches through a z segment of pks planes: PKS in the
-// batched ensemble, visc_pks() of the grid for one grid
-#ifndef HM_PTX
-#define HM_PTX 32
-#endif
-#ifndef HM_PTY
-#define HM_PTY 16
-#endif
-#ifndef HM_PKS
-#define HM_PKS 16
-#endif
-constexpr int PTX = HM_PTX, PTY = HM_PTY, PKS = HM_PKS;
-__host__ __device__ inline unsigned par_tiles(int nx, int ny, int nz, int pks = PKS) {
+// (x, y) columns and marches through a z segment of pks planes
+constexpr int PTX = 32, PTY = 16;
+__host__ __device__ inline unsigned par_tiles(int nx, int ny, int nz, int pks) {
   return (unsigned)(((nx + PTX - 1) / PTX) * ((ny + PTY - 1) / PTY) * ((nz + pks - 1) / pks));
 }
-// Segment length of the one-grid viscous kernel: the longest of 128, 64, 32
-// planes that still gives at least VISC_MIN_TILES tiles (the kernel holds
-// one 512-thread block per CU, 256 CUs), else PKS.  Longer segments read
-// fewer halo planes: a segment stages 8 planes besides its own.
-#ifndef HM_VISC_MIN_TILES
-#define HM_VISC_MIN_TILES 512
-#endif
-inline int visc_pks(int nx, int ny, int nz) {
-  for (int p = 128; p > PKS; p >>= 1)
-    if (par_tiles(nx, ny, nz, p) >= (unsigned)HM_VISC_MIN_TILES) return p;
-  return PKS;
-}
+// segment length of the viscous-term kernel over `count` grids that run together
+int visc_segment(int count, const int (*n)[3]);
 
 // batched ensemble passes (hm_pass.hip): members of one scheme
 struct EnsMember {
@@ -195,10 +176,10 @@ void launch_ens_stage(const Scheme &sc, int rows, const EnsMember *mem, int nmem
                       double *acc, int stage, hipStream_t st);
 
 // viscous terms of all members (hm_kernels.hip): one launch over the
-// (member, par_tiles) items, ptiles0 = each member's first item (nmem + 1
-// entries); primitive variables of all members
+// (member, par_tiles) items of pks planes, ptiles0 = each member's first item
+// (nmem + 1 entries); primitive variables of all members
 void launch_ens_visc(const Scheme &sc, const EnsMember *mem, int nmem, const unsigned *ptiles0, unsigned nitems,
-                     hipStream_t st);
+                     int pks, hipStream_t st);
 void launch_ens_prims(const Scheme &sc, const EnsMember *mem, int nmem, const double *u, size_t ncell,
                       hipStream_t st);
 

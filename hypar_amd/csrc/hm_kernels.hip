@@ -15,6 +15,8 @@
 //   k_aos_to_soa, k_soa_to_aos  layout conversion at the host transfers
 #include <hip/hip_runtime.h>
 
+#include <cmath>
+
 #include "hm_device.h"
 #include "hm_internal.h"
 
@@ -74,8 +76,7 @@ __device__ __forceinline__ void visc_flux(double fv[4], const QT &q, const doubl
 // FirstDerivativeFourthOrder.c:103) and Dd the same central difference of
 // the flux.  par[c*ncell + cell], c = momentum x, y, z, energy (the mass
 // component is zero).  Q holds u, v, w, T of every cell, Q[c*ncell + cell];
-// the viscosity is mu = T^0.76 = exp(0.76 log T) (raiseto,
-// include/math_ops.h).
+// the viscosity is mu = T^0.76 (pow076).
 //
 // Where the stencil of Dd leaves the grid (positions -2, -1, n, n+1 along
 // d) the reference reads the fluxes of its ghost layers: the primitive
@@ -96,20 +97,25 @@ __device__ __forceinline__ void visc_flux(double fv[4], const QT &q, const doubl
 // planes q-2..q+2 held in registers (in a thread-private part of LDS for
 // the halo point).  The next plane's loads are issued before the current
 // plane's arithmetic and stored to LDS after it.  The x and y fluxes of plane q go to
-// LDS, where their x and y differences are formed.  The z fluxes of the
-// column stay in a five-plane register ring, so the term of plane q-2 is
-// complete once plane q is done.  The z differences of the segment need FVz
-// on planes k0-2..k1+1, so the march covers them; on the ghost planes (-2,
-// -1, nz, nz+1) the z flux comes from direct loads of the column.
+// LDS, where their x and y differences are formed.  The z flux of plane q
+// goes at once into the sums of the planes q-2..q+2 whose z difference reads
+// it, five running sums per component, to which the x + y part of plane q is
+// added; the sum of plane q-2 is then complete.  The z differences of the
+// segment need FVz on planes k0-2..k1+1, so the march covers them; on the
+// ghost planes (-2, -1, nz, nz+1) the z flux comes from direct loads of the
+// column.
+//
+// Vector issue and LDS bandwidth bound it (two waves per SIMD, 100 KB of LDS
+// per block).  Running sums in place of a flux ring and a buffer of x + y
+// parts, index arithmetic kept out of the march and pow076 took the 256^3
+// launch from 0.67 to 0.50 ms, and with the segment rule of visc_segment the
+// 64^3 one from 87 to 23 us and the 16x12x20 one from 91 to 16 us.
 template <int TX, int TY>
 struct ViscParShared {
   double q[4][TY + 8][TX + 8];  // plane q of Q: x0-4..x0+TX+3, y0-4..y0+TY+3
   double fx[4][TY][TX + 4];     // x fluxes of the tile's rows at x0-2..x0+TX+1
   double fy[4][TY + 4][TX];     // y fluxes of the tile's columns at y0-2..y0+TY+1
-  // z ring of each halo point, planes by p mod 5, and the x + y part of
-  // the own column's term on planes q-2..q, by p mod 3 (private to the thread)
-  double hr[5][4][4 * TX + 4 * TY];
-  double pxy[3][4][TX * TY];
+  double hr[5][4][4 * TX + 4 * TY];  // z ring of each halo point, slot advancing with the plane
 };
 
 __device__ __forceinline__ int wrapi(int p, int n) {
@@ -131,16 +137,23 @@ __device__ __forceinline__ double ghost_deriv(int slot, const F &f) {
 }
 
 // Viscous flux along DIR at a ghost position: derivative along DIR only
-// (d[c], already scaled), primitive values q.
+// (d[c], already scaled), primitive values q, viscosity mu.
 template <int DIR>
-__device__ __forceinline__ void ghost_flux(double fv[4], const QT &q, const double (&d)[4], const ViscParams &vp) {
-  const double mu = exp(0.76 * log(q.T));
+__device__ __forceinline__ void ghost_flux(double fv[4], const QT &q, const double (&d)[4], double mu,
+                                           const ViscParams &vp) {
   double gr[4][3];
 #pragma unroll
   for (int c = 0; c < 4; c++)
 #pragma unroll
     for (int e = 0; e < 3; e++) gr[c][e] = e == DIR ? d[c] : 0.0;
   visc_flux<DIR>(fv, q, gr, mu, vp);
+}
+
+// 12 times the 4th-order central difference, summed in the reference's order:
+// T is close to 1 and its differences small, so another order differs from
+// the reference by more than the term's other roundings
+__device__ __forceinline__ double d4u(double fm2, double fm1, double fp1, double fp2) {
+  return fm2 - 8 * fm1 + 8 * fp1 - fp2;
 }
 
 // tile b of the grid; every thread of the block takes part
@@ -185,8 +198,12 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
                                 : (hkind == 0 && hj < ny && hi >= -2 && hi < nx + 2);
   const bool hint = hkind == 1 ? (hj >= 0 && hj < ny) : (hi >= 0 && hi < nx);
 
-  auto ldq = [&](size_t c, int k, double (&r)[4]) {
-    const size_t o = (size_t)wrapi(k, nz) * plane + c;
+  const double r12 = 1.0 / 12.0;
+  const double odx = own ? dxa[3 + i] * r12 : 0.0, ody = own ? dya[3 + j] * r12 : 0.0;
+  const double hdx = hneed && hint ? dxa[3 + hi] * r12 : 0.0, hdy = hneed && hint ? dya[3 + hj] * r12 : 0.0;
+
+  auto ldq = [&](size_t c, int k, double (&r)[4]) {  // k in [-4, nz + 4]
+    const size_t o = (size_t)wrap(k, nz) * plane + c;
 #pragma unroll
     for (int v = 0; v < 4; v++) r[v] = Q[(size_t)v * ncell + o];
   };
@@ -202,33 +219,34 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
   };
   // gradient at tile offset (ox, oy) of interior plane q; zr(s, v) is
   // component v on plane q-2+s of the point
-  auto grad = [&](int ox, int oy, int q, const auto &zr, double (&gr)[4][3]) {
-    const double dxi = dxa[3 + x0 + ox], dyi = dya[3 + y0 + oy], dzi = dza[3 + q];
+  // dxi, dyi: the point's dxinv and dyinv over 12
+  auto grad = [&](int ox, int oy, int q, double dxi, double dyi, const auto &zr, double (&gr)[4][3]) {
+    const double dzi = dza[3 + q] * r12;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      gr[v][0] = d4c(sq(v, oy, ox - 2), sq(v, oy, ox - 1), sq(v, oy, ox + 1), sq(v, oy, ox + 2)) * dxi;
-      gr[v][1] = d4c(sq(v, oy - 2, ox), sq(v, oy - 1, ox), sq(v, oy + 1, ox), sq(v, oy + 2, ox)) * dyi;
-      gr[v][2] = d4c(zr(0, v), zr(1, v), zr(3, v), zr(4, v)) * dzi;
+      gr[v][0] = d4u(sq(v, oy, ox - 2), sq(v, oy, ox - 1), sq(v, oy, ox + 1), sq(v, oy, ox + 2)) * dxi;
+      gr[v][1] = d4u(sq(v, oy - 2, ox), sq(v, oy - 1, ox), sq(v, oy + 1, ox), sq(v, oy + 2, ox)) * dyi;
+      gr[v][2] = d4u(zr(0, v), zr(1, v), zr(3, v), zr(4, v)) * dzi;
     }
   };
   // ghost-layer x / y flux at tile offset (ox, oy)
-  auto ghost_x = [&](int ox, int oy) {
+  auto ghost_x = [&](int ox, int oy, double mu) {
     const int gx = x0 + ox, slot = gx < 0 ? gx + 2 : gx - nx + 2;
     double d[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) d[v] = ghost_deriv(slot, [&](int o) { return sq(v, oy, ox + o); }) * dxa[3 + gx];
     double fv[4];
-    ghost_flux<0>(fv, qat(ox, oy), d, vp);
+    ghost_flux<0>(fv, qat(ox, oy), d, mu, vp);
 #pragma unroll
     for (int v = 0; v < 4; v++) sh.fx[v][oy][ox + 2] = fv[v];
   };
-  auto ghost_y = [&](int ox, int oy) {
+  auto ghost_y = [&](int ox, int oy, double mu) {
     const int gy = y0 + oy, slot = gy < 0 ? gy + 2 : gy - ny + 2;
     double d[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) d[v] = ghost_deriv(slot, [&](int o) { return sq(v, oy + o, ox); }) * dya[3 + gy];
     double fv[4];
-    ghost_flux<1>(fv, qat(ox, oy), d, vp);
+    ghost_flux<1>(fv, qat(ox, oy), d, mu, vp);
 #pragma unroll
     for (int v = 0; v < 4; v++) sh.fy[v][oy + 2][ox] = fv[v];
   };
@@ -238,41 +256,44 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
   // registers and stored once the previous plane's reads are done
   constexpr int NQP = (TX + 8) * (TY + 8), NR = (NQP + NT - 1) / NT;
   double pre[NR][4];
+  int so[NR];  // offset of the point within a plane
+#pragma unroll
+  for (int r = 0; r < NR; r++) {
+    const int c = min(t + r * NT, NQP - 1);
+    so[r] = wrapi(y0 - 4 + c / (TX + 8), ny) * nx + wrapi(x0 - 4 + c % (TX + 8), nx);
+  }
   auto fetch_plane = [&](int q) {
     const size_t pk = (size_t)q * plane;
 #pragma unroll
-    for (int r = 0; r < NR; r++) {
-      const int c = t + r * NT;
-      if (c < NQP) {
-        const int ox = c % (TX + 8), oy = c / (TX + 8);
-        const size_t o = pk + (size_t)wrapi(y0 - 4 + oy, ny) * nx + wrapi(x0 - 4 + ox, nx);
+    for (int r = 0; r < NR; r++)
+      if (t + r * NT < NQP)
 #pragma unroll
-        for (int v = 0; v < 4; v++) pre[r][v] = Q[(size_t)v * ncell + o];
-      }
-    }
+        for (int v = 0; v < 4; v++) pre[r][v] = Q[(size_t)v * ncell + pk + so[r]];
   };
   auto store_plane = [&]() {
 #pragma unroll
     for (int r = 0; r < NR; r++) {
       const int c = t + r * NT;
-      if (c < NQP) {
-        const int ox = c % (TX + 8), oy = c / (TX + 8);
+      if (c < NQP)
 #pragma unroll
-        for (int v = 0; v < 4; v++) sh.q[v][oy][ox] = pre[r][v];
-      }
+        for (int v = 0; v < 4; v++) (&sh.q[v][0][0])[c] = pre[r][v];
     }
   };
 
   // rings of planes q-2..q+2 of the own column (registers) and the halo
-  // point (LDS, plane p in slot p mod 5), and the next plane of each, loaded
-  // a step ahead
+  // point (LDS; plane p of the march in slot (p - k0 + 4) mod 5), and the
+  // next plane of each, loaded a step ahead
   double rq[5][4], nq[4], nh[4];
-  double fz[5][4];
-  auto hslot = [&](int p, int v) -> double & { return sh.hr[wrapi(p, 5)][v][t]; };
+  double sum[5][4];  // running sums of planes q-2..q+2
+  int h5 = 0;        // slot of plane q-2
+  auto hslot = [&](int s, int v) -> double & {  // plane q-2+s
+    const int p = h5 + s;
+    return sh.hr[p >= 5 ? p - 5 : p][v][t];
+  };
 #pragma unroll
   for (int s = 0; s < 5; s++)
 #pragma unroll
-    for (int v = 0; v < 4; v++) rq[s][v] = fz[s][v] = 0.0;
+    for (int v = 0; v < 4; v++) rq[s][v] = sum[s][v] = 0.0;
 #pragma unroll
   for (int v = 0; v < 4; v++) nh[v] = 0.0;
 #pragma unroll
@@ -282,7 +303,7 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
       double r[4];
       ldq(hcol, k0 - 4 + s, r);
 #pragma unroll
-      for (int v = 0; v < 4; v++) hslot(k0 - 4 + s, v) = r[v];
+      for (int v = 0; v < 4; v++) hslot(s, v) = r[v];
     }
   }
   ldq(col, k0, nq);
@@ -300,7 +321,7 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
     for (int v = 0; v < 4; v++) rq[4][v] = nq[v];
     if (hkind >= 0)
 #pragma unroll
-      for (int v = 0; v < 4; v++) hslot(q + 2, v) = nh[v];
+      for (int v = 0; v < 4; v++) hslot(4, v) = nh[v];
     const bool gz = q < 0 || q >= nz;     // a ghost plane along z (uniform)
     const bool outq = q >= k0 && q < k1;  // a plane whose x and y terms are formed
     const bool next = q + 1 < k1 + 2 && q + 1 >= 0 && q + 1 < nz;  // plane q+1 is staged
@@ -311,28 +332,30 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
       if (hkind >= 0) ldq(hcol, q + 3, nh);
     }
     double fzq[4] = {0.0, 0.0, 0.0, 0.0};
+    // the ring's middle entries hold the periodic copy of every point, also
+    // beyond the grid, so one evaluation serves interior and ghost fluxes
+    double mu = pow076(rq[2][3]);
     if (gz) {
       if (own) {
         const int slot = q < 0 ? q + 2 : q - nz + 2;
         double d[4];
 #pragma unroll
         for (int v = 0; v < 4; v++)
-          d[v] = ghost_deriv(slot, [&](int o) { return Q[(size_t)v * ncell + (size_t)wrapi(q + o, nz) * plane + col]; }) *
+          d[v] = ghost_deriv(slot, [&](int o) { return Q[(size_t)v * ncell + (size_t)wrap(q + o, nz) * plane + col]; }) *
                  dza[3 + q];
-        const size_t o = (size_t)wrapi(q, nz) * plane + col;
+        const size_t o = (size_t)wrap(q, nz) * plane + col;
         QT qv;
         qv.u = Q[o];
         qv.v = Q[ncell + o];
         qv.w = Q[2 * ncell + o];
         qv.T = Q[3 * ncell + o];
-        ghost_flux<2>(fzq, qv, d, vp);
+        ghost_flux<2>(fzq, qv, d, mu, vp);
       }
     } else {
       if (own) {
         double gr[4][3];
-        grad(lx, ly, q, [&](int s2, int v) { return rq[s2][v]; }, gr);
+        grad(lx, ly, q, odx, ody, [&](int s2, int v) { return rq[s2][v]; }, gr);
         const QT qv = qat(lx, ly);
-        const double mu = exp(0.76 * log(qv.T));
         visc_flux<2>(fzq, qv, gr, mu, vp);
         if (outq) {
           double fv[4];
@@ -346,15 +369,15 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
       } else if (outq) {
         // the column lies past the grid: ghost-layer x flux at i = nx, nx+1
         // (rows inside), ghost-layer y flux at j = ny, ny+1 (columns inside)
-        if (j < ny && i < nx + 2) ghost_x(lx, ly);
-        if (i < nx && j < ny + 2) ghost_y(lx, ly);
+        if (j < ny && i < nx + 2) ghost_x(lx, ly, mu);
+        if (i < nx && j < ny + 2) ghost_y(lx, ly, mu);
       }
       if (outq && hneed) {
+        mu = pow076(hslot(2, 3));
         if (hint) {
           double gr[4][3];
-          grad(hx, hy, q, [&](int s2, int v) { return hslot(q - 2 + s2, v); }, gr);
+          grad(hx, hy, q, hdx, hdy, [&](int s2, int v) { return hslot(s2, v); }, gr);
           const QT qv = qat(hx, hy);
-          const double mu = exp(0.76 * log(qv.T));
           double fv[4];
           if (hkind == 0) {
             visc_flux<0>(fv, qv, gr, mu, vp);
@@ -366,37 +389,47 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
             for (int v = 0; v < 4; v++) sh.fy[v][hy + 2][hx] = fv[v];
           }
         } else if (hkind == 0) {
-          ghost_x(hx, hy);
+          ghost_x(hx, hy, mu);
         } else {
-          ghost_y(hx, hy);
+          ghost_y(hx, hy, mu);
         }
       }
+    }
+    // plane p = q-2+s reads FVz(q) with weight -1/12, 8/12, 0, -8/12, 1/12
+    // times its dzinv (planes outside the segment are not stored; their
+    // metric index is clamped into the array)
+    {
+      const double z0 = -r12 * dza[3 + max(q - 2, -3)], z1 = 8.0 * r12 * dza[3 + max(q - 1, -3)];
+      const double z3 = -8.0 * r12 * dza[3 + min(q + 1, nz + 2)], z4 = r12 * dza[3 + min(q + 2, nz + 2)];
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        sum[0][v] += z0 * fzq[v];
+        sum[1][v] += z1 * fzq[v];
+        sum[3][v] += z3 * fzq[v];
+        sum[4][v] = z4 * fzq[v];
+      }
+    }
+    __syncthreads();
+    if (next) store_plane();  // nothing reads plane q from LDS any more
+    if (outq && own) {
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const double px = odx * d4u(sh.fx[v][ly][lx], sh.fx[v][ly][lx + 1], sh.fx[v][ly][lx + 3], sh.fx[v][ly][lx + 4]);
+        const double py = ody * d4u(sh.fy[v][ly][lx], sh.fy[v][ly + 1][lx], sh.fy[v][ly + 3][lx], sh.fy[v][ly + 4][lx]);
+        sum[2][v] += px + py;
+      }
+    }
+    const int p = q - 2;  // plane whose sum is now complete
+    if (p >= k0 && own) {
+      const size_t o = (size_t)p * plane + col;
+#pragma unroll
+      for (int v = 0; v < 4; v++) par[(size_t)v * ncell + o] = sum[0][v];
     }
 #pragma unroll
     for (int s = 0; s < 4; s++)
 #pragma unroll
-      for (int v = 0; v < 4; v++) fz[s][v] = fz[s + 1][v];
-#pragma unroll
-    for (int v = 0; v < 4; v++) fz[4][v] = fzq[v];
-    __syncthreads();
-    if (next) store_plane();  // nothing reads plane q from LDS any more
-    if (outq && own) {
-      const double dxi = dxa[3 + i], dyi = dya[3 + j];
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const double px = dxi * d4c(sh.fx[v][ly][lx], sh.fx[v][ly][lx + 1], sh.fx[v][ly][lx + 3], sh.fx[v][ly][lx + 4]);
-        const double py = dyi * d4c(sh.fy[v][ly][lx], sh.fy[v][ly + 1][lx], sh.fy[v][ly + 3][lx], sh.fy[v][ly + 4][lx]);
-        sh.pxy[wrapi(q, 3)][v][t] = px + py;
-      }
-    }
-    const int p = q - 2;  // plane whose z difference is now complete
-    if (p >= k0 && own) {
-      const double dzi = dza[3 + p];
-      const size_t o = (size_t)p * plane + col;
-#pragma unroll
-      for (int v = 0; v < 4; v++)
-        par[(size_t)v * ncell + o] = sh.pxy[wrapi(p, 3)][v][t] + dzi * d4c(fz[0][v], fz[1][v], fz[3][v], fz[4][v]);
-    }
+      for (int v = 0; v < 4; v++) sum[s][v] = sum[s + 1][v];
+    h5 = h5 == 4 ? 0 : h5 + 1;
   }
 }
 
@@ -414,6 +447,7 @@ struct EnsViscArgs {
   int nmem;
   const unsigned *ptiles0;
   unsigned nitems;
+  int pks;
   ViscParams vp;
 };
 
@@ -428,7 +462,7 @@ __global__ void __launch_bounds__(PTX * PTY) k_ens_visc(EnsViscArgs a) {
     else hi = mid - 1;
   }
   const EnsMember &M = a.mem[lo];
-  visc_par_tile<PTX, PTY>(M.q, M.par, M.n[0], M.n[1], M.n[2], M.dxg, a.vp, (int)(item - a.ptiles0[lo]), PKS, sh);
+  visc_par_tile<PTX, PTY>(M.q, M.par, M.n[0], M.n[1], M.n[2], M.dxg, a.vp, (int)(item - a.ptiles0[lo]), a.pks, sh);
 }
 
 // primitive variables of every member's state
@@ -574,17 +608,46 @@ static ViscParams visc_params(const Scheme &sc) {
   return vp;
 }
 
+// A segment of p planes marches p + 4 and starts on 4 more, and a CU holds one
+// block, so with W blocks on 256 CUs one grid takes ceil(W/256) (p + 6) plane
+// times; an ensemble, whose blocks differ in length, its total over 256 and
+// half the longest.  The length with the least such time is taken; a shorter
+// one has to win 3%.
+int visc_segment(int count, const int (*n)[3]) {
+  constexpr int CUS = 256;
+  int nmax = 0;
+  for (int m = 0; m < count; m++) nmax = n[m][2] > nmax ? n[m][2] : nmax;
+  int best = nmax;
+  double tbest = 0.0;
+  for (int parts = 1; parts <= nmax; parts++) {
+    const int p = (nmax + parts - 1) / parts;
+    if (parts > 1 && p == (nmax + parts - 2) / (parts - 1)) continue;
+    double blocks = 0.0, work = 0.0;
+    for (int m = 0; m < count; m++) {
+      const double b = par_tiles(n[m][0], n[m][1], n[m][2], p);
+      blocks += b;
+      work += b * ((n[m][2] < p ? n[m][2] : p) + 6);
+    }
+    const double t = count == 1 ? ceil(blocks / CUS) * (p + 6) : fmax(work / CUS + 0.5 * (p + 6), p + 6);
+    if (parts == 1 || t < 0.97 * tbest) {
+      tbest = t;
+      best = p;
+    }
+  }
+  return best;
+}
+
 void launch_visc_par(const Grid &g, const Scheme &sc, const double *Q, double *par, const double *dxg,
                      hipStream_t st) {
-  const int pks = visc_pks(g.n[0], g.n[1], g.n[2]);
-  const unsigned nb = par_tiles(g.n[0], g.n[1], g.n[2], pks);
-  hipLaunchKernelGGL(k_visc_par, dim3(nb), dim3(PTX * PTY), 0, st, Q, par, g.n[0], g.n[1], g.n[2], pks, dxg,
+  const unsigned nb = par_tiles(g.n[0], g.n[1], g.n[2], g.pks);
+  hipLaunchKernelGGL(k_visc_par, dim3(nb), dim3(PTX * PTY), 0, st, Q, par, g.n[0], g.n[1], g.n[2], g.pks, dxg,
                      visc_params(sc));
 }
 
 void launch_ens_visc(const Scheme &sc, const EnsMember *mem, int nmem, const unsigned *ptiles0, unsigned nitems,
-                     hipStream_t st) {
+                     int pks, hipStream_t st) {
   EnsViscArgs a;
+  a.pks = pks;
   a.mem = mem;
   a.nmem = nmem;
   a.ptiles0 = ptiles0;
