@@ -34,7 +34,9 @@
 namespace hm {
 
 constexpr int VJP_LINE_MAX = 512;  // longest grid line an adjoint workgroup holds
-constexpr int VJP_LDS = 23;        // doubles of LDS per cell of the component-wise line VJP
+constexpr int VJP_CS = 11;         // doubles per cell record of a line VJP: state [5], flux [5], pad
+constexpr int VJP_ES = 13;         // doubles per exchange record of the component-wise line VJP: [12], pad
+constexpr int VJP_LDS = VJP_CS + VJP_ES;  // doubles of LDS per cell of the component-wise line VJP
 
 __device__ __forceinline__ int wrapn(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
@@ -65,86 +67,49 @@ __device__ __forceinline__ LineSlot line_slot(size_t item, int n, size_t nlines)
   return s;
 }
 
-// one side of a WENO5 interpolation from its smoothness indicators beta_k
-// and candidate values f_k: the interpolated value, the weights, ob times
-// d out/d beta_k (g1..g3) and, for the YC weights, ob times d out/d tau (gt)
-// with tau the YC indicator passed in.  W selects the weights
-// (include/interpolation.h:265-285, 314-341, 426-447, 479-500):
-//  * JS:     a_k = c_k/(beta_k + eps)^2;
-//            d out/d beta_k = -2 w_k (f_k - out)/(beta_k + eps)
-//  * Z, YC:  a_k = c_k (1 + (t/(beta_k + eps))^2), t = |beta_3 - beta_1| (Z)
-//            or tau (YC); t's own derivative is folded into g1, g3 (Z) or
-//            returned in gt (YC)
+// One side of WENO5 in the form of hm_pass.hip: from l_k = 3/4 (beta_k + eps)
+// and the candidates' differences p_k from the upwind cell's value (times 2,
+// 12, 6), c = twice the difference of the interpolated value from that cell's
+// value, and the reverse of it: ob times the derivative of c with respect to
+// p_k (w1..w3), l_k (g1..g3) and, for the YC weights, the stencil's 4th
+// difference d4 (gt).  W selects the weights
+// (include/interpolation.h:265-285, 314-341, 426-447, 479-500).  With
+// q_k = the product of the other two l, h_k = p_k - kappa_k c,
+// kappa = 1, 6, 3, and N, A the sums of a_k p_k and kappa_k a_k:
+//  * JS:     a_k = q_k^2;              d c/d l_k = -2 a_k h_k/(l_k A)
+//  * Z, YC:  a_k = q_k^2 (l_k^2 + t^2), t = l_3 - l_1 (Z) or 3/4 d4^2 (YC);
+//            d c/d l_k = -2 t^2 q_k^2 h_k/(l_k A), and t's own derivative
+//            2 t sum(q_k^2 h_k)/A goes into g1, g3 (Z) or gt (YC)
 //  * mapped: the JS weights u_k mapped by u (c + c^2 - 3 c u + u^2)/
 //            (c^2 + u (1 - 2c)) and renormalised; the adjoint goes back
 //            through the mapping and the JS normalisation
 //  * optimal (no_limiting): the constant weights 0.1, 0.6, 0.3
-// The a_k are formed multiplied through by their common denominator; one
-// reciprocal of (sum a_k)(prod (beta_k + eps)) gives both 1/sum a_k and the
-// 1/(beta_k + eps) (the mapped weights take a second one for the mapping).
+// (sum a_k h_k = 0 takes the cross terms out.)  One reciprocal of
+// A l_1 l_2 l_3 gives 1/A and the 1/(l_k A); the mapped weights take a second
+// one for the mapping.
 struct W5Side {
-  double out, w1, w2, w3, g1, g2, g3, gt;
+  double c, w1, w2, w3, g1, g2, g3, gt;
 };
 
 template <int W>
-__device__ __forceinline__ W5Side w5_side(double b1, double b2, double b3, double f1, double f2, double f3,
-                                          double eps, double ob, double tau) {
-  const double e1 = b1 + eps, e2 = b2 + eps, e3 = b3 + eps;
-  const double s1 = e1 * e1, s2 = e2 * e2, s3 = e3 * e3;
+__device__ __forceinline__ W5Side w5_side(double l1, double l2, double l3, double p1, double p2, double p3, double d4,
+                                          double ob) {
   W5Side r;
   r.gt = 0.0;
   if (W == WENO_OPTIMAL) {
-    // no_limiting: constant optimal weights, no dependence on beta_k
-    r.w1 = 0.1;
-    r.w2 = 0.6;
-    r.w3 = 0.3;
-    r.out = 0.1 * f1 + 0.6 * f2 + 0.3 * f3;
+    r.c = 0.1 * (p1 + p2 + p3);
+    r.w1 = r.w2 = r.w3 = 0.1 * ob;
     r.g1 = r.g2 = r.g3 = 0.0;
-  } else if (W == WENO_JS) {
-    const double a1 = 0.1 * (s2 * s3), a2 = 0.6 * (s1 * s3), a3 = 0.3 * (s1 * s2);
-    const double A = a1 + a2 + a3, e23 = e2 * e3, P = e1 * e23;
-    const double q = nr_rcp(A * P);
-    const double inv = q * P, k = -2.0 * ob * (q * A);
-    r.w1 = a1 * inv;
-    r.w2 = a2 * inv;
-    r.w3 = a3 * inv;
-    r.out = r.w1 * f1 + r.w2 * f2 + r.w3 * f3;
-    r.g1 = k * r.w1 * (f1 - r.out) * e23;
-    r.g2 = k * r.w2 * (f2 - r.out) * (e1 * e3);
-    r.g3 = k * r.w3 * (f3 - r.out) * (e1 * e2);
-  } else if (W == WENO_Z || W == WENO_YC) {
-    const double t = W == WENO_Z ? fabs(b3 - b1) : tau, t2 = t * t;
-    const double p1 = s2 * s3, p2 = s1 * s3, p3 = s1 * s2;  // products of the other two s_k
-    const double a1 = 0.1 * (s1 + t2) * p1, a2 = 0.6 * (s2 + t2) * p2, a3 = 0.3 * (s3 + t2) * p3;
-    const double A = a1 + a2 + a3, e23 = e2 * e3, P = e1 * e23;
-    const double q = nr_rcp(A * P);
-    const double inv = q * P;
-    r.w1 = a1 * inv;
-    r.w2 = a2 * inv;
-    r.w3 = a3 * inv;
-    r.out = r.w1 * f1 + r.w2 * f2 + r.w3 * f3;
-    // d out/d a_k (unscaled a_k) = s1 s2 s3 (f_k - out)/A, d a_k/d beta_k =
-    // -2 c_k t^2/(beta_k + eps)^3 and d a_k/d t = 2 c_k t/(beta_k + eps)^2
-    const double h1 = ob * (f1 - r.out), h2 = ob * (f2 - r.out), h3 = ob * (f3 - r.out);
-    r.g1 = (-2.0 * 0.1) * t2 * h1 * p1 * e23 * q;
-    r.g2 = (-2.0 * 0.6) * t2 * h2 * p2 * (e1 * e3) * q;
-    r.g3 = (-2.0 * 0.3) * t2 * h3 * p3 * (e1 * e2) * q;
-    const double gt = 2.0 * t * inv * (0.1 * h1 * p1 + 0.6 * h2 * p2 + 0.3 * h3 * p3);
-    if (W == WENO_Z) {
-      // t = |beta_3 - beta_1|; at beta_3 = beta_1 the derivative is taken as 0
-      const double sg = b3 > b1 ? 1.0 : (b3 < b1 ? -1.0 : 0.0);
-      r.g3 += sg * gt;
-      r.g1 -= sg * gt;
-    } else {
-      r.gt = gt;
-    }
-  } else {
+    return r;
+  }
+  const double q1 = l2 * l3, q2 = l1 * l3, q3 = l1 * l2, P = l1 * q1;
+  const double s1 = q1 * q1, s2 = q2 * q2, s3 = q3 * q3;
+  if (W == WENO_MAPPED) {
     const double c1 = 0.1, c2 = 0.6, c3 = 0.3;
-    const double at1 = c1 * (s2 * s3), at2 = c2 * (s1 * s3), at3 = c3 * (s1 * s2);
-    const double At = at1 + at2 + at3, e23 = e2 * e3, P = e1 * e23;
-    const double q = nr_rcp(At * P);
+    const double A = s1 + 3.0 * (2.0 * s2 + s3);
+    const double q = nr_rcp(A * P);
     const double it = q * P;
-    const double u1 = at1 * it, u2 = at2 * it, u3 = at3 * it;  // JS weights
+    const double u1 = s1 * it, u2 = s2 * (6.0 * it), u3 = s3 * (3.0 * it);  // JS weights
     const double N1 = c1 + c1 * c1 - 3 * c1 * u1 + u1 * u1, D1 = c1 * c1 + u1 * (1.0 - 2.0 * c1);
     const double N2 = c2 + c2 * c2 - 3 * c2 * u2 + u2 * u2, D2 = c2 * c2 + u2 * (1.0 - 2.0 * c2);
     const double N3 = c3 + c3 * c3 - 3 * c3 * u3 + u3 * u3, D3 = c3 * c3 + u3 * (1.0 - 2.0 * c3);
@@ -152,91 +117,109 @@ __device__ __forceinline__ W5Side w5_side(double b1, double b2, double b3, doubl
     const double B1 = u1 * N1 * o1, B2 = u2 * N2 * o2, B3 = u3 * N3 * o3, B = B1 + B2 + B3;
     const double qm = nr_rcp(B * DD);
     const double im = qm * DD;
-    r.w1 = B1 * im;
-    r.w2 = B2 * im;
-    r.w3 = B3 * im;
-    r.out = r.w1 * f1 + r.w2 * f2 + r.w3 * f3;
-    // d out/d a_k = DD (f_k - out)/B with a_k = u_k N_k/D_k, whose derivative
+    const double f1 = p1, f2 = (1.0 / 6.0) * p2, f3 = (1.0 / 3.0) * p3;
+    const double w1 = B1 * im, w2 = B2 * im, w3 = B3 * im;
+    r.c = w1 * f1 + w2 * f2 + w3 * f3;
+    r.w1 = ob * w1;
+    r.w2 = ob * w2 * (1.0 / 6.0);
+    r.w3 = ob * w3 * (1.0 / 3.0);
+    // d c/d a_k = DD (f_k - c)/B with a_k = u_k N_k/D_k, whose derivative
     // is ((N_k + u_k N_k') D_k - u_k N_k D_k')/D_k^2; DD/(B D_k^2) = o_k^2 qm
-    const double h1 = ob * (f1 - r.out), h2 = ob * (f2 - r.out), h3 = ob * (f3 - r.out);
+    const double h1 = ob * (f1 - r.c), h2 = ob * (f2 - r.c), h3 = ob * (f3 - r.c);
     const double du1 = h1 * ((N1 + u1 * (2 * u1 - 3 * c1)) * D1 - u1 * N1 * (1.0 - 2.0 * c1)) * (o1 * o1) * qm;
     const double du2 = h2 * ((N2 + u2 * (2 * u2 - 3 * c2)) * D2 - u2 * N2 * (1.0 - 2.0 * c2)) * (o2 * o2) * qm;
     const double du3 = h3 * ((N3 + u3 * (2 * u3 - 3 * c3)) * D3 - u3 * N3 * (1.0 - 2.0 * c3)) * (o3 * o3) * qm;
-    // through u_k = at_k/sum at, at_k = c_k/(beta_k + eps)^2
-    const double U = du1 * u1 + du2 * u2 + du3 * u3, iP = q * At;
-    r.g1 = -2.0 * (du1 - U) * u1 * e23 * iP;
-    r.g2 = -2.0 * (du2 - U) * u2 * (e1 * e3) * iP;
-    r.g3 = -2.0 * (du3 - U) * u3 * (e1 * e2) * iP;
+    // through u_k = at_k/sum at, at_k = c_k/l_k^2
+    const double U = du1 * u1 + du2 * u2 + du3 * u3, iP = -2.0 * (q * A);
+    r.g1 = (du1 - U) * u1 * q1 * iP;
+    r.g2 = (du2 - U) * u2 * q2 * iP;
+    r.g3 = (du3 - U) * u3 * q3 * iP;
+    return r;
+  }
+  double a1 = s1, a2 = s2, a3 = s3, t = 0.0, t2 = 1.0;
+  if (W != WENO_JS) {
+    t = W == WENO_Z ? l3 - l1 : 0.75 * (d4 * d4);
+    t2 = t * t;
+    a1 *= l1 * l1 + t2;
+    a2 *= l2 * l2 + t2;
+    a3 *= l3 * l3 + t2;
+  }
+  const double A = a1 + scalar(3.0) * (2.0 * a2 + a3);
+  const double q = nr_rcp(A * P);
+  const double inv = q * P;
+  r.c = (a1 * p1 + a2 * p2 + a3 * p3) * inv;
+  const double oi = ob * inv, k = (-2.0 * ob) * (W == WENO_JS ? q : t2 * q);
+  r.w1 = a1 * oi;
+  r.w2 = a2 * oi;
+  r.w3 = a3 * oi;
+  const double h1 = s1 * (p1 - r.c), h2 = s2 * (p2 - 6.0 * r.c), h3 = s3 * (p3 - 3.0 * r.c);
+  r.g1 = k * (q1 * h1);
+  r.g2 = k * (q2 * h2);
+  r.g3 = k * (q3 * h3);
+  if (W != WENO_JS) {
+    const double gt = 2.0 * t * oi * (h1 + h2 + h3);
+    if (W == WENO_Z) {
+      r.g3 += gt;
+      r.g1 -= gt;
+    } else {
+      r.gt = 1.5 * d4 * gt;
+    }
   }
   return r;
 }
 
-// reverse of the left- and right-biased WENO5 of one interface, with
-// smoothness indicators from b[0..5] and interpolated values from g[0..5]
-// (cells I-3..I+2; g = b except for the modified energy, a function of the
-// same state): adds obL d vl/d(b, g) + obR d vr/d(b, g) to bb and returns
-// vl, vr.  The second differences the two sides share are formed once and
-// their adjoints summed.
+// reverse of the left- and right-biased WENO5 of one interface, as functions
+// of the five first differences D of cells I-3..I+2 (the values themselves
+// enter only as b[2] and b[3], which the caller takes back): sets G to
+// obL d vl/d D + obR d vr/d D and returns jump = (vr - b[3]) - (vl - b[2]) +
+// D[2] = vr - vl and corr = (vl - b[2]) + (vr - b[3]).  e are the second
+// differences; the indicators are those of hm_pass.hip
+// (l = e^2 + 3/4 x (x + e) and e^2 + 3/4 x y).  G may be D.
 template <int W>
-__device__ __forceinline__ void weno5_lr_vjp(const double b[6], const double g[6], double eps, double obL,
-                                             double obR, double bb[6], double &vl, double &vr) {
-  const double c1312 = 13.0 / 12.0, c14 = 0.25, s6 = 1.0 / 6.0;
-  const double d1 = b[0] - 2 * b[1] + b[2], d2 = b[1] - 2 * b[2] + b[3];
-  const double d3 = b[2] - 2 * b[3] + b[4], d4 = b[3] - 2 * b[4] + b[5];
-  const double q2 = c1312 * (d2 * d2), q3 = c1312 * (d3 * d3);
-  const double rl1 = b[0] - 4 * b[1] + 3 * b[2], rl2 = b[1] - b[3], rl3 = 3 * b[2] - 4 * b[3] + b[4];
-  const double rr1 = b[5] - 4 * b[4] + 3 * b[3], rr2 = b[4] - b[2], rr3 = 3 * b[3] - 4 * b[2] + b[1];
-  // YC: undivided 4th differences of the two stencils, tau = their squares
-  const double tl = W == WENO_YC ? b[0] - 4 * b[1] + 6 * b[2] - 4 * b[3] + b[4] : 0.0;
-  const double tr = W == WENO_YC ? b[5] - 4 * b[4] + 6 * b[3] - 4 * b[2] + b[1] : 0.0;
-  // left: second differences d1, d2, d3; right (mirrored): d4, d3, d2
-  const W5Side L = w5_side<W>(c1312 * (d1 * d1) + c14 * (rl1 * rl1), q2 + c14 * (rl2 * rl2),
-                              q3 + c14 * (rl3 * rl3), (2 * s6) * g[0] + (-7 * s6) * g[1] + (11 * s6) * g[2],
-                              (-s6) * g[1] + (5 * s6) * g[2] + (2 * s6) * g[3],
-                              (2 * s6) * g[2] + (5 * s6) * g[3] + (-s6) * g[4], eps, obL, tl * tl);
-  const W5Side R = w5_side<W>(c1312 * (d4 * d4) + c14 * (rr1 * rr1), q3 + c14 * (rr2 * rr2),
-                              q2 + c14 * (rr3 * rr3), (2 * s6) * g[5] + (-7 * s6) * g[4] + (11 * s6) * g[3],
-                              (-s6) * g[4] + (5 * s6) * g[3] + (2 * s6) * g[2],
-                              (2 * s6) * g[3] + (5 * s6) * g[2] + (-s6) * g[1], eps, obR, tr * tr);
-  vl = L.out;
-  vr = R.out;
-  // interpolated values
-  const double wl1 = obL * L.w1, wl2 = obL * L.w2, wl3 = obL * L.w3;
-  const double wr1 = obR * R.w1, wr2 = obR * R.w2, wr3 = obR * R.w3;
-  // smoothness indicators: second differences and the one-sided differences
-  const double D1 = (2 * c1312) * d1 * L.g1, D2 = (2 * c1312) * d2 * (L.g2 + R.g3);
-  const double D3 = (2 * c1312) * d3 * (L.g3 + R.g2), D4 = (2 * c1312) * d4 * R.g1;
-  const double L1 = (2 * c14) * rl1 * L.g1, L2 = (2 * c14) * rl2 * L.g2, L3 = (2 * c14) * rl3 * L.g3;
-  const double R1 = (2 * c14) * rr1 * R.g1, R2 = (2 * c14) * rr2 * R.g2, R3 = (2 * c14) * rr3 * R.g3;
-  bb[0] += (2 * s6) * wl1 + D1 + L1;
-  bb[1] += (-7 * s6) * wl1 + (-s6) * wl2 + (-s6) * wr3 - 2 * D1 + D2 - 4 * L1 + L2 + R3;
-  bb[2] += (11 * s6) * wl1 + (5 * s6) * wl2 + (2 * s6) * wl3 + (2 * s6) * wr2 + (5 * s6) * wr3 + D1 - 2 * D2 + D3 +
-           3 * L1 + 3 * L3 - R2 - 4 * R3;
-  bb[3] += (2 * s6) * wl2 + (5 * s6) * wl3 + (11 * s6) * wr1 + (5 * s6) * wr2 + (2 * s6) * wr3 + D2 - 2 * D3 + D4 -
-           L2 - 4 * L3 + 3 * R1 + 3 * R3;
-  bb[4] += (-s6) * wl3 + (-7 * s6) * wr1 + (-s6) * wr2 + D3 - 2 * D4 + L3 - 4 * R1 + R2;
-  bb[5] += (2 * s6) * wr1 + D4 + R1;
+__device__ __forceinline__ void weno5_lr_vjp(const double (&D)[5], double eps34, double obL, double obR,
+                                             double (&G)[5], double &jump, double &corr) {
+  const double D1 = D[1], D2 = D[2], D3 = D[3];
+  const double e0 = D1 - D[0], e1 = D2 - D1, e2 = D3 - D2, e3 = D[4] - D3;
+  const double s0 = e0 * e0 + eps34, s1 = e1 * e1 + eps34, s2 = e2 * e2 + eps34, s3 = e3 * e3 + eps34;
+  const double k34 = scalar(0.75), k23 = scalar(2.0 / 3.0);
+  const double x1 = k34 * D1, x2 = k34 * D2, x3 = k34 * D3, F = 4.0 * D2;
+  const W5Side L = w5_side<W>(x1 * (D1 + e0) + s0, x1 * D2 + s1, x2 * (D2 - e2) + s2, k23 * e0 + D1, 2.0 * D1 + F,
+                              F - D3, (e0 + e2) - 2.0 * e1, 0.5 * obL);
+  const W5Side R = w5_side<W>(x3 * (D3 - e3) + s3, x3 * D2 + s2, x2 * (D2 + e1) + s1, D3 - k23 * e3, 2.0 * D3 + F,
+                              F - D1, (e1 + e3) - 2.0 * e2, -0.5 * obR);
+  jump = D2 - 0.5 * (R.c + L.c);
+  corr = 0.5 * (L.c - R.c);
+  // onto the e and, beside them, the D
+  double E0 = L.g1 * (2.0 * e0 + x1) + k23 * L.w1;
+  double E1 = 2.0 * e1 * (L.g2 + R.g3) + x2 * R.g3;
+  double E2 = 2.0 * e2 * (L.g3 + R.g2) - x2 * L.g3;
+  double E3 = R.g1 * (2.0 * e3 - x3) - k23 * R.w1;
+  const double B1 = L.g1 * (k34 * e0 + 2.0 * x1) + L.g2 * x2 + (L.w1 + 2.0 * L.w2 - R.w3);
+  const double B2 = L.g2 * x1 + L.g3 * (2.0 * x2 - k34 * e2) + R.g3 * (k34 * e1 + 2.0 * x2) + R.g2 * x3 +
+                    4.0 * ((L.w2 + L.w3) + (R.w2 + R.w3));
+  const double B3 = R.g1 * (2.0 * x3 - k34 * e3) + R.g2 * x2 + (R.w1 + 2.0 * R.w2 - L.w3);
   if (W == WENO_YC) {
-    const double TL = 2.0 * tl * L.gt, TR = 2.0 * tr * R.gt;
-    bb[0] += TL;
-    bb[1] += -4 * TL + TR;
-    bb[2] += 6 * TL - 4 * TR;
-    bb[3] += -4 * TL + 6 * TR;
-    bb[4] += TL - 4 * TR;
-    bb[5] += TR;
+    E0 += L.gt;
+    E1 += R.gt - 2.0 * L.gt;
+    E2 += L.gt - 2.0 * R.gt;
+    E3 += R.gt;
   }
+  G[0] = -E0;
+  G[1] = B1 + E0 - E1;
+  G[2] = B2 + E1 - E2;
+  G[3] = B3 + E2 - E3;
+  G[4] = E3;
 }
 
 // gradient of c + |v_d| of one state with respect to its conserved variables
 template <int DIR>
 __device__ __forceinline__ void speed_vjp(const double *u, double gamma, double ab, double ub[NV]) {
   const double gm1 = gamma - 1.0;
-  const double rho = u[0], ir = 1.0 / rho;
+  const double rho = u[0], ir = nr_rcp(rho);
   const double v[3] = {u[1] * ir, u[2] * ir, u[3] * ir};
   const double q2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
   const double Por = gm1 * (u[4] * ir - 0.5 * q2);  // P / rho
-  const double c = sqrt(gamma * Por);
-  const double k = ab * gamma / (2.0 * c);           // d a / d(P/rho)
+  const double k = (0.5 * ab * gamma) * nr_rsq(gamma * Por);  // d a / d(P/rho)
   ub[0] += k * gm1 * (-u[4] * ir * ir + q2 * ir);
   for (int j = 0; j < 3; j++) ub[1 + j] += k * gm1 * (-v[j] * ir);
   ub[4] += k * gm1 * ir;
@@ -252,28 +235,30 @@ __device__ __forceinline__ void roe_avg_vjp(const double *uL, const double *uR, 
                                             double gH, double ubL[NV], double ubR[NV]) {
   const double gm1 = gamma - 1.0;
   const double *U[2] = {uL, uR};
-  double t[2], v[2][3], H[2], rho[2], q2[2];
+  double t[2], v[2][3], H[2], rho[2], q2[2], ird[2], rt[2];
   for (int s = 0; s < 2; s++) {
     rho[s] = U[s][0];
-    const double ir = 1.0 / rho[s];
+    const double ir = nr_rcp(rho[s]);
+    ird[s] = ir;
     for (int j = 0; j < 3; j++) v[s][j] = U[s][1 + j] * ir;
     q2[s] = v[s][0] * v[s][0] + v[s][1] * v[s][1] + v[s][2] * v[s][2];
     H[s] = gamma * U[s][4] * ir - gm1 * 0.5 * q2[s];
-    t[s] = sqrt(rho[s]);
+    rt[s] = nr_rsq(rho[s]);
+    t[s] = sqrt_of(rho[s], rt[s]);
   }
-  const double den = 1.0 / (t[0] + t[1]);
+  const double den = nr_rcp(t[0] + t[1]);
   double va[3];
   for (int j = 0; j < 3; j++) va[j] = (t[0] * v[0][j] + t[1] * v[1][j]) * den;
   const double Ha = (t[0] * H[0] + t[1] * H[1]) * den;
   double *UB[2] = {ubL, ubR};
   for (int s = 0; s < 2; s++) {
-    const double w = t[s] * den, ir = 1.0 / rho[s];
+    const double w = t[s] * den, ir = ird[s];
     double gt = gH * (H[s] - Ha) * den;
     for (int j = 0; j < 3; j++) gt += gv[j] * (v[s][j] - va[j]) * den;
     const double gHs = gH * w;
     double gvs[3];
     for (int j = 0; j < 3; j++) gvs[j] = gv[j] * w;
-    UB[s][0] += gt / (2.0 * t[s]) + gHs * (-gamma * U[s][4] * ir * ir + gm1 * q2[s] * ir);
+    UB[s][0] += 0.5 * gt * rt[s] + gHs * (-gamma * U[s][4] * ir * ir + gm1 * q2[s] * ir);
     for (int j = 0; j < 3; j++) {
       UB[s][0] += gvs[j] * (-v[s][j] * ir);
       UB[s][1 + j] += gvs[j] * ir + gHs * (-gm1 * v[s][j] * ir);
@@ -292,29 +277,49 @@ __device__ __forceinline__ void roe_speed_vjp(const double *uL, const double *uR
     double t[2], v[2][3], H[2];
     const double *U[2] = {uL, uR};
     for (int s = 0; s < 2; s++) {
-      const double ir = 1.0 / U[s][0];
+      const double ir = nr_rcp(U[s][0]);
       for (int j = 0; j < 3; j++) v[s][j] = U[s][1 + j] * ir;
       H[s] = gamma * U[s][4] * ir - gm1 * 0.5 * (v[s][0] * v[s][0] + v[s][1] * v[s][1] + v[s][2] * v[s][2]);
-      t[s] = sqrt(U[s][0]);
+      t[s] = nr_sqrt(U[s][0]);
     }
-    const double den = 1.0 / (t[0] + t[1]);
+    const double den = nr_rcp(t[0] + t[1]);
     for (int j = 0; j < 3; j++) va[j] = (t[0] * v[0][j] + t[1] * v[1][j]) * den;
     Ha = (t[0] * H[0] + t[1] * H[1]) * den;
   }
-  const double ca = sqrt(gm1 * (Ha - 0.5 * (va[0] * va[0] + va[1] * va[1] + va[2] * va[2])));
-  const double gH = ab * gm1 / (2.0 * ca);
+  const double gH = 0.5 * ab * gm1 * nr_rsq(gm1 * (Ha - 0.5 * (va[0] * va[0] + va[1] * va[1] + va[2] * va[2])));
   double gv[3];
-  for (int j = 0; j < 3; j++) gv[j] = -ab * gm1 * va[j] / (2.0 * ca);
+  for (int j = 0; j < 3; j++) gv[j] = -gH * va[j];
   const double sg = va[DIR] > 0 ? 1.0 : (va[DIR] < 0 ? -1.0 : 0.0);
   gv[DIR] += ab * sg;
   roe_avg_vjp(uL, uR, gamma, gv, gH, ubL, ubR);
+}
+
+// Euler flux along DIR of a cell's state (navierstokes3d.h:118-139)
+template <int DIR>
+__device__ __forceinline__ void vjp_flux(const double *u, double gamma, double f[NV]) {
+  const double ir = nr_rcp(u[0]);
+  const double v[3] = {u[1] * ir, u[2] * ir, u[3] * ir};
+  const double P = (gamma - 1.0) * (u[4] - 0.5 * u[0] * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]));
+  f[0] = u[1 + DIR];
+  for (int j = 0; j < 3; j++) f[1 + j] = u[1 + DIR] * v[j];
+  f[1 + DIR] += P;
+  f[4] = (u[4] + P) * v[DIR];
+}
+
+// c + |v_d| of one state
+template <int DIR>
+__device__ __forceinline__ double vjp_speed(const double *u, double gamma) {
+  const double ir = nr_rcp(u[0]);
+  const double v[3] = {u[1] * ir, u[2] * ir, u[3] * ir};
+  const double q2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
+  return nr_sqrt(gamma * (gamma - 1.0) * (u[4] * ir - 0.5 * q2)) + fabs(v[DIR]);
 }
 
 // ub += A(u)^T fb, A = d(Euler flux along DIR)/d(conserved variables)
 template <int DIR>
 __device__ __forceinline__ void flux_jac_T(const double *u, double gamma, const double fb[NV], double ub[NV]) {
   const double gm1 = gamma - 1.0;
-  const double rho = u[0], ir = 1.0 / rho;
+  const double rho = u[0], ir = nr_rcp(rho);
   const double v[3] = {u[1] * ir, u[2] * ir, u[3] * ir};
   const double q2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
   const double P = gm1 * (u[4] - 0.5 * rho * q2);
@@ -332,28 +337,29 @@ __device__ __forceinline__ void flux_jac_T(const double *u, double gamma, const 
 // Roe state of an interface for the adjoints of Roe upwinding and of the
 // characteristic scheme, and the rows of L with their derivatives
 struct RoeAdj {
-  double v[3], vn, a, a2, ia2, ek, h0;
+  double v[3], vn, a, a2, ia, ia2, ek, h0;  // h0 = a^2/(gamma-1) + ek = the averaged enthalpy
 };
 
 template <int DIR>
 __device__ __forceinline__ RoeAdj roe_adj_state(const double uL[NV], const double uR[NV], double gamma) {
   const double gm1 = gamma - 1.0;
   RoeAdj s;
-  const double iL = 1.0 / uL[0], iR = 1.0 / uR[0];
+  const double iL = nr_rcp(uL[0]), iR = nr_rcp(uR[0]);
   double vL[3], vR[3];
   for (int j = 0; j < 3; j++) { vL[j] = uL[1 + j] * iL; vR[j] = uR[1 + j] * iR; }
   const double qL = vL[0] * vL[0] + vL[1] * vL[1] + vL[2] * vL[2];
   const double qR = vR[0] * vR[0] + vR[1] * vR[1] + vR[2] * vR[2];
   const double HL = gamma * uL[4] * iL - gm1 * 0.5 * qL, HR = gamma * uR[4] * iR - gm1 * 0.5 * qR;
-  const double tL = sqrt(uL[0]), tR = sqrt(uR[0]), den = 1.0 / (tL + tR);
+  const double tL = nr_sqrt(uL[0]), tR = nr_sqrt(uR[0]), den = nr_rcp(tL + tR);
   for (int j = 0; j < 3; j++) s.v[j] = (tL * vL[j] + tR * vR[j]) * den;
   const double H = (tL * HL + tR * HR) * den;
   s.ek = 0.5 * (s.v[0] * s.v[0] + s.v[1] * s.v[1] + s.v[2] * s.v[2]);
   s.a2 = (H - s.ek) * gm1;
-  s.a = sqrt(s.a2);
-  s.ia2 = 1.0 / s.a2;
+  s.ia = nr_rsq(s.a2);
+  s.a = sqrt_of(s.a2, s.ia);
+  s.ia2 = s.ia * s.ia;
   s.vn = s.v[DIR];
-  s.h0 = s.a2 / gm1 + s.ek;
+  s.h0 = H;
   return s;
 }
 
@@ -392,7 +398,7 @@ __device__ __forceinline__ void l_row(const RoeAdj &s, double gm1, int k, double
 template <int DIR>
 __device__ __forceinline__ void l_row_vjp(const RoeAdj &s, double gm1, int k, const double X[NV], double gv[3],
                                           double &ab) {
-  const double a = s.a, ia2 = s.ia2, ia = a * ia2, ia3 = ia2 * ia;
+  const double a = s.a, ia2 = s.ia2, ia = s.ia, ia3 = ia2 * ia;
   const double vX = s.v[0] * X[1] + s.v[1] * X[2] + s.v[2] * X[3];
   if (k == 0) {
     for (int j = 0; j < 3; j++) gv[j] += gm1 * ia2 * (X[1 + j] - X[0] * s.v[j]);
@@ -411,9 +417,15 @@ __device__ __forceinline__ void l_row_vjp(const RoeAdj &s, double gm1, int k, co
   }
 }
 
+// |l| with Harten's entropy fix, as the passes form it, and its derivative
+__device__ __forceinline__ double vjp_harten(double l) {
+  const double delta = 0.000001, delta2 = delta * delta, inv2d = 0.5 / delta;
+  const double al = fabs(l);
+  return al < delta ? (l * l + delta2) * inv2d : al;
+}
 __device__ __forceinline__ double harten_d(double l) {
   const double delta = 0.000001;
-  return fabs(l) < delta ? l / delta : (l > 0 ? 1.0 : (l < 0 ? -1.0 : 0.0));
+  return fmin(fmax(l * (1.0 / delta), -1.0), 1.0);
 }
 
 // nu (+)= (d rhs_DIR / d u)^T mu along one direction, one workgroup per line,
@@ -476,7 +488,7 @@ __device__ __forceinline__ void visc_gather_cell(const double (&us)[NV], const d
     }
   }
   const double gm1 = gamma - 1.0;
-  const double ir = 1.0 / us[0];
+  const double ir = nr_rcp(us[0]);
   const double vx = us[1] * ir, vy = us[2] * ir, vz = us[3] * ir;
   const double q2 = vx * vx + vy * vy + vz * vz;
   const double k = gamma * gm1 * qb[3];  // T = gamma (gamma-1) (e/rho - |m|^2/(2 rho^2))
@@ -538,12 +550,10 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
   else if (DIR == 1) { base = (line % nx) + (line / nx) * (size_t)nx * ny; stride = nx; }
   else { base = line; stride = (size_t)nx * ny; }
   const double *dxd = dxg + 3 + (DIR >= 1 ? nx + 6 : 0) + (DIR == 2 ? ny + 6 : 0);
-  double *sU = smem;            // [5][n]
-  double *sFl = sU + 5 * n;     // [5][n]
-  double *sC4 = sFl + 5 * n;    // [n]
-  double *cF = sC4 + n;         // [6][n]
-  double *cU = cF + 6 * n;      // [6][n]
-  const double inv_gm1 = 1.0 / (gamma - 1.0);
+  constexpr int CS = VJP_CS, ES = VJP_ES;
+  double *sC = smem;        // [n][CS]: state [5], flux [5]
+  double *E = sC + CS * n;  // [n][ES]
+  const double eps34 = 0.75 * eps;
   const int tm = active ? wrapn(t - 1, n) : 0;
   double g[NV] = {0, 0, 0, 0, 0};
   if (active) {
@@ -552,23 +562,27 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
     vjp_load_cell(u, lam, nu_in, ncell, c, us, lm, ni);
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      sU[v * n + t] = us[v];
-      // dxinv mu of this cell, staged in the (not yet used) slot buffer
-      cF[v * n + t] = dxd[t] * (cb * lm[v] + (nu_in ? ca * ni[v] : 0.0));
+      sC[t * CS + v] = us[v];
+      // dxinv mu of this cell, staged in the (not yet used) exchange buffer
+      E[t * ES + v] = dxd[t] * (cb * lm[v] + (nu_in ? ca * ni[v] : 0.0));
     }
-    const Prim q = flowvar(us, gamma);
     double fl[NV];
-    euler_flux<DIR>(fl, q);
+    vjp_flux<DIR>(us, gamma, fl);
 #pragma unroll
-    for (int v = 0; v < NV; v++) sFl[v * n + t] = fl[v];
-    sC4[t] = modified_energy(q, inv_gm1);
+    for (int v = 0; v < NV; v++) sC[t * CS + NV + v] = fl[v];
   }
   __syncthreads();
   if (active)
 #pragma unroll
-    for (int v = 0; v < NV; v++) g[v] = cF[v * n + t] - cF[v * n + tm];
+    for (int v = 0; v < NV; v++) g[v] = E[t * ES + v] - E[tm * ES + v];
   __syncthreads();
-  int cs[6];
+  const double *cs[6];  // records of the stencil's cells
+  const double *ei[6];  // exchange records that touch this cell: slot s of interface t+3-s
+#pragma unroll
+  for (int s = 0; s < 6; s++) {
+    cs[s] = sC + (active ? wrapn(t + s - 3, n) : 0) * CS;
+    ei[s] = E + (active ? wrapn(t + 3 - s, n) : 0) * ES + s;
+  }
   double alpha = 0.0, abar = 0.0;
   int sel = 0;
   // Roe: d = R |Lambda| L du with du = (uR - uL)/2 and fI = fh - d
@@ -576,25 +590,23 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
   // so that the solution WENO adjoints are -/+ wR/2
   double wR[NV] = {0, 0, 0, 0, 0}, du[NV] = {0, 0, 0, 0, 0};
   if (active && UPW == UPWIND_ROE) {
-#pragma unroll
-    for (int s = 0; s < 6; s++) cs[s] = wrapn(t + s - 3, n);
     double u2[NV], u3[NV];
 #pragma unroll
-    for (int v = 0; v < NV; v++) { u2[v] = sU[v * n + cs[2]]; u3[v] = sU[v * n + cs[3]]; }
+    for (int v = 0; v < NV; v++) { u2[v] = cs[2][v]; u3[v] = cs[3][v]; }
     const RoeAdj s = roe_adj_state<DIR>(u2, u3, gamma);
     const double gm1 = gamma - 1.0;
     const double eb = g[4];
     const double sumb = g[0] + s.v[0] * g[1] + s.v[1] * g[2] + s.v[2] * g[3];
     const double difb = g[1 + DIR] + s.vn * eb;
     double lg[5];  // (R^T lambda_F)_k |lambda_k|
-    lg[0] = (sumb + s.ek * eb) * harten_abs(s.vn);
-    lg[1] = (sumb + s.h0 * eb - s.a * difb) * harten_abs(s.vn - s.a);
-    lg[2] = (sumb + s.h0 * eb + s.a * difb) * harten_abs(s.vn + s.a);
+    lg[0] = (sumb + s.ek * eb) * vjp_harten(s.vn);
+    lg[1] = (sumb + s.h0 * eb - s.a * difb) * vjp_harten(s.vn - s.a);
+    lg[2] = (sumb + s.h0 * eb + s.a * difb) * vjp_harten(s.vn + s.a);
     if (DIR == 0) { lg[3] = -g[2] - s.v[1] * eb; lg[4] = g[3] + s.v[2] * eb; }
     else if (DIR == 1) { lg[3] = g[1] + s.v[0] * eb; lg[4] = -g[3] - s.v[2] * eb; }
     else { lg[3] = -g[1] - s.v[0] * eb; lg[4] = g[2] + s.v[1] * eb; }
-    lg[3] *= harten_abs(s.vn);
-    lg[4] *= harten_abs(s.vn);
+    lg[3] *= vjp_harten(s.vn);
+    lg[4] *= vjp_harten(s.vn);
 #pragma unroll 1
     for (int k = 0; k < 5; k++) {
       double row[NV];
@@ -605,16 +617,12 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
     }
   }
   if (active && UPW == UPWIND_RUSANOV) {
-#pragma unroll
-    for (int s = 0; s < 6; s++) cs[s] = wrapn(t + s - 3, n);
     double u2[NV], u3[NV];
 #pragma unroll
-    for (int v = 0; v < NV; v++) { u2[v] = sU[v * n + cs[2]]; u3[v] = sU[v * n + cs[3]]; }
-    const Prim q2 = flowvar(u2, gamma), q3 = flowvar(u3, gamma);
-    const Prim a = roe_average(u2, u3, gamma);
-    const double aL = sqrt(gamma * q2.P / q2.rho) + fabs(vel<DIR>(q2));
-    const double aR = sqrt(gamma * q3.P / q3.rho) + fabs(vel<DIR>(q3));
-    const double aA = sqrt(gamma * a.P / a.rho) + fabs(vel<DIR>(a));
+    for (int v = 0; v < NV; v++) { u2[v] = cs[2][v]; u3[v] = cs[3][v]; }
+    const double aL = vjp_speed<DIR>(u2, gamma), aR = vjp_speed<DIR>(u3, gamma);
+    const RoeAdj a = roe_adj_state<DIR>(u2, u3, gamma);
+    const double aA = a.a + fabs(a.vn);
     const double m01 = fmax(aL, aR), m12 = fmax(aR, aA);
     alpha = fmax(m01, m12);
     // alpha = max(max(aL,aR), max(aR,aA)): derivative of the selected term
@@ -624,28 +632,27 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
 #pragma unroll
   for (int v = 0; v < NV; v++) {
     if (active) {
-      double fb[6] = {0, 0, 0, 0, 0, 0}, ub[6] = {0, 0, 0, 0, 0, 0};
-      double F[6], U[6], C[6];
+      double D[5], G[5], jump, corr;
+      double *e = E + t * ES;
 #pragma unroll
-      for (int s = 0; s < 6; s++) {
-        F[s] = sFl[v * n + cs[s]];
-        U[s] = sU[v * n + cs[s]];
-        C[s] = v == 4 ? sC4[cs[s]] : U[s];
-      }
-      double fl, fr, uLv, uRv;
-      // fluxes: smoothness and values are the same stencil
-      weno5_lr_vjp<W>(F, F, eps, 0.5 * g[v], 0.5 * g[v], fb, fl, fr);
-      // solution: weights from u, values from the modified solution (the
-      // same function of u, so both adjoints land on u)
-      const double ob = UPW == UPWIND_ROE ? 0.5 * wR[v] : 0.5 * alpha * g[v];
-      weno5_lr_vjp<W>(U, C, eps, ob, -ob, ub, uLv, uRv);
-      if (UPW == UPWIND_ROE) du[v] = 0.5 * (uRv - uLv);
-      else abar += -0.5 * (uRv - uLv) * g[v];
-      // slot s of interface t belongs to cell t-3+s
+      for (int part = 0; part < 2; part++) {
+        // the flux, then the solution; slot s of interface t belongs to cell
+        // t-3+s and takes the adjoints of the two differences next to it
 #pragma unroll
-      for (int s = 0; s < 6; s++) {
-        cF[s * n + t] = fb[s];
-        cU[s * n + t] = ub[s];
+        for (int s = 0; s < 5; s++) D[s] = cs[s + 1][part == 0 ? NV + v : v] - cs[s][part == 0 ? NV + v : v];
+        if (part == 0) {
+          weno5_lr_vjp<W>(D, eps34, 0.5 * g[v], 0.5 * g[v], G, jump, corr);
+        } else {
+          const double ob = UPW == UPWIND_ROE ? 0.5 * wR[v] : 0.5 * alpha * g[v];
+          weno5_lr_vjp<W>(D, eps34, ob, -ob, G, jump, corr);
+          G[2] -= ob;
+          if (UPW == UPWIND_ROE) du[v] = 0.5 * jump;
+          else abar += -0.5 * jump * g[v];
+        }
+        const double mean = part == 0 ? 0.5 * g[v] : 0.0;  // the mean of the two cells' fluxes
+#pragma unroll
+        for (int s = 0; s < 6; s++)
+          e[6 * part + s] = (s > 0 ? G[s - 1] : 0.0) - (s < 5 ? G[s] : 0.0) + (s == 2 || s == 3 ? mean : 0.0);
       }
     }
     __syncthreads();
@@ -654,23 +661,22 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
     if (active) {
 #pragma unroll
       for (int s = 0; s < 6; s++) {
-        const int i = wrapn(t + 3 - s, n);
-        accF[v] += cF[s * n + i];
-        accU[v] += cU[s * n + i];
+        accF[v] += ei[s][0];
+        accU[v] += ei[s][6];
       }
     }
     __syncthreads();
   }
   // adjoint of the upwinding's dependence on the two cells next to interface
-  // t, cell t-1 (slot in cF) and cell t (slot in cU): the Rusanov speed, or
+  // t, cell t-1 (entries 0..4) and cell t (5..9): the Rusanov speed, or
   // the Roe state inside R |Lambda| L
   if (active) {
     double u2[NV], u3[NV], ub2[NV] = {0, 0, 0, 0, 0}, ub3[NV] = {0, 0, 0, 0, 0};
 #pragma unroll
-    for (int v = 0; v < NV; v++) { u2[v] = sU[v * n + cs[2]]; u3[v] = sU[v * n + cs[3]]; }
+    for (int v = 0; v < NV; v++) { u2[v] = cs[2][v]; u3[v] = cs[3][v]; }
     if (UPW == UPWIND_ROE) {
       const RoeAdj s = roe_adj_state<DIR>(u2, u3, gamma);
-      const double gm1 = gamma - 1.0;
+      const double gm1 = gamma - 1.0, igm1 = nr_rcp(gm1);
       // adjoint of d is -lambda_F; lambda_g = R^T (-lambda_F)
       double ld[NV];
 #pragma unroll
@@ -685,9 +691,9 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
       if (DIR == 0) { lgk[3] = -ld[2] - s.v[1] * eb; lgk[4] = ld[3] + s.v[2] * eb; }
       else if (DIR == 1) { lgk[3] = ld[1] + s.v[0] * eb; lgk[4] = -ld[3] - s.v[2] * eb; }
       else { lgk[3] = -ld[1] - s.v[0] * eb; lgk[4] = ld[2] + s.v[1] * eb; }
-      lam_k[0] = lam_k[3] = lam_k[4] = harten_abs(s.vn);
-      lam_k[1] = harten_abs(s.vn - s.a);
-      lam_k[2] = harten_abs(s.vn + s.a);
+      lam_k[0] = lam_k[3] = lam_k[4] = vjp_harten(s.vn);
+      lam_k[1] = vjp_harten(s.vn - s.a);
+      lam_k[2] = vjp_harten(s.vn + s.a);
       double gv[3] = {0, 0, 0}, ab = 0.0;
       // rows of L: p_k = l_k . du, g_k = |lambda_k| p_k
 #pragma unroll
@@ -708,7 +714,7 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
       const double h0b = eb * (gk[1] + gk[2]);
       const double ekb = eb * gk[0] + h0b;
       gv[DIR] += eb * s.a * (gk[2] - gk[1]);
-      ab += difb * (gk[2] - gk[1]) + h0b * 2.0 * s.a / gm1;
+      ab += difb * (gk[2] - gk[1]) + h0b * 2.0 * s.a * igm1;
       if (DIR == 0) { gv[1] -= eb * gk[3]; gv[2] += eb * gk[4]; }
       else if (DIR == 1) { gv[0] += eb * gk[3]; gv[2] -= eb * gk[4]; }
       else { gv[1] += eb * gk[4]; gv[0] -= eb * gk[3]; }
@@ -718,7 +724,7 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
       gv[DIR] += harten_d(s.vn) * (lgk[0] * pk[0] + lgk[3] * pk[3] + lgk[4] * pk[4]) + hm * lgk[1] * pk[1] +
                  hp * lgk[2] * pk[2];
       ab += hp * lgk[2] * pk[2] - hm * lgk[1] * pk[1];
-      const double ka = ab * gm1 / (2.0 * s.a);
+      const double ka = 0.5 * ab * gm1 * s.ia;
       for (int j = 0; j < 3; j++) gv[j] -= ka * s.v[j];
       roe_avg_vjp(u2, u3, gamma, gv, ka, ub2, ub3);
     } else {
@@ -728,8 +734,8 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
     }
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      cF[v * n + t] = ub2[v];
-      cU[v * n + t] = ub3[v];
+      E[t * ES + v] = ub2[v];
+      E[t * ES + NV + v] = ub3[v];
     }
   }
   __syncthreads();
@@ -738,8 +744,8 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
     double uc[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      uc[v] = sU[v * n + t];
-      accU[v] += cF[v * n + tp] + cU[v * n + t];
+      uc[v] = sC[t * CS + v];
+      accU[v] += E[tp * ES + v] + E[t * ES + NV + v];
     }
     flux_jac_T<DIR>(uc, gamma, accF, accU);
     const size_t c = base + (size_t)t * stride;
@@ -759,33 +765,30 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
 // with Harten's fix (Roe) or the Rusanov speed; this is the reference's
 // R (WENO of L f) - R |Lambda| L R (WENO of L u) with L R = I
 // (Interp1PrimFifthOrderWENOChar.c:86-198, NavierStokes3DUpwind.c:40-124).
-// The reverse pass runs field by field: WENO adjoints of the projected
-// stencils, then back through L onto the cells' fluxes and states, while the
-// derivatives of L, R and l_k with respect to the Roe state (v, a) are summed
-// and finally taken back through the Roe average onto cells I-1 and I.  The
-// interpolated values use the modified solution, which equals u exactly in
-// exact arithmetic, so both adjoints land on u.
+// As in hm_pass.hip only first differences are projected: the mean of the two
+// cells' fluxes passes L and R unchanged, so neither it nor its adjoint
+// depends on the Roe state.  The reverse pass takes the five projected fields
+// of the fluxes, then those of the states: the WENO adjoint of each field in
+// place of its differences, then point by point back through the rows of L,
+// while the derivatives of L, R and l_k with respect to the Roe state (v, a)
+// are summed and finally taken back through the Roe average onto cells I-1
+// and I.
 // longest grid line a characteristic adjoint workgroup holds: at 512 cells
 // the block is 8 wavefronts, two per SIMD (the register budget the
 // two-wave hint sets for every block size) and 88 KiB of LDS
 constexpr int VJP_CHAR_LINE_MAX = 512;
-constexpr int VJP_CHAR_CS = 11;   // doubles per cell record: state [5], flux [5], pad
-constexpr int VJP_CHAR_ES = 11;   // doubles per exchange record
+constexpr int VJP_CHAR_CS = VJP_CS;
+constexpr int VJP_CHAR_EV = 3;                    // variables exchanged at once
+constexpr int VJP_CHAR_ES = 6 * VJP_CHAR_EV + 1;  // doubles per exchange record, odd
 constexpr int VJP_CHAR_LDS = VJP_CHAR_CS + VJP_CHAR_ES;  // doubles of LDS per cell of the line
 
 // nu (+)= (d hyp_DIR-part of rhs / d u)^T mu along one direction for the
 // characteristic scheme; one workgroup per line, one thread per interface,
 // modes as k_rhs_vjp.  LDS (dynamic, VJP_CHAR_LDS doubles per cell of the
-// line), cell-major so that one address per stencil cell serves all its
-// variables through immediate offsets, with odd record lengths so that the
-// 64-bit accesses of a wave spread over all banks: a record per cell of its
-// state and flux [n][11] and an exchange record per interface [n][11].
-// The WENO5 of L f and the WENO5 of L u are taken back in two parts of five
-// fields each.  After each field k every interface posts the adjoints of its
-// six projected values and its row of L; every cell then takes the six posts
-// that touch it back through those rows, in a fixed order, so the sums are
-// deterministic.  The Roe-state derivatives of R, L and |lambda_k| are summed
-// field by field in registers.
+// line), laid out as for the component-wise scheme: a record per cell of its
+// state and flux and one per interface of its adjoints on the six stencil
+// cells, three variables at a time.  Every cell sums the six posts that touch
+// it in a fixed order, so the result is deterministic.
 template <int DIR, int UPW, int W, bool VG = false>
 __device__ __forceinline__ void rhs_vjp_char_line(
     const double *__restrict__ u, const double *__restrict__ lam, const double *__restrict__ nu_in, double ca,
@@ -801,8 +804,8 @@ __device__ __forceinline__ void rhs_vjp_char_line(
   const double *dxd = dxg + 3 + (DIR >= 1 ? nx + 6 : 0) + (DIR == 2 ? ny + 6 : 0);
   constexpr int CS = VJP_CHAR_CS, ES = VJP_CHAR_ES;
   double *sC = smem;        // [n][CS]: state [5], flux [5]
-  double *E = sC + CS * n;  // [n][ES]: six stencil adjoints [6], row of L [5]
-  const double gm1 = gamma - 1.0;
+  double *E = sC + CS * n;  // [n][ES]
+  const double gm1 = gamma - 1.0, igm1 = nr_rcp(gm1), eps34 = 0.75 * eps;
   double lF[NV] = {0, 0, 0, 0, 0};  // adjoint of the interface flux
   if (active) {
     const size_t c = base + (size_t)t * stride;
@@ -814,9 +817,8 @@ __device__ __forceinline__ void rhs_vjp_char_line(
       // dxinv mu of this cell, staged in the (not yet used) exchange buffer
       E[t * ES + v] = dxd[t] * (cb * lm[v] + (nu_in ? ca * ni[v] : 0.0));
     }
-    const Prim q = flowvar(us, gamma);
     double fl[NV];
-    euler_flux<DIR>(fl, q);
+    vjp_flux<DIR>(us, gamma, fl);
 #pragma unroll
     for (int v = 0; v < NV; v++) sC[t * CS + NV + v] = fl[v];
   }
@@ -827,156 +829,163 @@ __device__ __forceinline__ void rhs_vjp_char_line(
     for (int v = 0; v < NV; v++) lF[v] = E[t * ES + v] - E[tm * ES + v];
   }
   __syncthreads();
-  int cs[6];
+  const double *cs[6];  // records of the stencil's cells
+  const double *ei[6];  // exchange records that touch this cell: slot p of interface t+3-p
 #pragma unroll
-  for (int p = 0; p < 6; p++) cs[p] = active ? wrapn(t + p - 3, n) : 0;
+  for (int p = 0; p < 6; p++) {
+    cs[p] = sC + (active ? wrapn(t + p - 3, n) : 0) * CS;
+    ei[p] = E + (active ? wrapn(t + 3 - p, n) : 0) * ES + p * VJP_CHAR_EV;
+  }
   RoeAdj s = {};
-  double ls = 0.0, lm = 0.0, lp = 0.0, sumb = 0.0, difb = 0.0;
+  double lk[3] = {0, 0, 0};  // |lambda| of the entropy and shear, the u-a and the u+a fields
   int sel = 0;
-  const double eb = lF[4];
   if (active) {
     double u2[NV], u3[NV];
 #pragma unroll
-    for (int v = 0; v < NV; v++) { u2[v] = sC[cs[2] * CS + v]; u3[v] = sC[cs[3] * CS + v]; }
+    for (int v = 0; v < NV; v++) { u2[v] = cs[2][v]; u3[v] = cs[3][v]; }
     s = roe_adj_state<DIR>(u2, u3, gamma);
     if (UPW == UPWIND_RUSANOV) {
       // max(max(aL, aR), max(aR, aA)), the branch the forward selects
-      const Prim q2 = flowvar(u2, gamma), q3 = flowvar(u3, gamma);
-      const double aL = sqrt(gamma * q2.P / q2.rho) + fabs(vel<DIR>(q2));
-      const double aR = sqrt(gamma * q3.P / q3.rho) + fabs(vel<DIR>(q3));
+      const double aL = vjp_speed<DIR>(u2, gamma), aR = vjp_speed<DIR>(u3, gamma);
       const double aA = s.a + fabs(s.vn);
       const double m01 = fmax(aL, aR), m12 = fmax(aR, aA);
-      ls = lm = lp = fmax(m01, m12);
+      lk[0] = lk[1] = lk[2] = fmax(m01, m12);
       sel = m01 >= m12 ? (aL >= aR ? 0 : 1) : (aR >= aA ? 1 : 2);
     } else {
-      ls = harten_abs(s.vn);
-      lm = harten_abs(s.vn - s.a);
-      lp = harten_abs(s.vn + s.a);
+      lk[0] = vjp_harten(s.vn);
+      lk[1] = vjp_harten(s.vn - s.a);
+      lk[2] = vjp_harten(s.vn + s.a);
     }
-    // lambda_g = R^T lambda_F (columns of R, navierstokes3d.h:384-470)
-    sumb = lF[0] + s.v[0] * lF[1] + s.v[1] * lF[2] + s.v[2] * lF[3];
-    difb = lF[1 + DIR] + s.vn * eb;
   }
+  // the two shear fields (one row of L each: CA or CB times (x_J - v_J x_0))
+  constexpr int JA = DIR == 0 ? 1 : 0, JB = DIR == 2 ? 1 : 2;  // velocity components
+  constexpr double CA = DIR == 1 ? 1.0 : -1.0, CB = -CA;
   double gv[3] = {0, 0, 0}, ab = 0.0, alb = 0.0;
-  // part 0 takes the WENO5 of L f (left and right biased) back onto the cell
-  // fluxes, part 1 the WENO5 of L u onto the cell states; in between, the
-  // flux adjoint of every cell goes through its flux Jacobian
+  // part 0 takes the WENO5 of L f back onto the cell fluxes, part 1 the WENO5
+  // of L u onto the cell states; in between, the flux adjoint of every cell
+  // goes through its flux Jacobian
   double acc[NV] = {0, 0, 0, 0, 0};
+  auto take_back = [&](auto tag) {
+    constexpr int part = decltype(tag)::value;
+    constexpr int S = part == 0 ? NV : 0;  // flux or state within the cell record
+    double xb[5][NV];                  // adjoints of the five differences
+    if (active) {
+      const double kh = 0.5 * gm1 * s.ia2, aih = 0.5 * s.ia;
+      const double gek = kh * s.ek, avn = aih * s.vn;
+      double d[5][5];  // fields: entropy, u-a, u+a, the two shear fields
 #pragma unroll
-  for (int part = 0; part < 2; part++) {
-    const int S = part == 0 ? NV : 0;  // flux or state within the cell record
+      for (int p = 0; p < 5; p++) {
+        double x[NV];
 #pragma unroll
-    for (int k = 0; k < 5; k++) {
-      // the shear rows k = 3, 4 of L have two entries: r0 at 0 and +-1 at J
-      const bool shear = k >= 3;
-      constexpr int JA = DIR == 0 ? 2 : 1, JB = DIR == 2 ? 2 : 3;
-      constexpr double CA = DIR == 1 ? 1.0 : -1.0, CB = DIR == 1 ? -1.0 : 1.0;
-      const int J = k == 3 ? JA : JB;
-      const double cJ = k == 3 ? CA : CB;
-      if (active) {
-        double gb;  // (R^T lambda_F)_k
+        for (int v = 0; v < NV; v++) x[v] = cs[p + 1][S + v] - cs[p][S + v];
+        const double w = s.v[0] * x[1] + s.v[1] * x[2] + s.v[2] * x[3] - x[4];
+        const double h = gek * x[0] - kh * w, m = avn * x[0] - aih * x[1 + DIR];
+        d[0][p] = x[0] - 2.0 * h;
+        d[1][p] = h + m;
+        d[2][p] = h - m;
+        d[3][p] = CA * (x[1 + JA] - s.v[JA] * x[0]);
+        d[4][p] = CB * (x[1 + JB] - s.v[JB] * x[0]);
+      }
+      // (R^T lambda_F)_k (columns of R, navierstokes3d.h:384-470)
+      const double eb = lF[4];
+      const double sumb = lF[0] + s.v[0] * lF[1] + s.v[1] * lF[2] + s.v[2] * lF[3];
+      const double difb = lF[1 + DIR] + s.vn * eb;
+      double g[5];  // this part's share of g_k
+#pragma unroll
+      for (int k = 0; k < 5; k++) {
+        double gb;
         if (k == 0) gb = sumb + s.ek * eb;
         else if (k == 1) gb = sumb + s.h0 * eb - s.a * difb;
         else if (k == 2) gb = sumb + s.h0 * eb + s.a * difb;
-        else if (DIR == 0) gb = k == 3 ? -lF[2] - s.v[1] * eb : lF[3] + s.v[2] * eb;
-        else if (DIR == 1) gb = k == 3 ? lF[1] + s.v[0] * eb : -lF[3] - s.v[2] * eb;
-        else gb = k == 3 ? -lF[1] - s.v[0] * eb : lF[2] + s.v[1] * eb;
-        const double lk = k == 1 ? lm : (k == 2 ? lp : ls);
-        double row[NV], pr[6], b[6];
-        if (!shear) {
-          l_row<DIR>(s, gm1, k, row);
-#pragma unroll
-          for (int p = 0; p < 6; p++) {
-            double x = 0.0;
-#pragma unroll
-            for (int v = 0; v < NV; v++) x += row[v] * sC[cs[p] * CS + S + v];
-            pr[p] = x;
-          }
+        else if (k == 3) gb = CA * (lF[1 + JA] + s.v[JA] * eb);
+        else gb = CB * (lF[1 + JB] + s.v[JB] * eb);
+        const double l = k == 1 ? lk[1] : (k == 2 ? lk[2] : lk[0]);
+        double jump, corr;
+        if (part == 0) {
+          weno5_lr_vjp<W>(d[k], eps34, 0.5 * gb, 0.5 * gb, d[k], jump, corr);
+          g[k] = 0.5 * corr;
         } else {
-          if (DIR == 0) row[0] = k == 3 ? s.v[1] : -s.v[2];
-          else if (DIR == 1) row[0] = k == 3 ? -s.v[0] : s.v[2];
-          else row[0] = k == 3 ? s.v[0] : -s.v[1];
-#pragma unroll
-          for (int p = 0; p < 6; p++) pr[p] = row[0] * sC[cs[p] * CS + S] + cJ * sC[cs[p] * CS + S + J];
+          const double ob = 0.5 * l * gb;
+          weno5_lr_vjp<W>(d[k], eps34, ob, -ob, d[k], jump, corr);
+          d[k][2] -= ob;
+          g[k] = -0.5 * l * jump;
+          const double lb = -0.5 * jump * gb;  // adjoint of l_k: Harten's |lambda| (Roe) or the common Rusanov speed
+          if (UPW == UPWIND_ROE) {
+            const double hb = harten_d(k == 1 ? s.vn - s.a : (k == 2 ? s.vn + s.a : s.vn)) * lb;
+            gv[DIR] += hb;
+            if (k == 1) ab -= hb;
+            if (k == 2) ab += hb;
+          } else {
+            alb += lb;
+          }
         }
-        const double obL = part == 0 ? 0.5 * gb : 0.5 * lk * gb;
+        // one field at a time: interleaved, the WENO adjoints of the heavier
+        // weights do not fit the 256 registers of two waves per SIMD
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // R g at the Roe state
+      const double gsum = g[0] + g[1] + g[2], gdif = g[2] - g[1];
 #pragma unroll
-        for (int p = 0; p < 6; p++) b[p] = 0.0;
-        double wl, wr;
-        weno5_lr_vjp<W>(pr, pr, eps, obL, part == 0 ? obL : -obL, b, wl, wr);
-        // post the six adjoints and the row; X for the row's derivatives
-        double X[NV] = {0, 0, 0, 0, 0};
+      for (int j = 0; j < 3; j++) gv[j] += (lF[1 + j] + eb * s.v[j]) * gsum;
+      gv[DIR] += eb * s.a * gdif;
+      gv[JA] += CA * eb * g[3];
+      gv[JB] += CB * eb * g[4];
+      ab += difb * gdif + eb * (g[1] + g[2]) * 2.0 * s.a * igm1;
+      // back through the rows of L, and the rows' own derivatives: sums of the
+      // adjoints of h and m above against x
+      double hx0 = 0.0, hw = 0.0, mx0 = 0.0, mxd = 0.0, sa = 0.0, sb = 0.0;
+      asm volatile("" ::: "memory");  // read the records again: held, the 25 differences take 50 registers
 #pragma unroll
-        for (int p = 0; p < 6; p++) E[t * ES + p] = b[p];
-        if (!shear) {
+      for (int p = 0; p < 5; p++) {
+        double x[NV];
+#pragma unroll
+        for (int v = 0; v < NV; v++) x[v] = cs[p + 1][S + v] - cs[p][S + v];
+        const double w = s.v[0] * x[1] + s.v[1] * x[2] + s.v[2] * x[3] - x[4];
+        const double hb = (d[1][p] + d[2][p]) - 2.0 * d[0][p], mb = d[1][p] - d[2][p];
+        const double a = CA * d[3][p], b = CB * d[4][p], wb = -kh * hb;
+        hx0 += hb * x[0];
+        hw += hb * w;
+        mx0 += mb * x[0];
+        mxd += mb * x[1 + DIR];
+        sa += a * x[0];
+        sb += b * x[0];
+#pragma unroll
+        for (int j = 0; j < 3; j++) gv[j] += wb * x[1 + j];
+        xb[p][0] = d[0][p] + gek * hb + avn * mb - s.v[JA] * a - s.v[JB] * b;
+#pragma unroll
+        for (int j = 0; j < 3; j++) xb[p][1 + j] = s.v[j] * wb;
+        xb[p][1 + DIR] -= aih * mb;
+        xb[p][1 + JA] += a;
+        xb[p][1 + JB] += b;
+        xb[p][4] = -wb;
+      }
+      // h = kh (ek x_0 - w), m = aih (v_d x_0 - x_d), kh = (gamma-1)/(2a^2), aih = 1/(2a)
+      const double khb = s.ek * hx0 - hw, ekb = kh * hx0;
+#pragma unroll
+      for (int j = 0; j < 3; j++) gv[j] += s.v[j] * ekb;
+      gv[DIR] += aih * mx0;
+      gv[JA] -= sa;
+      gv[JB] -= sb;
+      ab -= s.ia * (2.0 * kh * khb + aih * (s.vn * mx0 - mxd));
+    }
+    // post the adjoints of the six cells (differences of those of the
+    // differences, and in part 0 the mean of the two cells' fluxes), take the
+    // posts that touch this cell
+#pragma unroll
+    for (int v0 = 0; v0 < NV; v0 += VJP_CHAR_EV) {
+      if (active)
+#pragma unroll
+        for (int v = v0; v < NV && v < v0 + VJP_CHAR_EV; v++)
 #pragma unroll
           for (int p = 0; p < 6; p++)
-#pragma unroll
-            for (int v = 0; v < NV; v++) X[v] += b[p] * sC[cs[p] * CS + S + v];
-#pragma unroll
-          for (int v = 0; v < NV; v++) E[t * ES + 6 + v] = row[v];
-        } else {
-          // only r0 depends on the Roe state
-#pragma unroll
-          for (int p = 0; p < 6; p++) X[0] += b[p] * sC[cs[p] * CS + S];
-          E[t * ES + 6] = row[0];
-        }
-        // this part's share of the forward g_k = (fL + fR)/2 - l_k (uR - uL)/2
-        const double gk = part == 0 ? 0.5 * (wl + wr) : -0.5 * lk * (wr - wl);
-        // term k of R g at the Roe state
-        if (k < 3) {
-#pragma unroll
-          for (int j = 0; j < 3; j++) gv[j] += (lF[1 + j] + eb * s.v[j]) * gk;
-          if (k > 0) {
-            const double sg = k == 2 ? 1.0 : -1.0;
-            gv[DIR] += sg * eb * s.a * gk;
-            ab += sg * difb * gk + eb * gk * 2.0 * s.a / gm1;
-          }
-        } else if (DIR == 0) {
-          if (k == 3) gv[1] -= eb * gk; else gv[2] += eb * gk;
-        } else if (DIR == 1) {
-          if (k == 3) gv[0] += eb * gk; else gv[2] -= eb * gk;
-        } else {
-          if (k == 3) gv[0] -= eb * gk; else gv[1] += eb * gk;
-        }
-        // l_k: Harten's |lambda| (Roe) or the common Rusanov speed
-        if (part == 1) {
-          const double lbk = -0.5 * (wr - wl) * gb;  // adjoint of l_k
-          if (UPW == UPWIND_ROE) {
-            if (k == 1) { const double h = harten_d(s.vn - s.a) * lbk; gv[DIR] += h; ab -= h; }
-            else if (k == 2) { const double h = harten_d(s.vn + s.a) * lbk; gv[DIR] += h; ab += h; }
-            else gv[DIR] += harten_d(s.vn) * lbk;
-          } else {
-            alb += lbk;
-          }
-        }
-        l_row_vjp<DIR>(s, gm1, k, X, gv, ab);
-      }
+            E[t * ES + p * VJP_CHAR_EV + v - v0] = (p > 0 ? xb[p - 1][v] : 0.0) - (p < 5 ? xb[p][v] : 0.0) +
+                                                   (part == 0 && (p == 2 || p == 3) ? 0.5 * lF[v] : 0.0);
       __syncthreads();
-      // cell t takes post p of interface t+3-p, p = 0..5, back through that
-      // interface's row
-      if (active) {
-        if (!shear) {
+      if (active)
 #pragma unroll
-          for (int p = 0; p < 6; p++) {
-            const double *e = E + wrapn(t + 3 - p, n) * ES;
-            const double bp = e[p];
+        for (int v = v0; v < NV && v < v0 + VJP_CHAR_EV; v++)
 #pragma unroll
-            for (int v = 0; v < NV; v++) acc[v] += bp * e[6 + v];
-          }
-        } else {
-          double bsum = 0.0;
-#pragma unroll
-          for (int p = 0; p < 6; p++) {
-            const double *e = E + wrapn(t + 3 - p, n) * ES;
-            const double bp = e[p];
-            acc[0] += bp * e[6];
-            bsum += bp;
-          }
-          acc[JA] += (k == 3 ? CA : 0.0) * bsum;
-          acc[JB] += (k == 4 ? CB : 0.0) * bsum;
-        }
-      }
+          for (int p = 0; p < 6; p++) acc[v] += ei[p][v - v0];
       __syncthreads();
     }
     if (part == 0 && active) {
@@ -987,19 +996,21 @@ __device__ __forceinline__ void rhs_vjp_char_line(
 #pragma unroll
       for (int v = 0; v < NV; v++) acc[v] = ub[v];
     }
-  }
+  };
+  take_back(std::integral_constant<int, 0>{});
+  take_back(std::integral_constant<int, 1>{});
   // the Roe state's (and the Rusanov speed's) dependence on cells t-1 and t
   if (active) {
     double u2[NV], u3[NV], ub2[NV] = {0, 0, 0, 0, 0}, ub3[NV] = {0, 0, 0, 0, 0};
 #pragma unroll
-    for (int v = 0; v < NV; v++) { u2[v] = sC[cs[2] * CS + v]; u3[v] = sC[cs[3] * CS + v]; }
+    for (int v = 0; v < NV; v++) { u2[v] = cs[2][v]; u3[v] = cs[3][v]; }
     if (UPW == UPWIND_RUSANOV) {
       if (sel == 0) speed_vjp<DIR>(u2, gamma, alb, ub2);
       else if (sel == 1) speed_vjp<DIR>(u3, gamma, alb, ub3);
       else roe_speed_vjp<DIR>(u2, u3, gamma, alb, ub2, ub3);
     }
     // a = sqrt((H - |v|^2/2)(gamma-1)) -> (v, H) of the Roe average -> the two cells
-    const double ka = ab * gm1 / (2.0 * s.a);
+    const double ka = 0.5 * ab * gm1 * s.ia;
     for (int j = 0; j < 3; j++) gv[j] -= ka * s.v[j];
     roe_avg_vjp(u2, u3, gamma, gv, ka, ub2, ub3);
 #pragma unroll
@@ -1172,7 +1183,7 @@ __device__ __forceinline__ void visc_vjp_tile(const double *__restrict__ Q, cons
         gr[c][2] = d4c(q[0][c], q[1][c], q[3][c], q[4][c]) * dz[k];
       }
       const double qc[4] = {q[2][0], q[2][1], q[2][2], q[2][3]};
-      const double mu = exp(0.76 * log(qc[3]));
+      const double mu = pow076(qc[3]);
       double qb[4] = {0, 0, 0, 0}, grb[4][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, mub = 0.0;
       // direction by direction: reader r = pos - s reads this cell's flux
       // with weight d4w(s) dxinv(r), inside the grid only
@@ -1194,7 +1205,7 @@ __device__ __forceinline__ void visc_vjp_tile(const double *__restrict__ Q, cons
         else if (d == 1) mub += visc_flux_vjp<1>(qc, gr, mu, vc, fb, qb, grb);
         else mub += visc_flux_vjp<2>(qc, gr, mu, vc, fb, qb, grb);
       }
-      qb[3] += mub * (0.76 * mu / qc[3]);
+      qb[3] += mub * (0.76 * mu * nr_rcp(qc[3]));
       const size_t idx = pk + col;
       const double dxe[3] = {dx[i], dy[j], dz[k]};
 #pragma unroll
@@ -1279,10 +1290,10 @@ __device__ __forceinline__ void visc_vjp_ghost_line(const double *__restrict__ Q
       for (int e = 0; e < 3; e++) gr[c][e] = e == DIR ? d * dxgh : 0.0;
     }
     const double q[4] = {w[3][0], w[3][1], w[3][2], w[3][3]};
-    const double mu = exp(0.76 * log(q[3]));
+    const double mu = pow076(q[3]);
     double qb[4] = {0, 0, 0, 0}, grb[4][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
     const double mub = visc_flux_vjp<DIR>(q, gr, mu, vc, fb, qb, grb);
-    qb[3] += mub * (0.76 * mu / q[3]);
+    qb[3] += mub * (0.76 * mu * nr_rcp(q[3]));
 #pragma unroll
     for (int c = 0; c < 4; c++) acc[slot + 3][c] += qb[c];
 #pragma unroll

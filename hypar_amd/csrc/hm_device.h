@@ -41,6 +41,14 @@ __device__ __forceinline__ Prim flowvar(const double *u, double gamma) {
   return q;
 }
 
+// A constant held in scalar registers: without it the compiler folds the
+// constant into the two-address fused multiply-add and copies the addend
+// first (one extra instruction each time).
+__device__ __forceinline__ double scalar(double c) {
+  asm("" : "+s"(c));
+  return c;
+}
+
 // 1/d, d > 0 and normal, from the hardware estimate r: with e = 1 - d r,
 // r + r (e + e^2) leaves an error of e^3.  The estimate's e is at most 4.7e-8
 // (measured over 4 million arguments, mantissas over the whole range), so

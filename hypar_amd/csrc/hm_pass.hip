@@ -133,14 +133,6 @@ __device__ __forceinline__ void cell_data(const double u[NV], const PassConst &k
   if (UPW == UPWIND_RUSANOV) c[11] = nr_sqrt(k.gamma * P * ir) + fabs(vn);
 }
 
-// A constant held in scalar registers: without it the compiler folds the
-// constant into the two-address fused multiply-add and copies the addend
-// first (one extra instruction each time).
-__device__ __forceinline__ double scalar(double c) {
-  asm("" : "+s"(c));
-  return c;
-}
-
 // One side of WENO5 at an interface: twice the difference between the
 // interpolated value and the value of the upwind cell next to the interface
 // (include/interpolation.h:265-500, Interp1PrimFifthOrderWENO.c:146-158).
