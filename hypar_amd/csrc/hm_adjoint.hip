@@ -41,28 +41,55 @@ constexpr int VJP_LDS = VJP_CS + VJP_ES;  // doubles of LDS per cell of the comp
 __device__ __forceinline__ int wrapn(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
 // Lines per workgroup of the line VJPs: a block of `threads` threads (a
-// multiple of 64, at least n) takes threads / n consecutive lines of length
-// n, so that lines shorter than the block do not leave wavefronts idle (two
-// 64-cell lines per 128-thread block).
+// multiple of 64, at least n) takes threads / n consecutive lines of length n.
 __host__ __device__ __forceinline__ int vjp_lines_per_block(int threads, int n) { return threads / n; }
 
-// the line and interface of this thread for work item `item` (a group of
-// vjp_lines_per_block lines) of a direction with nlines lines of length n;
-// sub is the thread's line within the group, whose share of the dynamic LDS
-// starts sub * (doubles per cell) * n in.  live is false for threads past the
-// group's last line.
+// Threads of a block for lines of length n: of the blocks of at most 256
+// threads the one whose lanes are busiest, the larger of equals.  More lines
+// per block leave fewer lanes idle (a 66-cell line alone fills half of two
+// wavefronts) and make the y and z lines' accesses of neighbouring lanes
+// neighbours in x.  Lines over 256 cells take a block each.  At 256 threads
+// the characteristic kernel's LDS (240 B per thread) leaves two blocks per CU,
+// the two wavefronts per SIMD its registers allow.
+inline int vjp_threads(int n) {
+  if (n > 256) return (n + 63) / 64 * 64;
+  int best = 0;
+  double eff = 0.0;
+  for (int t = (n + 63) / 64 * 64; t <= 256; t += 64) {
+    const double e = (double)(t / n * n) / t;
+    if (e >= eff) {
+      eff = e;
+      best = t;
+    }
+  }
+  return best;
+}
+
+// This thread's place in work item `item` (a group of lines = threads / n
+// consecutive lines) of a direction with nlines lines of length n.  Threads
+// run through the lines of the group first and along the line second, and so
+// do their LDS records: thread r holds cell and interface t of line
+// item * lines + r % lines in record r, and the record k places further along
+// the line is r + k lines, wrapped at size = lines * n.  live is false for
+// threads past the group's last line.
 struct LineSlot {
   size_t line;
-  int t, sub;
+  int t, r, lines, size;
   bool live;
+  __device__ __forceinline__ int at(int k) const {
+    const int i = r + k * lines;
+    return i < 0 ? i + size : (i >= size ? i - size : i);
+  }
 };
 __device__ __forceinline__ LineSlot line_slot(size_t item, int n, size_t nlines) {
-  const int lpb = vjp_lines_per_block((int)blockDim.x, n), sub = (int)threadIdx.x / n;
   LineSlot s;
-  s.line = item * lpb + sub;
-  s.live = sub < lpb && s.line < nlines;
-  s.t = (int)threadIdx.x - sub * n;
-  s.sub = s.live ? sub : 0;
+  s.lines = vjp_lines_per_block((int)blockDim.x, n);
+  s.size = s.lines * n;
+  const int r = (int)threadIdx.x, t = r / s.lines;
+  s.line = item * s.lines + (r - t * s.lines);
+  s.live = r < s.size && s.line < nlines;
+  s.t = s.live ? t : 0;
+  s.r = s.live ? r : 0;
   if (!s.live) s.line = 0;
   return s;
 }
@@ -541,20 +568,20 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
                                              double *__restrict__ nu, double *__restrict__ L, int mode, int nx,
                                              int ny, int nz, const double *__restrict__ dxg, double gamma,
                                              double eps, const double *__restrict__ QB,
-                                             const double *__restrict__ GB, size_t line, int t, bool active,
-                                             double *smem) {
+                                             const double *__restrict__ GB, const LineSlot &sl, double *smem) {
+  const size_t line = sl.line;
+  const int t = sl.t, r0 = sl.r;
+  const bool active = sl.live;
   const size_t ncell = (size_t)nx * ny * nz;
-  const int n = DIR == 0 ? nx : (DIR == 1 ? ny : nz);
   size_t base, stride;
   if (DIR == 0) { base = line * nx; stride = 1; }
   else if (DIR == 1) { base = (line % nx) + (line / nx) * (size_t)nx * ny; stride = nx; }
   else { base = line; stride = (size_t)nx * ny; }
   const double *dxd = dxg + 3 + (DIR >= 1 ? nx + 6 : 0) + (DIR == 2 ? ny + 6 : 0);
   constexpr int CS = VJP_CS, ES = VJP_ES;
-  double *sC = smem;        // [n][CS]: state [5], flux [5]
-  double *E = sC + CS * n;  // [n][ES]
+  double *sC = smem;        // [sl.size][CS]: state [5], flux [5]
+  double *E = sC + CS * sl.size;  // [sl.size][ES]
   const double eps34 = 0.75 * eps;
-  const int tm = active ? wrapn(t - 1, n) : 0;
   double g[NV] = {0, 0, 0, 0, 0};
   if (active) {
     const size_t c = base + (size_t)t * stride;
@@ -562,26 +589,26 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
     vjp_load_cell(u, lam, nu_in, ncell, c, us, lm, ni);
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      sC[t * CS + v] = us[v];
+      sC[r0 * CS + v] = us[v];
       // dxinv mu of this cell, staged in the (not yet used) exchange buffer
-      E[t * ES + v] = dxd[t] * (cb * lm[v] + (nu_in ? ca * ni[v] : 0.0));
+      E[r0 * ES + v] = dxd[t] * (cb * lm[v] + (nu_in ? ca * ni[v] : 0.0));
     }
     double fl[NV];
     vjp_flux<DIR>(us, gamma, fl);
 #pragma unroll
-    for (int v = 0; v < NV; v++) sC[t * CS + NV + v] = fl[v];
+    for (int v = 0; v < NV; v++) sC[r0 * CS + NV + v] = fl[v];
   }
   __syncthreads();
   if (active)
 #pragma unroll
-    for (int v = 0; v < NV; v++) g[v] = E[t * ES + v] - E[tm * ES + v];
+    for (int v = 0; v < NV; v++) g[v] = E[r0 * ES + v] - E[sl.at(-1) * ES + v];
   __syncthreads();
   const double *cs[6];  // records of the stencil's cells
   const double *ei[6];  // exchange records that touch this cell: slot s of interface t+3-s
 #pragma unroll
   for (int s = 0; s < 6; s++) {
-    cs[s] = sC + (active ? wrapn(t + s - 3, n) : 0) * CS;
-    ei[s] = E + (active ? wrapn(t + 3 - s, n) : 0) * ES + s;
+    cs[s] = sC + sl.at(s - 3) * CS;
+    ei[s] = E + sl.at(3 - s) * ES + s;
   }
   double alpha = 0.0, abar = 0.0;
   int sel = 0;
@@ -633,7 +660,7 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
   for (int v = 0; v < NV; v++) {
     if (active) {
       double D[5], G[5], jump, corr;
-      double *e = E + t * ES;
+      double *e = E + r0 * ES;
 #pragma unroll
       for (int part = 0; part < 2; part++) {
         // the flux, then the solution; slot s of interface t belongs to cell
@@ -734,18 +761,18 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
     }
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      E[t * ES + v] = ub2[v];
-      E[t * ES + NV + v] = ub3[v];
+      E[r0 * ES + v] = ub2[v];
+      E[r0 * ES + NV + v] = ub3[v];
     }
   }
   __syncthreads();
   if (active) {
-    const int tp = wrapn(t + 1, n);
+    const int tp = sl.at(1);
     double uc[NV];
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      uc[v] = sC[t * CS + v];
-      accU[v] += E[tp * ES + v] + E[t * ES + NV + v];
+      uc[v] = sC[r0 * CS + v];
+      accU[v] += E[tp * ES + v] + E[r0 * ES + NV + v];
     }
     flux_jac_T<DIR>(uc, gamma, accF, accU);
     const size_t c = base + (size_t)t * stride;
@@ -794,17 +821,19 @@ __device__ __forceinline__ void rhs_vjp_char_line(
     const double *__restrict__ u, const double *__restrict__ lam, const double *__restrict__ nu_in, double ca,
     double cb, double *__restrict__ nu, double *__restrict__ L, int mode, int nx, int ny, int nz,
     const double *__restrict__ dxg, double gamma, double eps, const double *__restrict__ QB,
-    const double *__restrict__ GB, size_t line, int t, bool active, double *smem) {
+    const double *__restrict__ GB, const LineSlot &sl, double *smem) {
+  const size_t line = sl.line;
+  const int t = sl.t, r0 = sl.r;
+  const bool active = sl.live;
   const size_t ncell = (size_t)nx * ny * nz;
-  const int n = DIR == 0 ? nx : (DIR == 1 ? ny : nz);
   size_t base, stride;
   if (DIR == 0) { base = line * nx; stride = 1; }
   else if (DIR == 1) { base = (line % nx) + (line / nx) * (size_t)nx * ny; stride = nx; }
   else { base = line; stride = (size_t)nx * ny; }
   const double *dxd = dxg + 3 + (DIR >= 1 ? nx + 6 : 0) + (DIR == 2 ? ny + 6 : 0);
   constexpr int CS = VJP_CHAR_CS, ES = VJP_CHAR_ES;
-  double *sC = smem;        // [n][CS]: state [5], flux [5]
-  double *E = sC + CS * n;  // [n][ES]
+  double *sC = smem;        // [sl.size][CS]: state [5], flux [5]
+  double *E = sC + CS * sl.size;  // [sl.size][ES]
   const double gm1 = gamma - 1.0, igm1 = nr_rcp(gm1), eps34 = 0.75 * eps;
   double lF[NV] = {0, 0, 0, 0, 0};  // adjoint of the interface flux
   if (active) {
@@ -813,28 +842,27 @@ __device__ __forceinline__ void rhs_vjp_char_line(
     vjp_load_cell(u, lam, nu_in, ncell, c, us, lm, ni);
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      sC[t * CS + v] = us[v];
+      sC[r0 * CS + v] = us[v];
       // dxinv mu of this cell, staged in the (not yet used) exchange buffer
-      E[t * ES + v] = dxd[t] * (cb * lm[v] + (nu_in ? ca * ni[v] : 0.0));
+      E[r0 * ES + v] = dxd[t] * (cb * lm[v] + (nu_in ? ca * ni[v] : 0.0));
     }
     double fl[NV];
     vjp_flux<DIR>(us, gamma, fl);
 #pragma unroll
-    for (int v = 0; v < NV; v++) sC[t * CS + NV + v] = fl[v];
+    for (int v = 0; v < NV; v++) sC[r0 * CS + NV + v] = fl[v];
   }
   __syncthreads();
   if (active) {
-    const int tm = wrapn(t - 1, n);
 #pragma unroll
-    for (int v = 0; v < NV; v++) lF[v] = E[t * ES + v] - E[tm * ES + v];
+    for (int v = 0; v < NV; v++) lF[v] = E[r0 * ES + v] - E[sl.at(-1) * ES + v];
   }
   __syncthreads();
   const double *cs[6];  // records of the stencil's cells
   const double *ei[6];  // exchange records that touch this cell: slot p of interface t+3-p
 #pragma unroll
   for (int p = 0; p < 6; p++) {
-    cs[p] = sC + (active ? wrapn(t + p - 3, n) : 0) * CS;
-    ei[p] = E + (active ? wrapn(t + 3 - p, n) : 0) * ES + p * VJP_CHAR_EV;
+    cs[p] = sC + sl.at(p - 3) * CS;
+    ei[p] = E + sl.at(3 - p) * ES + p * VJP_CHAR_EV;
   }
   RoeAdj s = {};
   double lk[3] = {0, 0, 0};  // |lambda| of the entropy and shear, the u-a and the u+a fields
@@ -978,7 +1006,7 @@ __device__ __forceinline__ void rhs_vjp_char_line(
         for (int v = v0; v < NV && v < v0 + VJP_CHAR_EV; v++)
 #pragma unroll
           for (int p = 0; p < 6; p++)
-            E[t * ES + p * VJP_CHAR_EV + v - v0] = (p > 0 ? xb[p - 1][v] : 0.0) - (p < 5 ? xb[p][v] : 0.0) +
+            E[r0 * ES + p * VJP_CHAR_EV + v - v0] = (p > 0 ? xb[p - 1][v] : 0.0) - (p < 5 ? xb[p][v] : 0.0) +
                                                    (part == 0 && (p == 2 || p == 3) ? 0.5 * lF[v] : 0.0);
       __syncthreads();
       if (active)
@@ -991,7 +1019,7 @@ __device__ __forceinline__ void rhs_vjp_char_line(
     if (part == 0 && active) {
       double uc[NV], ub[NV] = {0, 0, 0, 0, 0};
 #pragma unroll
-      for (int v = 0; v < NV; v++) uc[v] = sC[t * CS + v];
+      for (int v = 0; v < NV; v++) uc[v] = sC[r0 * CS + v];
       flux_jac_T<DIR>(uc, gamma, acc, ub);
 #pragma unroll
       for (int v = 0; v < NV; v++) acc[v] = ub[v];
@@ -1015,21 +1043,21 @@ __device__ __forceinline__ void rhs_vjp_char_line(
     roe_avg_vjp(u2, u3, gamma, gv, ka, ub2, ub3);
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      E[t * ES + v] = ub2[v];
-      E[t * ES + NV + v] = ub3[v];
+      E[r0 * ES + v] = ub2[v];
+      E[r0 * ES + NV + v] = ub3[v];
     }
   }
   __syncthreads();
   if (active) {
-    const int tp = wrapn(t + 1, n);
+    const int tp = sl.at(1);
 #pragma unroll
-    for (int v = 0; v < NV; v++) acc[v] += E[tp * ES + v] + E[t * ES + NV + v];
+    for (int v = 0; v < NV; v++) acc[v] += E[tp * ES + v] + E[r0 * ES + NV + v];
     const size_t c = base + (size_t)t * stride;
     double vb[NV] = {0, 0, 0, 0, 0};
     if (VG) {
       double uc[NV];
 #pragma unroll
-      for (int v = 0; v < NV; v++) uc[v] = sC[t * CS + v];
+      for (int v = 0; v < NV; v++) uc[v] = sC[r0 * CS + v];
       visc_gather_cell(uc, QB, GB, nx, ny, nz, gamma, c, vb);
     }
     vjp_store(nu, L, lam, mode, ncell, c, acc, VG, vb);
@@ -1323,8 +1351,7 @@ __global__ void __launch_bounds__(VJP_LINE_MAX) k_rhs_vjp(const double *__restri
   extern __shared__ double smem[];
   const int n = DIR == 0 ? nx : (DIR == 1 ? ny : nz);
   const LineSlot s = line_slot(xcd_block(), n, (size_t)nx * ny * nz / n);
-  rhs_vjp_line<DIR, UPW, W, VG>(u, lam, nu_in, ca, cb, nu, L, mode, nx, ny, nz, dxg, gamma, eps, QB, GB, s.line,
-                                s.t, s.live, smem + (size_t)s.sub * VJP_LDS * n);
+  rhs_vjp_line<DIR, UPW, W, VG>(u, lam, nu_in, ca, cb, nu, L, mode, nx, ny, nz, dxg, gamma, eps, QB, GB, s, smem);
 }
 
 template <int DIR, int UPW, int W, bool VG>
@@ -1336,8 +1363,7 @@ __global__ void __launch_bounds__(VJP_CHAR_LINE_MAX) __attribute__((amdgpu_waves
   extern __shared__ double smem[];
   const int n = DIR == 0 ? nx : (DIR == 1 ? ny : nz);
   const LineSlot s = line_slot(xcd_block(), n, (size_t)nx * ny * nz / n);
-  rhs_vjp_char_line<DIR, UPW, W, VG>(u, lam, nu_in, ca, cb, nu, L, mode, nx, ny, nz, dxg, gamma, eps, QB, GB,
-                                     s.line, s.t, s.live, smem + (size_t)s.sub * VJP_CHAR_LDS * n);
+  rhs_vjp_char_line<DIR, UPW, W, VG>(u, lam, nu_in, ca, cb, nu, L, mode, nx, ny, nz, dxg, gamma, eps, QB, GB, s, smem);
 }
 
 __global__ void __launch_bounds__(VT) k_visc_vjp_tile(const double *__restrict__ Q, const double *__restrict__ lam,
@@ -1422,8 +1448,7 @@ __global__ void __launch_bounds__(VJP_LINE_MAX) k_ens_rhs_vjp(EnsVjp a, const un
     const int m = ens_find(first, a.nmem, item);
     const EnsMember M = a.mem[m];
     const LineSlot s = line_slot(item - first[m], M.n[DIR], M.ncell / M.n[DIR]);
-    rhs_vjp_line<DIR, UPW, W, VG>(ENS_MEMBER_ARGS(a, M), s.line, s.t, s.live,
-                                  smem + (size_t)s.sub * VJP_LDS * M.n[DIR]);
+    rhs_vjp_line<DIR, UPW, W, VG>(ENS_MEMBER_ARGS(a, M), s, smem);
     __syncthreads();
   }
 }
@@ -1437,8 +1462,7 @@ __global__ void __launch_bounds__(VJP_CHAR_LINE_MAX) __attribute__((amdgpu_waves
     const int m = ens_find(first, a.nmem, item);
     const EnsMember M = a.mem[m];
     const LineSlot s = line_slot(item - first[m], M.n[DIR], M.ncell / M.n[DIR]);
-    rhs_vjp_char_line<DIR, UPW, W, VG>(ENS_MEMBER_ARGS(a, M), s.line, s.t, s.live,
-                                       smem + (size_t)s.sub * VJP_CHAR_LDS * M.n[DIR]);
+    rhs_vjp_char_line<DIR, UPW, W, VG>(ENS_MEMBER_ARGS(a, M), s, smem);
     __syncthreads();
   }
 }
@@ -1534,7 +1558,7 @@ template <int DIR>
 static void launch_vjp_dir(const Grid &g, const Scheme &sc, const double *u, const double *lam, const double *nu_in,
                            double ca, double cb, double *nu, double *L, int mode, const double *dxg, hipStream_t st,
                            const double *QB = nullptr, const double *GB = nullptr) {
-  const unsigned threads = (unsigned)((g.n[DIR] + 63) / 64 * 64);
+  const unsigned threads = (unsigned)vjp_threads(g.n[DIR]);
   const unsigned lpb = (unsigned)vjp_lines_per_block((int)threads, g.n[DIR]);
   const unsigned lines = (unsigned)((g.ncell / g.n[DIR] + lpb - 1) / lpb);  // work items
   with_scheme(sc, [&](auto tag) {
@@ -1599,7 +1623,7 @@ bool ens_vjp_supported(const Scheme &sc, const int nmax[3]) {
 
 size_t ens_vjp_work_size(const Scheme &sc, size_t ncell) { return sc.Re > 0 ? 20 * ncell : 0; }
 
-int ens_vjp_threads(int nmax) { return (nmax + 63) / 64 * 64; }
+int ens_vjp_threads(int nmax) { return nmax <= 256 ? 256 : vjp_threads(nmax); }
 int ens_vjp_lines_per_item(int nmax, int n) { return vjp_lines_per_block(ens_vjp_threads(nmax), n); }
 
 template <int DIR>
