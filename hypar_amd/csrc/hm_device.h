@@ -94,12 +94,12 @@ __device__ __forceinline__ double pow076(double T) {
   const double f = m - 1.0, d = m + 1.0, r = nr_rcp(d);
   const double s = f * r, sl = __builtin_fma(-s, d, f) * r, z = s * s;
   double p = 0.21367029765733125;
-  p = __builtin_fma(p, z, 0.2209119995397776);
-  p = __builtin_fma(p, z, 0.2623343930169728);
-  p = __builtin_fma(p, z, 0.32059853416893563);
-  p = __builtin_fma(p, z, 0.41219858584787455);
-  p = __builtin_fma(p, z, 0.5770780163454895);
-  p = __builtin_fma(p, z, 0.9617966939259898);
+  p = __builtin_fma(p, z, scalar(0.2209119995397776));
+  p = __builtin_fma(p, z, scalar(0.2623343930169728));
+  p = __builtin_fma(p, z, scalar(0.32059853416893563));
+  p = __builtin_fma(p, z, scalar(0.41219858584787455));
+  p = __builtin_fma(p, z, scalar(0.5770780163454895));
+  p = __builtin_fma(p, z, scalar(0.9617966939259898));
   const double c0 = 2.8853900817779268;
   const double l = c0 * s;
   const double ll = __builtin_fma(s * z, p, __builtin_fma(c0, sl, __builtin_fma(c0, s, -l)));
@@ -109,16 +109,16 @@ __device__ __forceinline__ double pow076(double T) {
   const double n = __builtin_rint(y);
   const double g = (y - n) + lo;
   double q = 4.4558179083360645e-10;
-  q = __builtin_fma(q, g, 7.074194297288521e-09);
-  q = __builtin_fma(q, g, 1.0178057087733941e-07);
-  q = __builtin_fma(q, g, 1.3215432535912375e-06);
-  q = __builtin_fma(q, g, 1.5252733841556773e-05);
-  q = __builtin_fma(q, g, 0.00015403530463724353);
-  q = __builtin_fma(q, g, 0.001333355814640647);
-  q = __builtin_fma(q, g, 0.009618129107587256);
-  q = __builtin_fma(q, g, 0.055504108664821625);
-  q = __builtin_fma(q, g, 0.24022650695910158);
-  q = __builtin_fma(q, g, 0.6931471805599453);
+  q = __builtin_fma(q, g, scalar(7.074194297288521e-09));
+  q = __builtin_fma(q, g, scalar(1.0178057087733941e-07));
+  q = __builtin_fma(q, g, scalar(1.3215432535912375e-06));
+  q = __builtin_fma(q, g, scalar(1.5252733841556773e-05));
+  q = __builtin_fma(q, g, scalar(0.00015403530463724353));
+  q = __builtin_fma(q, g, scalar(0.001333355814640647));
+  q = __builtin_fma(q, g, scalar(0.009618129107587256));
+  q = __builtin_fma(q, g, scalar(0.055504108664821625));
+  q = __builtin_fma(q, g, scalar(0.24022650695910158));
+  q = __builtin_fma(q, g, scalar(0.6931471805599453));
   q = __builtin_fma(q, g, 1.0);
   q = __builtin_ldexp(q, (int)n);
   const double other = T < 0.0 ? __builtin_nan("") : T;

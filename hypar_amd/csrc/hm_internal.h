@@ -130,6 +130,7 @@ __host__ __device__ inline unsigned visc_tiles(int nx, int ny, int nz) {
 // tiles of the viscous-term kernel (hm_kernels.hip): a block owns PTX x PTY
 // (x, y) columns and marches through a z segment of pks planes
 constexpr int PTX = 32, PTY = 16;
+constexpr int PAR_THREADS = PTX * PTY + 4 * PTX + 4 * PTY;  // the tile's columns and its halo points
 __host__ __device__ inline unsigned par_tiles(int nx, int ny, int nz, int pks) {
   return (unsigned)(((nx + PTX - 1) / PTX) * ((ny + PTY - 1) / PTY) * ((nz + pks - 1) / pks));
 }

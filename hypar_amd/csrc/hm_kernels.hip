@@ -89,33 +89,36 @@ __device__ __forceinline__ void visc_flux(double fv[4], const QT &q, const doubl
 // ghost-layer fluxes where its stencils need them.
 //
 // A block owns a TX x TY tile of (x, y) columns and marches through the
-// planes of one z segment [k0, k1) (pks planes).  Plane q of Q with a
-// 4-cell halo in x and y is staged in LDS.  Every thread evaluates the
-// gradient at its own column and at most one halo point (the rows y0-2,
-// y0-1, y0+TY, y0+TY+1 and the columns x0-2, x0-1, x0+TX, x0+TX+1 of the
-// tile), taking the z derivative from a ring of that point's values on
-// planes q-2..q+2 held in registers (in a thread-private part of LDS for
-// the halo point).  The next plane's loads are issued before the current
-// plane's arithmetic and stored to LDS after it.  The x and y fluxes of plane q go to
-// LDS, where their x and y differences are formed.  The z flux of plane q
-// goes at once into the sums of the planes q-2..q+2 whose z difference reads
-// it, five running sums per component, to which the x + y part of plane q is
-// added; the sum of plane q-2 is then complete.  The z differences of the
-// segment need FVz on planes k0-2..k1+1, so the march covers them; on the
-// ghost planes (-2, -1, nz, nz+1) the z flux comes from direct loads of the
-// column.
+// planes of one z segment [k0, k1) (pks planes).  A thread evaluates the
+// gradient and the fluxes of one point: a column of the tile, or one of the
+// halo points whose x or y flux the tile's differences read (the rows y0-2,
+// y0-1, y0+TY, y0+TY+1 and the columns x0-2, x0-1, x0+TX, x0+TX+1); the halo
+// points take whole wavefronts.  A thread holds its point's values on planes
+// q-2..q+2 in registers: the z derivative comes from there, and the plane q+1
+// among them is what it stages in LDS for the others' x and y derivatives in
+// the next step, so only the 208 points beyond those of the block's threads
+// are loaded for LDS alone.  The x and y fluxes of plane q go to LDS, where
+// their x and y differences are formed.  Plane and fluxes are double-buffered,
+// which leaves one barrier per plane.  The z flux of plane q goes at once into
+// the sums of the planes q-2..q+2 whose z difference reads it, five running
+// sums per component, to which the x + y part of plane q is added; the sum of
+// plane q-2 is then complete.  The z differences of the segment need FVz on
+// planes k0-2..k1+1, so the march covers them; on the ghost planes (-2, -1,
+// nz, nz+1) the z flux comes from direct loads of the column.
 //
-// Vector issue and LDS bandwidth bound it (two waves per SIMD, 100 KB of LDS
-// per block).  Running sums in place of a flux ring and a buffer of x + y
-// parts, index arithmetic kept out of the march and pow076 took the 256^3
-// launch from 0.67 to 0.50 ms, and with the segment rule of visc_segment the
-// 64^3 one from 87 to 23 us and the 16x12x20 one from 91 to 16 us.
+// LDS bandwidth (3000 cycles per plane and CU) and vector issue (3200) bound
+// it, hardly overlapped because the block's wavefronts go through them
+// together: 3.3 us per plane.  Tiles of 16 x 16, two blocks per CU, took 603 us
+// at 256^3, this one 437 us; a form with 512 threads, two barriers per plane
+// and the halo points evaluated after the columns by some of the threads, 497
+// us (before that, with log and exp, a flux ring and a buffer of x + y parts,
+// 670 us).  64^3 takes 21 us, 16x12x20 14 us (87 and 91 us with segments of 16
+// planes and more).
 template <int TX, int TY>
 struct ViscParShared {
-  double q[4][TY + 8][TX + 8];  // plane q of Q: x0-4..x0+TX+3, y0-4..y0+TY+3
-  double fx[4][TY][TX + 4];     // x fluxes of the tile's rows at x0-2..x0+TX+1
-  double fy[4][TY + 4][TX];     // y fluxes of the tile's columns at y0-2..y0+TY+1
-  double hr[5][4][4 * TX + 4 * TY];  // z ring of each halo point, slot advancing with the plane
+  double q[2][4][TY + 8][TX + 8];  // a plane of Q: x0-4..x0+TX+3, y0-4..y0+TY+3
+  double fx[2][4][TY][TX + 4];     // x fluxes of the tile's rows at x0-2..x0+TX+1
+  double fy[2][4][TY + 4][TX];     // y fluxes of the tile's columns at y0-2..y0+TY+1
 };
 
 __device__ __forceinline__ int wrapi(int p, int n) {
@@ -123,17 +126,13 @@ __device__ __forceinline__ int wrapi(int p, int n) {
   return r < 0 ? r + n : r;
 }
 
-// d/dx_d of one primitive at the ghost position of slot s (0..3 for the
-// positions -2, -1, n, n+1) from f(o), its values at offsets o from that
-// position along d (periodic copies); not yet scaled by dxinv.  Only the
-// offsets a slot's stencil uses are read: -1..3 (slot 0), -3..1 (slot 3),
-// -2..2 (slots 1, 2).
-template <class F>
-__device__ __forceinline__ double ghost_deriv(int slot, const F &f) {
-  const double r12 = 1.0 / 12.0;
-  if (slot == 0) return (-3 * f(-1) - 10 * f(0) + 18 * f(1) - 6 * f(2) + f(3)) * r12;
-  if (slot == 3) return (-f(-3) + 6 * f(-2) - 18 * f(-1) + 10 * f(0) + 3 * f(1)) * r12;
-  return d4c(f(-2), f(-1), f(1), f(2));
+// Stencil of d/dx_d at the ghost position of slot s (0..3 for the positions
+// -2, -1, n, n+1): 12 times the weights of the five points from offset
+// ghost_first(slot) on (periodic copies).
+__device__ __forceinline__ int ghost_first(int slot) { return slot == 0 ? -1 : (slot == 3 ? -3 : -2); }
+__device__ __forceinline__ double ghost_weight(int slot, int k) {
+  const double lo[5] = {-3, -10, 18, -6, 1}, hi[5] = {-1, 6, -18, 10, 3}, mid[5] = {1, -8, 0, 8, -1};
+  return slot == 0 ? lo[k] : (slot == 3 ? hi[k] : mid[k]);
 }
 
 // Viscous flux along DIR at a ghost position: derivative along DIR only
@@ -162,8 +161,7 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
                                               int ny, int nz,
                                               const double *__restrict__ dxg,  // ghosted dxinv x|y|z
                                               const ViscParams &vp, int b, int pks, ViscParShared<TX, TY> &sh) {
-  constexpr int NT = TX * TY;
-  static_assert(4 * TX + 4 * TY <= NT, "every halo point needs a thread");
+  static_assert(TX * TY % 64 == 0 && 4 * TX % 64 == 0, "each kind of point takes whole wavefronts");
   const size_t ncell = (size_t)nx * ny * nz;
   const size_t plane = (size_t)nx * ny;
   const int ntx = (nx + TX - 1) / TX, nty = (ny + TY - 1) / TY;
@@ -172,268 +170,201 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
   const int k1 = min(k0 + pks, nz);
   const double *dxa = dxg, *dya = dxg + (nx + 6), *dza = dxg + (nx + 6) + (ny + 6);  // entry 3+p: position p
   const int t = threadIdx.x;
-  const int lx = t % TX, ly = t / TX;
-  const int i = x0 + lx, j = y0 + ly;
-  const bool own = i < nx && j < ny;
-  const size_t col = (size_t)wrapi(j, ny) * nx + wrapi(i, nx);
-  // halo point: y fluxes of rows y0-2, y0-1, y0+TY, y0+TY+1 (threads
-  // 0..4*TX-1), x fluxes of columns x0-2, x0-1, x0+TX, x0+TX+1 (the next
-  // 4*TY threads)
-  int hkind = -1, hx = 0, hy = 0;
-  if (t < 4 * TX) {
-    const int r = t / TX;
-    hkind = 1;
-    hx = t % TX;
-    hy = r < 2 ? r - 2 : TY + r - 2;
-  } else if (t < 4 * TX + 4 * TY) {
-    const int u = t - 4 * TX, r = u % 4;
-    hkind = 0;
-    hy = u / 4;
-    hx = r < 2 ? r - 2 : TX + r - 2;
+  // this thread's point: 2 a column of the tile, 1 a halo row's, 0 a halo column's
+  const int wt = __builtin_amdgcn_readfirstlane(t);
+  const int kind = wt < TX * TY ? 2 : (wt < TX * TY + 4 * TX ? 1 : 0);
+  int ox, oy;
+  if (kind == 2) {
+    ox = t % TX;
+    oy = t / TX;
+  } else if (kind == 1) {
+    const int u = t - TX * TY, r = u / TX;
+    ox = u % TX;
+    oy = r < 2 ? r - 2 : TY + r - 2;
+  } else {
+    const int u = t - TX * TY - 4 * TX, r = u % 4;
+    ox = r < 2 ? r - 2 : TX + r - 2;
+    oy = u / 4;
   }
-  const int hi = x0 + hx, hj = y0 + hy;
-  const size_t hcol = (size_t)wrapi(hj, ny) * nx + wrapi(hi, nx);
-  // does the halo point carry a flux the tile needs, and is it interior?
-  const bool hneed = hkind == 1 ? (hi < nx && hj >= -2 && hj < ny + 2)
-                                : (hkind == 0 && hj < ny && hi >= -2 && hi < nx + 2);
-  const bool hint = hkind == 1 ? (hj >= 0 && hj < ny) : (hi >= 0 && hi < nx);
-
+  const int i = x0 + ox, j = y0 + oy;
+  const size_t col = (size_t)wrapi(j, ny) * nx + wrapi(i, nx);
+  const bool inx = i >= 0 && i < nx, iny = j >= 0 && j < ny;
+  const bool own = kind == 2 && inx && iny;
+  // does the tile read this point's x (y) flux; it is a ghost-layer flux where
+  // the point lies beyond the grid along x (y)
+  const bool wantx = kind != 1 && iny && i < nx + 2, wanty = kind != 0 && inx && j < ny + 2;
+  const bool regular = inx && iny && (wantx || wanty);
   const double r12 = 1.0 / 12.0;
-  const double odx = own ? dxa[3 + i] * r12 : 0.0, ody = own ? dya[3 + j] * r12 : 0.0;
-  const double hdx = hneed && hint ? dxa[3 + hi] * r12 : 0.0, hdy = hneed && hint ? dya[3 + hj] * r12 : 0.0;
+  const double dxi = regular ? dxa[3 + i] * r12 : 0.0, dyi = regular ? dya[3 + j] * r12 : 0.0;
+
+  // a further point of the staged plane, beyond those of the block's threads:
+  // rows y0-4, y0-3, y0+TY+2, y0+TY+3, columns alike, and the 16 points
+  // across the corners
+  const int e = t >= TX * TY ? t - TX * TY : (t < 16 ? 4 * TX + 4 * TY + t : -1);
+  int ex = 0, ey = 0;
+  if (e >= 0 && e < 4 * TX) {
+    const int r = e / TX;
+    ex = e % TX;
+    ey = r < 2 ? r - 4 : TY + r;
+  } else if (e >= 0 && e < 4 * TX + 4 * TY) {
+    const int u = e - 4 * TX, r = u % 4;
+    ex = r < 2 ? r - 4 : TX + r;
+    ey = u / 4;
+  } else if (e >= 0) {
+    const int u = e - 4 * TX - 4 * TY, r = u % 4, w = u / 4;
+    ex = r < 2 ? r - 2 : TX + r - 2;
+    ey = w < 2 ? w - 2 : TY + w - 2;
+  }
+  const size_t ecol = (size_t)wrapi(y0 + ey, ny) * nx + wrapi(x0 + ex, nx);
 
   auto ldq = [&](size_t c, int k, double (&r)[4]) {  // k in [-4, nz + 4]
     const size_t o = (size_t)wrap(k, nz) * plane + c;
 #pragma unroll
     for (int v = 0; v < 4; v++) r[v] = Q[(size_t)v * ncell + o];
   };
-  // Q on LDS at tile offsets (ox, oy) (-4 <= ox < TX + 4, -4 <= oy < TY + 4)
-  auto sq = [&](int v, int oy, int ox) { return sh.q[v][oy + 4][ox + 4]; };
-  auto qat = [&](int ox, int oy) {
-    QT q;
-    q.u = sq(0, oy, ox);
-    q.v = sq(1, oy, ox);
-    q.w = sq(2, oy, ox);
-    q.T = sq(3, oy, ox);
-    return q;
-  };
-  // gradient at tile offset (ox, oy) of interior plane q; zr(s, v) is
-  // component v on plane q-2+s of the point
-  // dxi, dyi: the point's dxinv and dyinv over 12
-  auto grad = [&](int ox, int oy, int q, double dxi, double dyi, const auto &zr, double (&gr)[4][3]) {
-    const double dzi = dza[3 + q] * r12;
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      gr[v][0] = d4u(sq(v, oy, ox - 2), sq(v, oy, ox - 1), sq(v, oy, ox + 1), sq(v, oy, ox + 2)) * dxi;
-      gr[v][1] = d4u(sq(v, oy - 2, ox), sq(v, oy - 1, ox), sq(v, oy + 1, ox), sq(v, oy + 2, ox)) * dyi;
-      gr[v][2] = d4u(zr(0, v), zr(1, v), zr(3, v), zr(4, v)) * dzi;
-    }
-  };
-  // ghost-layer x / y flux at tile offset (ox, oy)
-  auto ghost_x = [&](int ox, int oy, double mu) {
-    const int gx = x0 + ox, slot = gx < 0 ? gx + 2 : gx - nx + 2;
-    double d[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++) d[v] = ghost_deriv(slot, [&](int o) { return sq(v, oy, ox + o); }) * dxa[3 + gx];
-    double fv[4];
-    ghost_flux<0>(fv, qat(ox, oy), d, mu, vp);
-#pragma unroll
-    for (int v = 0; v < 4; v++) sh.fx[v][oy][ox + 2] = fv[v];
-  };
-  auto ghost_y = [&](int ox, int oy, double mu) {
-    const int gy = y0 + oy, slot = gy < 0 ? gy + 2 : gy - ny + 2;
-    double d[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++) d[v] = ghost_deriv(slot, [&](int o) { return sq(v, oy + o, ox); }) * dya[3 + gy];
-    double fv[4];
-    ghost_flux<1>(fv, qat(ox, oy), d, mu, vp);
-#pragma unroll
-    for (int v = 0; v < 4; v++) sh.fy[v][oy + 2][ox] = fv[v];
-  };
 
-  // staging of plane q into LDS: every thread takes NR points of the
-  // (TX + 8) x (TY + 8) region; the loads are issued a plane ahead into
-  // registers and stored once the previous plane's reads are done
-  constexpr int NQP = (TX + 8) * (TY + 8), NR = (NQP + NT - 1) / NT;
-  double pre[NR][4];
-  int so[NR];  // offset of the point within a plane
+  // planes q-2..q+2 of the point, plane q+1 of the further point, and the
+  // sums of planes q-2..q+1 so far
+  double rq[5][4], pe[4] = {0.0, 0.0, 0.0, 0.0}, sum[4][4];
 #pragma unroll
-  for (int r = 0; r < NR; r++) {
-    const int c = min(t + r * NT, NQP - 1);
-    so[r] = wrapi(y0 - 4 + c / (TX + 8), ny) * nx + wrapi(x0 - 4 + c % (TX + 8), nx);
-  }
-  auto fetch_plane = [&](int q) {
-    const size_t pk = (size_t)q * plane;
+  for (int s = 0; s < 5; s++) ldq(col, k0 - 4 + s, rq[s]);
+  if (e >= 0) ldq(ecol, k0 - 2, pe);
 #pragma unroll
-    for (int r = 0; r < NR; r++)
-      if (t + r * NT < NQP)
+  for (int s = 0; s < 4; s++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) pre[r][v] = Q[(size_t)v * ncell + pk + so[r]];
+    for (int v = 0; v < 4; v++) sum[s][v] = 0.0;
+  int buf = 0;
+  auto stage = [&](int bq, const double (&r)[4]) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) sh.q[bq][v][oy + 4][ox + 4] = r[v];
+    if (e >= 0)
+#pragma unroll
+      for (int v = 0; v < 4; v++) sh.q[bq][v][ey + 4][ex + 4] = pe[v];
   };
-  auto store_plane = [&]() {
-#pragma unroll
-    for (int r = 0; r < NR; r++) {
-      const int c = t + r * NT;
-      if (c < NQP)
-#pragma unroll
-        for (int v = 0; v < 4; v++) (&sh.q[v][0][0])[c] = pre[r][v];
-    }
-  };
-
-  // rings of planes q-2..q+2 of the own column (registers) and the halo
-  // point (LDS; plane p of the march in slot (p - k0 + 4) mod 5), and the
-  // next plane of each, loaded a step ahead
-  double rq[5][4], nq[4], nh[4];
-  double sum[5][4];  // running sums of planes q-2..q+2
-  int h5 = 0;        // slot of plane q-2
-  auto hslot = [&](int s, int v) -> double & {  // plane q-2+s
-    const int p = h5 + s;
-    return sh.hr[p >= 5 ? p - 5 : p][v][t];
-  };
-#pragma unroll
-  for (int s = 0; s < 5; s++)
-#pragma unroll
-    for (int v = 0; v < 4; v++) rq[s][v] = sum[s][v] = 0.0;
-#pragma unroll
-  for (int v = 0; v < 4; v++) nh[v] = 0.0;
-#pragma unroll
-  for (int s = 0; s < 4; s++) {
-    ldq(col, k0 - 4 + s, rq[s + 1]);
-    if (hkind >= 0) {
-      double r[4];
-      ldq(hcol, k0 - 4 + s, r);
-#pragma unroll
-      for (int v = 0; v < 4; v++) hslot(s, v) = r[v];
-    }
-  }
-  ldq(col, k0, nq);
-  if (hkind >= 0) ldq(hcol, k0, nh);
-  if (k0 - 2 >= 0) {  // the first plane of the march, unless a ghost plane
-    fetch_plane(k0 - 2);
-    store_plane();
-  }
+  stage(buf, rq[2]);  // plane k0-2
+  if (e >= 0) ldq(ecol, k0 - 1, pe);
+  __syncthreads();
   for (int q = k0 - 2; q < k1 + 2; q++) {
+    const bool gz = q < 0 || q >= nz;     // a ghost plane along z (uniform)
+    const bool outq = q >= k0 && q < k1;  // a plane whose x and y terms are formed
+    // the middle entries hold the periodic copy of every point, also beyond
+    // the grid, so one evaluation serves interior and ghost fluxes
+    const QT qv = {rq[2][0], rq[2][1], rq[2][2], rq[2][3]};
+    const double mu = pow076(qv.T);
+    double fzq[4] = {0.0, 0.0, 0.0, 0.0};
+    if (gz) {
+      if (own) {
+        const int slot = q < 0 ? q + 2 : q - nz + 2, o0 = ghost_first(slot);
+        double d[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 5; k++) {
+          double r[4];
+          ldq(col, q + o0 + k, r);
+          const double w = ghost_weight(slot, k) * (r12 * dza[3 + q]);
+#pragma unroll
+          for (int v = 0; v < 4; v++) d[v] += w * r[v];
+        }
+        ghost_flux<2>(fzq, qv, d, mu, vp);
+      }
+    } else {
+      // Q on LDS at offsets (a, c) from the point
+      auto sq = [&](int v, int a, int c) { return sh.q[buf][v][oy + 4 + c][ox + 4 + a]; };
+      double fv[4];
+      if (regular && (outq || kind == 2)) {
+        double gr[4][3];
+        const double dzi = dza[3 + q] * r12;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          gr[v][0] = d4u(sq(v, -2, 0), sq(v, -1, 0), sq(v, 1, 0), sq(v, 2, 0)) * dxi;
+          gr[v][1] = d4u(sq(v, 0, -2), sq(v, 0, -1), sq(v, 0, 1), sq(v, 0, 2)) * dyi;
+          gr[v][2] = d4u(rq[0][v], rq[1][v], rq[3][v], rq[4][v]) * dzi;
+        }
+        if (kind == 2) visc_flux<2>(fzq, qv, gr, mu, vp);
+        if (outq && kind != 1) {
+          visc_flux<0>(fv, qv, gr, mu, vp);
+#pragma unroll
+          for (int v = 0; v < 4; v++) sh.fx[buf][v][oy][ox + 2] = fv[v];
+        }
+        if (outq && kind != 0) {
+          visc_flux<1>(fv, qv, gr, mu, vp);
+#pragma unroll
+          for (int v = 0; v < 4; v++) sh.fy[buf][v][oy + 2][ox] = fv[v];
+        }
+      }
+      // ghost-layer fluxes: x at i = -2, -1, nx, nx+1, y at j = -2, -1, ny, ny+1
+      if (outq && wantx && !inx) {
+        const int slot = i < 0 ? i + 2 : i - nx + 2, o0 = ghost_first(slot);
+        double d[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 5; k++) {
+          const double w = ghost_weight(slot, k) * (r12 * dxa[3 + i]);
+#pragma unroll
+          for (int v = 0; v < 4; v++) d[v] += w * sq(v, o0 + k, 0);
+        }
+        ghost_flux<0>(fv, qv, d, mu, vp);
+#pragma unroll
+        for (int v = 0; v < 4; v++) sh.fx[buf][v][oy][ox + 2] = fv[v];
+      }
+      if (outq && wanty && !iny) {
+        const int slot = j < 0 ? j + 2 : j - ny + 2, o0 = ghost_first(slot);
+        double d[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 5; k++) {
+          const double w = ghost_weight(slot, k) * (r12 * dya[3 + j]);
+#pragma unroll
+          for (int v = 0; v < 4; v++) d[v] += w * sq(v, 0, o0 + k);
+        }
+        ghost_flux<1>(fv, qv, d, mu, vp);
+#pragma unroll
+        for (int v = 0; v < 4; v++) sh.fy[buf][v][oy + 2][ox] = fv[v];
+      }
+    }
+    // stage plane q+1; the loads for the next plane are in flight during the
+    // barrier and the differences
+    stage(buf ^ 1, rq[3]);
 #pragma unroll
     for (int s = 0; s < 4; s++)
 #pragma unroll
       for (int v = 0; v < 4; v++) rq[s][v] = rq[s + 1][v];
-#pragma unroll
-    for (int v = 0; v < 4; v++) rq[4][v] = nq[v];
-    if (hkind >= 0)
-#pragma unroll
-      for (int v = 0; v < 4; v++) hslot(4, v) = nh[v];
-    const bool gz = q < 0 || q >= nz;     // a ghost plane along z (uniform)
-    const bool outq = q >= k0 && q < k1;  // a plane whose x and y terms are formed
-    const bool next = q + 1 < k1 + 2 && q + 1 >= 0 && q + 1 < nz;  // plane q+1 is staged
-    __syncthreads();
-    if (next) fetch_plane(q + 1);
     if (q + 1 < k1 + 2) {
-      ldq(col, q + 3, nq);
-      if (hkind >= 0) ldq(hcol, q + 3, nh);
+      ldq(col, q + 3, rq[4]);
+      if (e >= 0) ldq(ecol, q + 2, pe);
     }
-    double fzq[4] = {0.0, 0.0, 0.0, 0.0};
-    // the ring's middle entries hold the periodic copy of every point, also
-    // beyond the grid, so one evaluation serves interior and ghost fluxes
-    double mu = pow076(rq[2][3]);
-    if (gz) {
-      if (own) {
-        const int slot = q < 0 ? q + 2 : q - nz + 2;
-        double d[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-          d[v] = ghost_deriv(slot, [&](int o) { return Q[(size_t)v * ncell + (size_t)wrap(q + o, nz) * plane + col]; }) *
-                 dza[3 + q];
-        const size_t o = (size_t)wrap(q, nz) * plane + col;
-        QT qv;
-        qv.u = Q[o];
-        qv.v = Q[ncell + o];
-        qv.w = Q[2 * ncell + o];
-        qv.T = Q[3 * ncell + o];
-        ghost_flux<2>(fzq, qv, d, mu, vp);
-      }
-    } else {
-      if (own) {
-        double gr[4][3];
-        grad(lx, ly, q, odx, ody, [&](int s2, int v) { return rq[s2][v]; }, gr);
-        const QT qv = qat(lx, ly);
-        visc_flux<2>(fzq, qv, gr, mu, vp);
-        if (outq) {
-          double fv[4];
-          visc_flux<0>(fv, qv, gr, mu, vp);
-#pragma unroll
-          for (int v = 0; v < 4; v++) sh.fx[v][ly][lx + 2] = fv[v];
-          visc_flux<1>(fv, qv, gr, mu, vp);
-#pragma unroll
-          for (int v = 0; v < 4; v++) sh.fy[v][ly + 2][lx] = fv[v];
-        }
-      } else if (outq) {
-        // the column lies past the grid: ghost-layer x flux at i = nx, nx+1
-        // (rows inside), ghost-layer y flux at j = ny, ny+1 (columns inside)
-        if (j < ny && i < nx + 2) ghost_x(lx, ly, mu);
-        if (i < nx && j < ny + 2) ghost_y(lx, ly, mu);
-      }
-      if (outq && hneed) {
-        mu = pow076(hslot(2, 3));
-        if (hint) {
-          double gr[4][3];
-          grad(hx, hy, q, hdx, hdy, [&](int s2, int v) { return hslot(s2, v); }, gr);
-          const QT qv = qat(hx, hy);
-          double fv[4];
-          if (hkind == 0) {
-            visc_flux<0>(fv, qv, gr, mu, vp);
-#pragma unroll
-            for (int v = 0; v < 4; v++) sh.fx[v][hy][hx + 2] = fv[v];
-          } else {
-            visc_flux<1>(fv, qv, gr, mu, vp);
-#pragma unroll
-            for (int v = 0; v < 4; v++) sh.fy[v][hy + 2][hx] = fv[v];
-          }
-        } else if (hkind == 0) {
-          ghost_x(hx, hy, mu);
-        } else {
-          ghost_y(hx, hy, mu);
-        }
-      }
-    }
-    // plane p = q-2+s reads FVz(q) with weight -1/12, 8/12, 0, -8/12, 1/12
-    // times its dzinv (planes outside the segment are not stored; their
-    // metric index is clamped into the array)
-    {
+    __syncthreads();
+    if (kind == 2) {
+      // plane p = q-2+s reads FVz(q) with weight -1/12, 8/12, 0, -8/12, 1/12
+      // times its dzinv (planes outside the segment are not stored; their
+      // metric index is clamped into the array)
       const double z0 = -r12 * dza[3 + max(q - 2, -3)], z1 = 8.0 * r12 * dza[3 + max(q - 1, -3)];
       const double z3 = -8.0 * r12 * dza[3 + min(q + 1, nz + 2)], z4 = r12 * dza[3 + min(q + 2, nz + 2)];
+      if (q - 2 >= k0 && own) {  // the sum of plane q-2 is now complete
+        const size_t o = (size_t)(q - 2) * plane + col;
+#pragma unroll
+        for (int v = 0; v < 4; v++) par[(size_t)v * ncell + o] = sum[0][v] + z0 * fzq[v];
+      }
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        sum[0][v] += z0 * fzq[v];
-        sum[1][v] += z1 * fzq[v];
-        sum[3][v] += z3 * fzq[v];
-        sum[4][v] = z4 * fzq[v];
+        sum[0][v] = sum[1][v] + z1 * fzq[v];
+        sum[1][v] = sum[2][v];
+        sum[2][v] = sum[3][v] + z3 * fzq[v];
+        sum[3][v] = z4 * fzq[v];
+      }
+      if (outq && own) {
+        const auto &fx = sh.fx[buf];
+        const auto &fy = sh.fy[buf];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          const double px = dxi * d4u(fx[v][oy][ox], fx[v][oy][ox + 1], fx[v][oy][ox + 3], fx[v][oy][ox + 4]);
+          const double py = dyi * d4u(fy[v][oy][ox], fy[v][oy + 1][ox], fy[v][oy + 3][ox], fy[v][oy + 4][ox]);
+          sum[1][v] += px + py;
+        }
       }
     }
-    __syncthreads();
-    if (next) store_plane();  // nothing reads plane q from LDS any more
-    if (outq && own) {
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        const double px = odx * d4u(sh.fx[v][ly][lx], sh.fx[v][ly][lx + 1], sh.fx[v][ly][lx + 3], sh.fx[v][ly][lx + 4]);
-        const double py = ody * d4u(sh.fy[v][ly][lx], sh.fy[v][ly + 1][lx], sh.fy[v][ly + 3][lx], sh.fy[v][ly + 4][lx]);
-        sum[2][v] += px + py;
-      }
-    }
-    const int p = q - 2;  // plane whose sum is now complete
-    if (p >= k0 && own) {
-      const size_t o = (size_t)p * plane + col;
-#pragma unroll
-      for (int v = 0; v < 4; v++) par[(size_t)v * ncell + o] = sum[0][v];
-    }
-#pragma unroll
-    for (int s = 0; s < 4; s++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) sum[s][v] = sum[s + 1][v];
-    h5 = h5 == 4 ? 0 : h5 + 1;
+    buf ^= 1;
   }
 }
 
-__global__ void __launch_bounds__(PTX * PTY) k_visc_par(const double *__restrict__ Q, double *__restrict__ par,
+__global__ void __launch_bounds__(PAR_THREADS) k_visc_par(const double *__restrict__ Q, double *__restrict__ par,
                                                          int nx, int ny, int nz, int pks,
                                                          const double *__restrict__ dxg, ViscParams vp) {
   __shared__ ViscParShared<PTX, PTY> sh;
@@ -451,7 +382,7 @@ struct EnsViscArgs {
   ViscParams vp;
 };
 
-__global__ void __launch_bounds__(PTX * PTY) k_ens_visc(EnsViscArgs a) {
+__global__ void __launch_bounds__(PAR_THREADS) k_ens_visc(EnsViscArgs a) {
   __shared__ ViscParShared<PTX, PTY> sh;
   const unsigned item = blockIdx.x;  // one block per item (a loop over items spills 8 B per lane)
   if (item >= a.nitems) return;
@@ -640,7 +571,7 @@ int visc_segment(int count, const int (*n)[3]) {
 void launch_visc_par(const Grid &g, const Scheme &sc, const double *Q, double *par, const double *dxg,
                      hipStream_t st) {
   const unsigned nb = par_tiles(g.n[0], g.n[1], g.n[2], g.pks);
-  hipLaunchKernelGGL(k_visc_par, dim3(nb), dim3(PTX * PTY), 0, st, Q, par, g.n[0], g.n[1], g.n[2], g.pks, dxg,
+  hipLaunchKernelGGL(k_visc_par, dim3(nb), dim3(PAR_THREADS), 0, st, Q, par, g.n[0], g.n[1], g.n[2], g.pks, dxg,
                      visc_params(sc));
 }
 
@@ -653,7 +584,7 @@ void launch_ens_visc(const Scheme &sc, const EnsMember *mem, int nmem, const uns
   a.ptiles0 = ptiles0;
   a.nitems = nitems;
   a.vp = visc_params(sc);
-  hipLaunchKernelGGL(k_ens_visc, dim3(nitems), dim3(PTX * PTY), 0, st, a);
+  hipLaunchKernelGGL(k_ens_visc, dim3(nitems), dim3(PAR_THREADS), 0, st, a);
 }
 
 void launch_ens_prims(const Scheme &sc, const EnsMember *mem, int nmem, const double *u, size_t ncell,
