@@ -730,8 +730,13 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
   }
 }
 
+// three waves per SIMD (168 registers; left alone the characteristic passes
+// take 170-194 and two waves), except with the mapped weights, which would
+// spill 20 registers and more
+constexpr int x_waves(int interp, int weno) { return interp == INTERP_CHAR && weno == WENO_MAPPED ? 2 : 3; }
+
 template <int INTERP, int UPW, int W>
-__global__ void __launch_bounds__(256) k_pass_x(PassConst k, PassIO io) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(x_waves(INTERP, W)))) k_pass_x(PassConst k, PassIO io) {
   __shared__ XShared<4, UPW> sh;
   pass_x_body<INTERP, UPW, 4, W>(k, io, blockIdx.x, sh);
 }
@@ -805,7 +810,7 @@ __device__ __forceinline__ void ens_setup(const EnsArgs &a, int m, int dir, Pass
 }
 
 template <int INTERP, int UPW, int LPB, int W>
-__global__ void __launch_bounds__(64 * LPB) k_ens_x(EnsArgs a) {
+__global__ void __launch_bounds__(64 * LPB) __attribute__((amdgpu_waves_per_eu(x_waves(INTERP, W)))) k_ens_x(EnsArgs a) {
   __shared__ XShared<LPB, UPW> sh;
   for (unsigned item = blockIdx.x; item < a.nitems; item += gridDim.x) {
     const int m = ens_member(a, item);
