@@ -75,8 +75,8 @@ size_t auto_tape_budget(size_t held_bytes) {
 
 struct hm_solver {
   hm_solver() : g(), sc(), device(0), stream(nullptr), dxg(nullptr), R(nullptr), par(nullptr), Q(nullptr),
-                S{nullptr, nullptr},
-                acc(nullptr), part(nullptr), part_host(nullptr), npart(0), tmp(nullptr), tmp_elems(0),
+                S{nullptr, nullptr, nullptr},
+                part(nullptr), part_host(nullptr), npart(0), tmp(nullptr), tmp_elems(0),
                 tape_nsteps(0), tape_every(0), tape_dt(0.0) {
     for (int i = 0; i < TAPE_SETS; i++) tape_holds[i] = -1;
   }
@@ -88,8 +88,7 @@ struct hm_solver {
   double *R;          // hyperbolic-term accumulator of the passes, 5*ncell
   double *par;        // viscous term, 4*ncell (viscous runs only)
   double *Q;          // primitive variables u, v, w, T, 4*ncell (viscous only)
-  double *S[2];       // RK stage states (double-buffered)
-  double *acc;        // RK accumulator
+  double *S[3];       // RK stage states
   double *part;       // reduction partials (device)
   double *part_host;  // reduction partials (pinned host)
   unsigned npart;
@@ -169,68 +168,50 @@ hm_status check_state(const hm_solver *s, const void *p, const char *name) {
 // "rk 44" tableau (TimeExplicitRKInitialize.c:58-68)
 const double RK_A_SUB[3] = {0.5, 0.5, 1.0};  // A[s+1][s]
 const double RK_B[4] = {1.0 / 6.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0};
-// "rk ssprk3" tableau (TimeExplicitRKInitialize.c:69-79): A[1][0] = 1,
-// A[2][0] = A[2][1] = 1/4, b = 1/6, 1/6, 2/3
-const double SSP_A10 = 1.0, SSP_A20 = 0.25, SSP_A21 = 0.25;
-const double SSP_B[3] = {1.0 / 6.0, 1.0 / 6.0, 2.0 / 3.0};
-
-hm::PassBuffers stage_buffers(hm_solver *s, double *u, const double *U, double *Sn) {
-  hm::PassBuffers b;
-  b.U = U;
-  b.R = s->R;
-  b.par = s->par;
-  b.u = u;
-  b.S = Sn;
-  b.acc = s->acc;
-  b.out = nullptr;
-  b.Q = s->Q;
-  return b;
+// The update of RK4 stage `stage` on state u with stage states Sx (c in units
+// of dt when dt is 1): see StageUpdate
+hm::StageUpdate rk4_update(int stage, double *u, double dt, double *const Sx[3]) {
+  hm::StageUpdate q;
+  q.kind = stage == 0 ? hm::UPD_SELF : (stage < 3 ? hm::UPD_MIX : hm::UPD_RK4);
+  q.c = dt * (stage < 3 ? RK_A_SUB[stage] : RK_B[3]);
+  q.k = 0.0;
+  q.a0 = u;
+  q.a1 = Sx[1];
+  q.a2 = Sx[0];
+  q.out = stage < 3 ? Sx[stage] : u;
+  return q;
 }
 
-// One RK4 step of u in place through the fused direction passes.  Stage s
-// reads Sx[s-1] (u for s = 0) and writes Sx[s]; the last stage writes u.
-// Viscous runs need the primitive variables of u in Q on entry and leave
-// those of the new u there.
+// the launches of one stage on state U: the viscous term (viscous runs need
+// the primitive variables of U in Q and leave those of the new state there),
+// then the three passes with the update upd
+hm_status stage_launches(hm_solver *s, const double *U, const hm::StageUpdate &upd) {
+  if (s->sc.Re > 0) hm::launch_visc_par(s->g, s->sc, s->Q, s->par, s->dxg, s->stream);
+  const hm::PassBuffers b = {U, s->R, s->par, s->Q, upd};
+  for (int d = 0; d < 3; d++) hm::launch_pass(s->g, s->sc, d, b, hm::OUT_STAGE, s->dxg, s->stream);
+  return check_launch("Runge-Kutta stage passes");
+}
+
+// One RK4 step of u in place through the fused direction passes (TimeRK.c:126-195
+// with the "44" tableau).  Stage s reads Sx[s-1] (u for s = 0) and writes
+// Sx[s]; the last stage writes u from u and all three.
 hm_status rk4_step(hm_solver *s, double *u, double dt, double *const Sx[3]) {
-  const bool visc = s->sc.Re > 0;
   for (int stage = 0; stage < 4; stage++) {
-    const hm::PassBuffers b = stage_buffers(s, u, stage == 0 ? u : Sx[stage - 1], stage < 3 ? Sx[stage] : nullptr);
-    if (visc) hm::launch_visc_par(s->g, s->sc, s->Q, s->par, s->dxg, s->stream);
-    const double ca = stage < 3 ? dt * RK_A_SUB[stage] : 0.0, cb = dt * RK_B[stage];
-    for (int d = 0; d < 3; d++) hm::launch_pass(s->g, s->sc, d, b, hm::OUT_STAGE, stage, ca, cb, s->dxg, s->stream);
-    hm_status st = check_launch("RK4 stage passes");
+    hm_status st = stage_launches(s, stage == 0 ? u : Sx[stage - 1], rk4_update(stage, u, dt, Sx));
     if (st != HM_OK) return st;
   }
   return HM_OK;
 }
 
-// One SSPRK3 step of u in place (TimeRK.c:126-195 with the "ssprk3"
-// tableau):  U1 = u + dt k0,  U2 = (u + dt/4 k0) + dt/4 k1,
-// u_new = ((u + dt/6 k0) + dt/6 k1) + 2dt/3 k2, in the reference's order.
-// With the z pass's three-output update (O1 = a + c1 r, O2 = b + c2 r,
-// O3 = a + c3 r):
-//   stage 0 (from u):    acc = u + dt/6 k0, S0 = u + dt k0, S1 = u + dt/4 k0
-//   stage 1 (from S0):   acc = acc + dt/6 k1, S1 = S1 + dt/4 k1 (in place), acc again
-//   stage 2 (from S1):   u = acc + 2dt/3 k2 (all three outputs)
+// One SSPRK3 step of u in place (TimeRK.c:126-195 with the "ssprk3" tableau,
+// written through its stage states: see StageUpdate)
 hm_status ssprk3_step(hm_solver *s, double *u, double dt) {
-  const bool visc = s->sc.Re > 0;
-  double *acc = s->acc, *S0 = s->S[0], *S1 = s->S[1];
-  const double *Uin[3] = {u, S0, S1};
-  const double *A[3] = {u, acc, acc}, *B[3] = {u, S1, acc};
-  double *O1[3] = {acc, acc, u}, *O2[3] = {S0, S1, u}, *O3[3] = {S1, acc, u};
-  const double c1[3] = {dt * SSP_B[0], dt * SSP_B[1], dt * SSP_B[2]};
-  const double c2[3] = {dt * SSP_A10, dt * SSP_A21, dt * SSP_B[2]};
-  const double c3[3] = {dt * SSP_A20, dt * SSP_B[1], dt * SSP_B[2]};
-  // distinct outputs per stage: stage 1 stores acc twice (O3 = O1), stage 2
-  // stores u three times (O1 = O2 = O3, with B = A)
-  const int nout[3] = {3, 2, 1};
+  const double c[3] = {dt, 0.25 * dt, (2.0 / 3.0) * dt}, k[3] = {0.0, 0.25, 2.0 / 3.0};
+  const double *U[3] = {u, s->S[0], s->S[1]};
+  double *out[3] = {s->S[0], s->S[1], u};
   for (int stage = 0; stage < 3; stage++) {
-    const hm::PassBuffers b = stage_buffers(s, u, Uin[stage], nullptr);
-    if (visc) hm::launch_visc_par(s->g, s->sc, s->Q, s->par, s->dxg, s->stream);
-    for (int d = 0; d < 2; d++) hm::launch_pass(s->g, s->sc, d, b, hm::OUT_STAGE, stage, 0.0, 0.0, s->dxg, s->stream);
-    hm::launch_pass_z_affine(s->g, s->sc, b, A[stage], B[stage], O1[stage], O2[stage], O3[stage], c1[stage],
-                             c2[stage], c3[stage], nout[stage], s->dxg, s->stream);
-    hm_status st = check_launch("SSPRK3 stage passes");
+    hm_status st = stage_launches(
+        s, U[stage], {stage == 0 ? hm::UPD_SELF : hm::UPD_MIX, c[stage], k[stage], u, nullptr, nullptr, out[stage]});
     if (st != HM_OK) return st;
   }
   return HM_OK;
@@ -258,7 +239,7 @@ const char *hm_version(void) { return "hypar-mi355x 0.1 (gfx950, fp64)"; }
 void hm_destroy(hm_solver *s) {
   if (!s) return;
   hm::drop_bindings(s);
-  double *bufs[] = {s->dxg, s->R, s->par, s->Q, s->S[0], s->S[1], s->acc, s->part, s->tmp};
+  double *bufs[] = {s->dxg, s->R, s->par, s->Q, s->S[0], s->S[1], s->S[2], s->part, s->tmp};
   for (double *b : bufs)
     if (b) (void)hipFree(b);
   if (s->part_host) (void)hipHostFree(s->part_host);
@@ -330,7 +311,7 @@ hm_status hm_create(const hm_config *cfg, hm_solver **out) {
   }
   if ((st = dmalloc(&s->S[0], n5)) != HM_OK) goto bad;
   if ((st = dmalloc(&s->S[1], n5)) != HM_OK) goto bad;
-  if ((st = dmalloc(&s->acc, n5)) != HM_OK) goto bad;
+  if ((st = dmalloc(&s->S[2], n5)) != HM_OK) goto bad;
   s->npart = hm::reduction_blocks(n5);
   if ((st = dmalloc(&s->part, s->npart)) != HM_OK) goto bad;
   if (hipHostMalloc((void **)&s->part_host, s->npart * sizeof(double), hipHostMallocDefault) != hipSuccess) {
@@ -407,9 +388,8 @@ hm_status hm_rk4(hm_solver *s, double *u, double dt, int nsteps) {
   if (!std::isfinite(dt)) return fail(HM_ERR_ARG, "hm_rk4: dt is not finite");
   if (nsteps == 0) return HM_OK;
   if (s->sc.Re > 0) hm::launch_prims(s->g, s->sc, u, s->Q, s->stream);
-  double *const Sx[3] = {s->S[0], s->S[1], s->S[0]};
   for (int it = 0; it < nsteps; it++)
-    if ((st = rk4_step(s, u, dt, Sx)) != HM_OK) return st;
+    if ((st = rk4_step(s, u, dt, s->S)) != HM_OK) return st;
   return HM_OK;
 }
 
@@ -435,13 +415,8 @@ static hm_status rhs_passes(hm_solver *s, double *out, const double *u, int mode
     hm::launch_prims(s->g, s->sc, u, s->Q, s->stream);
     hm::launch_visc_par(s->g, s->sc, s->Q, s->par, s->dxg, s->stream);
   }
-  hm::PassBuffers b;
-  b.U = u;
-  b.R = s->R;
-  b.par = s->par;
-  b.u = b.S = b.acc = b.Q = nullptr;
-  b.out = out;
-  for (int d = 0; d < 3; d++) hm::launch_pass(s->g, s->sc, d, b, mode, 0, 0.0, 0.0, s->dxg, s->stream);
+  const hm::PassBuffers b = {u, s->R, s->par, nullptr, {hm::UPD_SELF, 0.0, 0.0, nullptr, nullptr, nullptr, out}};
+  for (int d = 0; d < 3; d++) hm::launch_pass(s->g, s->sc, d, b, mode, s->dxg, s->stream);
   return check_launch(name);
 }
 
@@ -973,20 +948,11 @@ hm_status hm_profile_kernels(hm_solver *s, const double *u, int reps, double *ms
     hm::launch_prims(s->g, s->sc, u, s->Q, s->stream);
     hm::launch_visc_par(s->g, s->sc, s->Q, s->par, s->dxg, s->stream);
   }
-  // the passes as stage 1 of an RK step runs them: the z pass reads u and
-  // acc and writes acc, the next stage state (and Q); u is not written
-  HM_HIP(hipMemsetAsync(s->acc, 0, 5 * s->g.ncell * sizeof(double), s->stream));
-  hm::PassBuffers b;
-  b.U = u;
-  b.R = s->R;
-  b.par = s->par;
-  b.u = const_cast<double *>(u);
-  b.S = s->S[1];
-  b.acc = s->acc;
-  b.out = nullptr;
-  b.Q = s->Q;  // primitive variables of the stage state (solver scratch)
+  // the passes as stage 1 of an RK4 step runs them: the z pass reads u and
+  // writes the next stage state (and Q); u is not written
+  const hm::PassBuffers b = {u, s->R, s->par, s->Q, {hm::UPD_MIX, 0.0, 0.0, u, nullptr, nullptr, s->S[1]}};
   for (int d = 0; d < 3 && st == HM_OK; d++)
-    st = timed(d, [&] { hm::launch_pass(s->g, s->sc, d, b, hm::OUT_STAGE, 1, 0.0, 0.0, s->dxg, s->stream); });
+    st = timed(d, [&] { hm::launch_pass(s->g, s->sc, d, b, hm::OUT_STAGE, s->dxg, s->stream); });
   if (st == HM_OK) {
     if (visc) {
       st = timed(3, [&] { hm::launch_visc_par(s->g, s->sc, s->Q, s->par, s->dxg, s->stream); });
@@ -1016,7 +982,7 @@ struct hm_ensemble {
   hm::EnsMember *mem_dev = nullptr;
   double *dxg = nullptr;
   size_t ncell = 0;
-  double *R = nullptr, *S[2] = {nullptr, nullptr}, *acc = nullptr;
+  double *R = nullptr, *S[3] = {nullptr, nullptr, nullptr};
   // viscous members: viscous terms and primitive variables of all members,
   // each member's first tile of the viscous-term launch, and (adjoint) of
   // the viscous VJP launches
@@ -1070,30 +1036,30 @@ void ens_drop_graph(hm_ensemble *e) {
   e->graph_u = nullptr;
 }
 
-// the launches of RK stage `stage` of all members on stage state U: the
-// viscous terms of U (viscous members; the previous stage's z pass left its
+// the launches of RK4 stage `stage` of all members on its state U (u or
+// Sx[stage - 1]): the viscous terms of U (viscous members; the previous stage's z pass left its
 // primitive variables in Q), then the three direction passes, as three
 // launches (shapes 0, 1) or one (shapes 2, 3)
-void ens_stage_launches(hm_ensemble *e, int stage, const double *U, double *u, double *Sn, hipStream_t st) {
+void ens_stage_launches(hm_ensemble *e, int stage, double *u, double *const Sx[3], hipStream_t st) {
+  const double *U = stage == 0 ? u : Sx[stage - 1];
+  const hm::StageUpdate upd = rk4_update(stage, u, 1.0, Sx);  // the kernels multiply by the members' dt
   if (e->sc.Re > 0) hm::launch_ens_visc(e->sc, e->mem_dev, e->nmem, e->ptiles0, e->nptiles, e->pks, st);
   const int ts = e->shape & 1;  // 0: 4 wavefronts per block, 1: 2
   if (e->shape >= 2) {
     const unsigned *const item0[3] = {e->xitem0[ts], e->item0[ts][1], e->item0[ts][2]};
     const unsigned nitems[3] = {e->nxitems[ts], e->nitems[ts][1], e->nitems[ts][2]};
     hm::launch_ens_stage(e->sc, ts == 0 ? 4 : 2, e->mem_dev, e->nmem, item0, nitems, e->item0[ts][0], hm::ENS_STAGE_XG,
-                         e->grid[0], e->cus, e->ctr, e->spin_limit, U, e->R, u, Sn, e->acc, stage, st);
+                         e->grid[0], e->cus, e->ctr, e->spin_limit, U, e->R, upd, st);
     return;
   }
   for (int d = 0; d < 3; d++)
-    hm::launch_ens_pass(e->sc, d, ts, e->mem_dev, e->nmem, e->item0[ts][d], e->nitems[ts][d], e->grid[d], U, e->R, u,
-                        Sn, e->acc, stage, st);
+    hm::launch_ens_pass(e->sc, d, ts, e->mem_dev, e->nmem, e->item0[ts][d], e->nitems[ts][d], e->grid[d], U, e->R,
+                        upd, st);
 }
 
-// the launches of one RK4 step of all members (stage s reads S[(s-1)%2],
-// writes S[s%2]; the last stage writes u)
+// the launches of one RK4 step of all members
 void ens_step_launches(hm_ensemble *e, double *u, hipStream_t st) {
-  for (int stage = 0; stage < 4; stage++)
-    ens_stage_launches(e, stage, stage == 0 ? u : e->S[(stage - 1) % 2], u, stage < 3 ? e->S[stage % 2] : nullptr, st);
+  for (int stage = 0; stage < 4; stage++) ens_stage_launches(e, stage, u, e->S, st);
 }
 
 // After launches of the one-launch-per-stage shapes: wait for the stream and
@@ -1129,8 +1095,7 @@ hm_status ens_capture(hm_ensemble *e, double *u) {
 hm_status ens_step_store(hm_ensemble *e, double *u, double *const U[3]) {
   hipStream_t st = e->stream;
   if (e->sc.Re > 0) hm::launch_ens_prims(e->sc, e->mem_dev, e->nmem, u, e->ncell, st);
-  for (int stage = 0; stage < 4; stage++)
-    ens_stage_launches(e, stage, stage == 0 ? u : U[stage - 1], u, stage < 3 ? U[stage] : nullptr, st);
+  for (int stage = 0; stage < 4; stage++) ens_stage_launches(e, stage, u, U, st);
   return check_launch("hm_ensemble: step");
 }
 
@@ -1149,7 +1114,7 @@ void hm_ensemble_destroy(hm_ensemble *e) {
   if (!e) return;
   ens_drop_graph(e);
   if (e->cap) (void)hipStreamDestroy(e->cap);
-  double *bufs[] = {e->dxg, e->R, e->S[0], e->S[1], e->acc, e->par, e->Q};
+  double *bufs[] = {e->dxg, e->R, e->S[0], e->S[1], e->S[2], e->par, e->Q};
   for (double *b : bufs)
     if (b) (void)hipFree(b);
   if (e->ctr) (void)hipFree(e->ctr);
@@ -1248,7 +1213,7 @@ hm_status hm_ensemble_create(const hm_config *members, int nmembers, hm_ensemble
   if ((st = dmalloc(&e->R, n5)) != HM_OK) goto bad;
   if ((st = dmalloc(&e->S[0], n5)) != HM_OK) goto bad;
   if ((st = dmalloc(&e->S[1], n5)) != HM_OK) goto bad;
-  if ((st = dmalloc(&e->acc, n5)) != HM_OK) goto bad;
+  if ((st = dmalloc(&e->S[2], n5)) != HM_OK) goto bad;
   if (hipMemcpy(e->dxg, dxh.data(), dxh.size() * sizeof(double), hipMemcpyHostToDevice) != hipSuccess) {
     st = fail(HM_ERR_HIP, "hm_ensemble_create: copy of dxinv failed");
     goto bad;

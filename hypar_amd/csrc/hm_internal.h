@@ -89,30 +89,38 @@ void launch_fluxdiff(const Grid &g, int dir, double *hyp, const double *fI, cons
 void launch_axpy(const double *x, double a, double *y, size_t n, hipStream_t st);
 void launch_fill(double *x, double value, size_t n, hipStream_t st);
 
+// Update of a Runge-Kutta stage by the z pass.  With r the stage's right-hand
+// side and U its state,
+//   UPD_SELF  out = U + c r                                  (the first stage)
+//   UPD_MIX   out = a0 + (k (U - a0) + c r)
+//   UPD_RK4   out = a1 + (((a2 - a1) + (U - a0))/3 + c r)
+// RK4 with the stage states U2 = u + dt/2 k1, U3 = u + dt/2 k2, U4 = u + dt k3
+// ends in u + dt (k1 + 2 k2 + 2 k3 + k4)/6 = U3 + ((U2 - U3) + (U4 - u))/3 +
+// dt/6 k4, and SSPRK3 (its tableau of TimeExplicitRKInitialize.c:69-79) is
+// U2 = u + dt k1, U3 = u + ((U2 - u) + dt k2)/4, u + 2/3 ((U3 - u) + dt k3).
+// The updates so need no accumulator: a stage reads at most u, the last RK4
+// stage u, U2 and U3, and writes one state.
+enum { UPD_SELF = 0, UPD_MIX = 1, UPD_RK4 = 2 };
+struct StageUpdate {
+  int kind;
+  double c, k;                  // c in units of dt for an ensemble, whose members have their own
+  const double *a0, *a1, *a2;   // operands the kind reads
+  double *out;
+};
+
 // fused direction passes (hm_pass.hip)
 struct PassBuffers {
   const double *U;        // stage state
   double *R;              // hyperbolic-term accumulator, 5*ncell
   const double *par;      // viscous term, 4*ncell (viscous runs; read by the z pass)
-  double *u, *S, *acc;    // RK4 state, next stage state, accumulator (z pass, OUT_STAGE)
-  double *out;            // right-hand side or hyperbolic term (z pass, OUT_RHS / OUT_HYP)
   double *Q;              // u, v, w, T of the new state (z pass, viscous OUT_STAGE)
+  StageUpdate upd;        // z pass: the stage's update (OUT_STAGE); out also takes OUT_RHS and OUT_HYP
 };
 // pass along dir: x stores its flux differences in R, y adds its own, z adds
 // its own and forms rhs = -hyp + par, then finishes the stage (mode
-// OUT_STAGE with stage, ca = dt*A[s+1][s], cb = dt*b[s]) or writes rhs
-// (OUT_RHS) or hyp (OUT_HYP)
-void launch_pass(const Grid &g, const Scheme &sc, int dir, const PassBuffers &b, int mode, int stage, double ca,
-                 double cb, const double *dxg, hipStream_t st);
-// the z pass with a three-output stage update: with r the right-hand side
-// and a, b the operands A, B at each cell, O1 = a + c1 r, O2 = b + c2 r (the
-// next stage state; its primitive variables go to b.Q when viscous),
-// O3 = a + c3 r.  The first nout (1-3) outputs are stored; an output left
-// out must repeat O1 (same array and value).  O2 may be B.  The x and y
-// passes of the stage are launch_pass's.
-void launch_pass_z_affine(const Grid &g, const Scheme &sc, const PassBuffers &b, const double *A, const double *B,
-                          double *O1, double *O2, double *O3, double c1, double c2, double c3, int nout,
-                          const double *dxg, hipStream_t st);
+// OUT_STAGE) or writes rhs (OUT_RHS) or hyp (OUT_HYP)
+void launch_pass(const Grid &g, const Scheme &sc, int dir, const PassBuffers &b, int mode, const double *dxg,
+                 hipStream_t st);
 // primitive variables (u, v, w, T) of u into Q
 void launch_prims(const Grid &g, const Scheme &sc, const double *u, double *Q, hipStream_t st);
 
@@ -155,12 +163,12 @@ unsigned ens_items_per_member(int dir, int shape, const int n[3], const int seg[
 // cells per march segment of the pass along dir (1 or 2) of `count` grids that
 // run together, into seg[count]
 void march_segments(int count, const int (*n)[3], int dir, int *seg);
-// one pass of RK stage `stage` over all members; grid = number of
-// persistent blocks (0: one block per work item)
+// one pass of an RK stage over all members; grid = number of persistent
+// blocks (0: one block per work item)
 void launch_ens_pass(const Scheme &sc, int dir, int shape, const EnsMember *mem, int nmem, const unsigned *item0,
-                     unsigned nitems, unsigned grid, const double *U, double *R, double *u, double *S, double *acc,
-                     int stage, hipStream_t st);
-// all three passes of RK stage `stage` over all members in one persistent
+                     unsigned nitems, unsigned grid, const double *U, double *R, const StageUpdate &upd,
+                     hipStream_t st);
+// all three passes of an RK stage over all members in one persistent
 // launch (rows = 4 or 2 wavefronts per block, the tile shapes of the split
 // passes; grid 0 = the blocks the GPU holds at once, cus CUs).  An x item
 // is ENS_STAGE_XG groups of x-lines: item0[0] lists each member's first x
@@ -173,8 +181,8 @@ void launch_ens_pass(const Scheme &sc, int dir, int shape, const EnsMember *mem,
 constexpr unsigned ENS_STAGE_XG = HM_ENS_XG;
 void launch_ens_stage(const Scheme &sc, int rows, const EnsMember *mem, int nmem, const unsigned *const item0[3],
                       const unsigned nitems[3], const unsigned *xgroups0, unsigned xg, unsigned grid, int cus,
-                      unsigned *ctr, unsigned spin_limit, const double *U, double *R, double *u, double *S,
-                      double *acc, int stage, hipStream_t st);
+                      unsigned *ctr, unsigned spin_limit, const double *U, double *R, const StageUpdate &upd,
+                      hipStream_t st);
 
 // viscous terms of all members (hm_kernels.hip): one launch over the
 // (member, par_tiles) items of pks planes, ptiles0 = each member's first item

@@ -89,27 +89,9 @@ struct PassIO {
   const double *U;    // stage state
   double *R;          // hyperbolic-term accumulator
   const double *par;  // viscous term, par[c*ncell + cell], c = momentum x, y, z, energy
-  double *u, *S, *acc, *out, *Q;
-  int visc, mode, stage;
-  double ca, cb;
-};
-
-// Stage update of the z pass in the separate kernel instantiations RK =
-// RK_AFFINE: with r the stage's right-hand side and a, b the operands A, B
-// at the cell,
-//   O1 = a + c1 r,  O2 = b + c2 r (the next stage state),  O3 = a + c3 r;
-// the caller picks operands, outputs and coefficients per stage.  The first
-// nout outputs are stored; the caller leaves out only an output that
-// repeats O1 (same array, same value), and every pointer is valid whether
-// stored or not.  The update has no per-stage branches that choose among
-// outputs: the compiler merged the stores of a three-way stage branch into
-// one store whose address register one path never set.
-enum { RK_CLASSIC = 0, RK_AFFINE = 1 };
-struct SspIO {
-  const double *A, *B;
-  double *O1, *O2, *O3;
-  double c1, c2, c3;
-  int nout;  // outputs stored: O1, then O2 (nout >= 2), then O3 (nout = 3)
+  double *Q;
+  StageUpdate upd;
+  int visc, mode;
 };
 
 // per-cell record of the pass direction (NavierStokes3DFlux.c:23-57)
@@ -407,58 +389,51 @@ __device__ __forceinline__ void store_r(double *p, double v) {
 }
 
 // Inputs of cell idx's output that come from global memory: its dxinv, the
-// hyperbolic term so far (y, z), the viscous term and the RK4 operands (z).
+// hyperbolic term so far (y, z), the viscous term and the update's operands (z).
 // The marching passes issue these loads in one block with the next ring
 // row's, so that their latencies overlap.
 struct EmitIn {
-  double dxi, par[NV], rin[NV], a[NV], b[NV];
+  double dxi, par[NV], rin[NV], a[NV], b[NV], c[NV];
 };
 
-template <int DIR, int RK = RK_CLASSIC, bool COH = false>
-__device__ __forceinline__ EmitIn emit_load(const PassConst &k, const PassIO &io, size_t idx, int pos,
-                                            const SspIO &sp = SspIO{}) {
+template <int DIR, bool COH = false>
+__device__ __forceinline__ EmitIn emit_load(const PassConst &k, const PassIO &io, size_t idx, int pos) {
   EmitIn in;
   in.dxi = k.dxg[(DIR >= 1 ? k.n[0] + 6 : 0) + (DIR == 2 ? k.n[1] + 6 : 0) + 3 + pos];
 #pragma unroll
-  for (int v = 0; v < NV; v++) in.par[v] = in.rin[v] = in.a[v] = in.b[v] = 0.0;
+  for (int v = 0; v < NV; v++) in.par[v] = in.rin[v] = in.a[v] = in.b[v] = in.c[v] = 0.0;
   if (DIR > 0)
 #pragma unroll
     for (int v = 0; v < NV; v++) in.rin[v] = load_r<COH>(io.R + (size_t)v * k.ncell + idx);
   if (DIR == 2 && io.visc && io.mode != OUT_HYP)
 #pragma unroll
     for (int c = 0; c < 4; c++) in.par[c + 1] = io.par[(size_t)c * k.ncell + idx];
-  // the RK4 operands of the 3N update (u at stage 0, acc and u at stages
-  // 1-2, acc at stage 3), one uniform branch per stage kind, each with its
+  // the operands of the update, one uniform branch per kind, each with its
   // loads in one block
-  if (RK == RK_AFFINE && DIR == 2) {
+  if (DIR == 2 && io.mode == OUT_STAGE) {
+    if (io.upd.kind == UPD_MIX) {
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      in.a[v] = sp.A[(size_t)v * k.ncell + idx];
-      in.b[v] = sp.B[(size_t)v * k.ncell + idx];
-    }
-  } else if (DIR == 2 && io.mode == OUT_STAGE) {
-    if (io.stage == 0) {
-#pragma unroll
-      for (int v = 0; v < NV; v++) in.a[v] = io.u[(size_t)v * k.ncell + idx];
-    } else if (io.stage == 3) {
-#pragma unroll
-      for (int v = 0; v < NV; v++) in.a[v] = io.acc[(size_t)v * k.ncell + idx];
-    } else {
+      for (int v = 0; v < NV; v++) in.a[v] = io.upd.a0[(size_t)v * k.ncell + idx];
+    } else if (io.upd.kind == UPD_RK4) {
 #pragma unroll
       for (int v = 0; v < NV; v++) {
-        in.a[v] = io.acc[(size_t)v * k.ncell + idx];
-        in.b[v] = io.u[(size_t)v * k.ncell + idx];
+        in.a[v] = io.upd.a0[(size_t)v * k.ncell + idx];
+        in.b[v] = io.upd.a1[(size_t)v * k.ncell + idx];
+        in.c[v] = io.upd.a2[(size_t)v * k.ncell + idx];
       }
     }
   }
   return in;
 }
 
-// Finish cell idx of the pass: flux difference and the pass's output.
-template <int DIR, int RK = RK_CLASSIC, bool COH = false>
+// Finish cell idx of the pass: flux difference and the pass's output.  uc is
+// the cell's stage state (z pass).  Every mode and kind of update stores one
+// array through one pointer: the compiler merged the stores of branches that
+// chose among outputs into one store whose address register one path never
+// set.
+template <int DIR, bool COH = false>
 __device__ __forceinline__ void emit_store(const PassConst &k, const PassIO &io, size_t idx, const EmitIn &in,
-                                           const double (&fm)[NV], const double (&fp)[NV],
-                                           const SspIO &sp = SspIO{}) {
+                                           const double (&fm)[NV], const double (&fp)[NV], const double (&uc)[NV]) {
   double r[NV];
 #pragma unroll
   for (int v = 0; v < NV; v++) {
@@ -473,55 +448,36 @@ __device__ __forceinline__ void emit_store(const PassConst &k, const PassIO &io,
     for (int v = 0; v < NV; v++) store_r<COH>(io.R + (size_t)v * k.ncell + idx, r[v]);
     return;
   }
-  if (io.mode != OUT_STAGE) {
+  if (io.mode == OUT_STAGE) {
+    const double c = io.upd.c;
+    if (io.upd.kind == UPD_SELF) {
 #pragma unroll
-    for (int v = 0; v < NV; v++) io.out[(size_t)v * k.ncell + idx] = r[v];
-    return;
-  }
-  double nu[NV];
-  if (RK == RK_AFFINE) {
+      for (int v = 0; v < NV; v++) r[v] = uc[v] + c * r[v];
+    } else if (io.upd.kind == UPD_MIX) {
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-      const size_t o = (size_t)v * k.ncell + idx;
-      nu[v] = in.b[v] + sp.c2 * r[v];
-      sp.O1[o] = in.a[v] + sp.c1 * r[v];
-      if (sp.nout > 1) sp.O2[o] = nu[v];
-      if (sp.nout > 2) sp.O3[o] = in.a[v] + sp.c3 * r[v];
-    }
-  } else {
-  // RK4 stage update in 3N form (TimeRK.c:126-195)
-#pragma unroll
-  for (int v = 0; v < NV; v++) {
-    const size_t o = (size_t)v * k.ncell + idx;
-    if (io.stage == 0) {
-      io.acc[o] = in.a[v] + io.cb * r[v];
-      nu[v] = in.a[v] + io.ca * r[v];
-      io.S[o] = nu[v];
-    } else if (io.stage < 3) {
-      io.acc[o] = in.a[v] + io.cb * r[v];
-      nu[v] = in.b[v] + io.ca * r[v];
-      io.S[o] = nu[v];
+      for (int v = 0; v < NV; v++) r[v] = in.a[v] + (io.upd.k * (uc[v] - in.a[v]) + c * r[v]);
     } else {
-      nu[v] = in.a[v] + io.cb * r[v];
-      io.u[o] = nu[v];
+#pragma unroll
+      for (int v = 0; v < NV; v++)
+        r[v] = in.b[v] + (((in.c[v] - in.b[v]) + (uc[v] - in.a[v])) * (1.0 / 3.0) + c * r[v]);
     }
   }
-  }
-  if (io.visc) {
+#pragma unroll
+  for (int v = 0; v < NV; v++) io.upd.out[(size_t)v * k.ncell + idx] = r[v];
+  if (io.visc && io.mode == OUT_STAGE) {
     // primitive variables (u, v, w, T) of the new state for the next
     // viscous-term evaluation (NavierStokes3DParabolicFunction.c:85-108)
     double q[4];
-    visc_prims(nu, k.gamma, q);
+    visc_prims(r, k.gamma, q);
 #pragma unroll
     for (int c = 0; c < 4; c++) io.Q[(size_t)c * k.ncell + idx] = q[c];
   }
 }
 
-template <int DIR, int RK = RK_CLASSIC, bool COH = false>
+template <int DIR, bool COH = false>
 __device__ __forceinline__ void emit(const PassConst &k, const PassIO &io, size_t idx, int pos,
-                                     const double (&fm)[NV], const double (&fp)[NV],
-                                     const SspIO &sp = SspIO{}) {
-  emit_store<DIR, RK, COH>(k, io, idx, emit_load<DIR, RK, COH>(k, io, idx, pos, sp), fm, fp, sp);
+                                     const double (&fm)[NV], const double (&fp)[NV], const double (&uc)[NV]) {
+  emit_store<DIR, COH>(k, io, idx, emit_load<DIR, COH>(k, io, idx, pos), fm, fp, uc);
 }
 
 // ---------------------------------------------------------------------------
@@ -585,7 +541,7 @@ __device__ __forceinline__ void pass_x_body(const PassConst &k, const PassIO &io
         fm[v] = sh.sF[w][v][lane];
         fp[v] = sh.sF[w][v][lane + 1];
       }
-      emit<0, RK_CLASSIC, COH>(k, io, base + cell, cell, fm, fp);
+      emit<0, COH>(k, io, base + cell, cell, fm, fp, fm);
     }
     __syncthreads();
   }
@@ -598,7 +554,7 @@ __device__ __forceinline__ void pass_x_body(const PassConst &k, const PassIO &io
       fm[v] = sh.sF[w][v][nx - x0];
       fp[v] = sh.sF0[w][v];
     }
-    emit<0, RK_CLASSIC, COH>(k, io, base + nx - 1, nx - 1, fm, fp);
+    emit<0, COH>(k, io, base + nx - 1, nx - 1, fm, fp, fm);
   }
 }
 
@@ -621,9 +577,9 @@ struct MShared {
 // segment that is a whole line keeps the flux of interface 0 for its last
 // cell; any other evaluates interfaces c0 .. c1, one more than its cells,
 // and starts on six rows of its neighbour.
-template <int DIR, int INTERP, int UPW, int MR, int W, int RK = RK_CLASSIC, bool COH = false>
+template <int DIR, int INTERP, int UPW, int MR, int W, bool COH = false>
 __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io, size_t item,
-                                            MShared<MR, UPW> &sh, const SspIO &sp = SspIO{}) {
+                                            MShared<MR, UPW> &sh) {
   constexpr int NRING = MShared<MR, UPW>::NRING, NFR = MShared<MR, UPW>::NFR;
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -676,6 +632,7 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
   for (int t0 = c0; t0 < tend; t0 += MR) {
     __syncthreads();
     const int t = t0 + w;
+    double uc[NV] = {0, 0, 0, 0, 0};  // stage state of cell t-1, which this wavefront emits
     if (t < tend) {
       const int sl0 = (t - 3 + NRING) % NRING;
       auto ld = [&](int s, int q) {
@@ -685,6 +642,9 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
       };
       double f[NV];
       iface<DIR, INTERP, UPW, W>(ld, k, f);
+      if (DIR == 2)
+#pragma unroll
+        for (int v = 0; v < NV; v++) uc[v] = ld(2, v);
       const int fs = t % NFR;
 #pragma unroll
       for (int v = 0; v < NV; v++) sh.sF[v][fs][lane] = f[v];
@@ -704,7 +664,7 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
     double un[NV];
     fetch_row(rn, un);
     const int ec = e < 0 ? 0 : (e > elast ? elast : e);
-    const EmitIn in = emit_load<DIR, RK, COH>(k, io, cbase + (size_t)ec * stride, ec, sp);
+    const EmitIn in = emit_load<DIR, COH>(k, io, cbase + (size_t)ec * stride, ec);
     if (more) stage_row(rn, un);
     if (emits) {
       double fm[NV], fp[NV];
@@ -714,19 +674,20 @@ __device__ __forceinline__ void pass_m_body(const PassConst &k, const PassIO &io
         fm[v] = sh.sF[v][a][lane];
         fp[v] = sh.sF[v][b][lane];
       }
-      emit_store<DIR, RK, COH>(k, io, cbase + (size_t)e * stride, in, fm, fp, sp);
+      emit_store<DIR, COH>(k, io, cbase + (size_t)e * stride, in, fm, fp, uc);
     }
   }
   // last row of a whole line: fI[n-1] and fI[n] = fI[0]
   if (whole && w == 0 && col) {
-    double fm[NV], fp[NV];
+    double fm[NV], fp[NV], uc[NV];
     const int a = (n - 1) % NFR;
 #pragma unroll
     for (int v = 0; v < NV; v++) {
       fm[v] = sh.sF[v][a][lane];
       fp[v] = sh.sF0[v][lane];
+      uc[v] = sh.sC[v][(n - 1) % NRING][lane];
     }
-    emit<DIR, RK, COH>(k, io, cbase + (size_t)(n - 1) * stride, n - 1, fm, fp, sp);
+    emit<DIR, COH>(k, io, cbase + (size_t)(n - 1) * stride, n - 1, fm, fp, uc);
   }
 }
 
@@ -749,14 +710,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k
   pass_m_body<DIR, INTERP, UPW, 4, W>(k, io, blockIdx.x, sh);
 }
 
-// the z pass with the three-output stage update (SSPRK3 stages)
-template <int INTERP, int UPW, int W>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_pass_z_affine(PassConst k, PassIO io,
-                                                                                             SspIO sp) {
-  __shared__ MShared<4, UPW> sh;
-  pass_m_body<2, INTERP, UPW, 4, W, RK_AFFINE>(k, io, blockIdx.x, sh, sp);
-}
-
 // ---------------------------------------------------------------------------
 // batched passes: all members of an ensemble in one persistent launch
 // ---------------------------------------------------------------------------
@@ -767,8 +720,9 @@ struct EnsArgs {
   unsigned nitems;
   double gamma, gm1, inv_gm1, eps34;  // eps34 = 3/4 of the WENO epsilon
   const double *U;         // stage states of all members (member m at 5*off)
-  double *R, *u, *S, *acc;
-  int mode, stage, visc;
+  double *R;
+  StageUpdate upd;
+  int visc;
 };
 
 // the member of a work item and the item's index within the member
@@ -796,17 +750,15 @@ __device__ __forceinline__ void ens_setup(const EnsArgs &a, int m, int dir, Pass
   io.U = a.U + o;
   io.R = a.R + o;
   io.par = M.par;
-  io.u = a.u + o;
-  io.S = a.S ? a.S + o : nullptr;
-  io.acc = a.acc + o;
-  io.out = nullptr;
   io.Q = M.q;
+  io.upd = a.upd;
+  io.upd.c = M.dt * a.upd.c;
+  io.upd.a0 = a.upd.a0 + o;
+  io.upd.a1 = a.upd.a1 + o;
+  io.upd.a2 = a.upd.a2 + o;
+  io.upd.out = a.upd.out + o;
   io.visc = a.visc;
-  io.mode = a.mode;
-  io.stage = a.stage;
-  const double A_sub[3] = {0.5, 0.5, 1.0}, b[4] = {1.0 / 6.0, 1.0 / 3.0, 1.0 / 3.0, 1.0 / 6.0};
-  io.ca = a.stage < 3 ? M.dt * A_sub[a.stage] : 0.0;
-  io.cb = M.dt * b[a.stage];
+  io.mode = OUT_STAGE;
 }
 
 template <int INTERP, int UPW, int LPB, int W>
@@ -961,13 +913,13 @@ __global__ void __launch_bounds__(64 * SH) __attribute__((amdgpu_waves_per_eu(2)
       PassConst k;
       PassIO io;
       ens_setup(s.a, m, 1, k, io);
-      pass_m_body<1, INTERP, UPW, SH, W, RK_CLASSIC, true>(k, io, local, sh.m);
+      pass_m_body<1, INTERP, UPW, SH, W, true>(k, io, local, sh.m);
       stage_signal(&done_y[m]);
     } else {
       PassConst k;
       PassIO io;
       ens_setup(s.a, m, 2, k, io);
-      pass_m_body<2, INTERP, UPW, SH, W, RK_CLASSIC, true>(k, io, local, sh.m);
+      pass_m_body<2, INTERP, UPW, SH, W, true>(k, io, local, sh.m);
       __syncthreads();
     }
   }
@@ -1036,10 +988,12 @@ void launch_d(const Grid &g, const Scheme &sc, const PassConst &k, const PassIO 
 
 }  // namespace
 
-namespace {
-void pass_args(const Grid &g, const Scheme &sc, const PassBuffers &b, int dir, int mode, int stage, double ca,
-               double cb, const double *dxg, PassConst &k, PassIO &io) {
+void launch_pass(const Grid &g, const Scheme &sc, int dir, const PassBuffers &b, int mode, const double *dxg,
+                 hipStream_t st) {
+  PassConst k;
+  PassIO io;
   for (int d = 0; d < 3; d++) k.n[d] = g.n[d];
+  k.seg = dir == 0 ? 0 : g.seg[dir];
   k.ncell = g.ncell;
   k.gamma = sc.gamma;
   k.gm1 = sc.gamma - 1.0;
@@ -1049,62 +1003,14 @@ void pass_args(const Grid &g, const Scheme &sc, const PassBuffers &b, int dir, i
   io.U = b.U;
   io.R = b.R;
   io.par = b.par;
-  io.u = b.u;
-  io.S = b.S;
-  io.acc = b.acc;
-  io.out = b.out;
   io.Q = b.Q;
+  io.upd = b.upd;
   io.visc = sc.Re > 0 ? 1 : 0;
   io.mode = mode;
-  io.stage = stage;
-  io.ca = ca;
-  io.cb = cb;
-  k.seg = dir == 0 ? 0 : g.seg[dir];
-}
-
-template <int INTERP, int UPW, int W>
-void launch_ssp_t(const Grid &g, const PassConst &k, const PassIO &io, const SspIO &sp, hipStream_t st) {
-  const size_t nb = march_items(g.ncell / g.n[2], g.n[2], k.seg);
-  hipLaunchKernelGGL((k_pass_z_affine<INTERP, UPW, W>), dim3((unsigned)nb), dim3(256), 0, st, k, io, sp);
-}
-
-template <int INTERP, int UPW>
-void launch_ssp_w(const Grid &g, const Scheme &sc, const PassConst &k, const PassIO &io, const SspIO &sp,
-                  hipStream_t st) {
-  if (sc.weno == WENO_MAPPED) launch_ssp_t<INTERP, UPW, WENO_MAPPED>(g, k, io, sp, st);
-  else if (sc.weno == WENO_Z) launch_ssp_t<INTERP, UPW, WENO_Z>(g, k, io, sp, st);
-  else if (sc.weno == WENO_YC) launch_ssp_t<INTERP, UPW, WENO_YC>(g, k, io, sp, st);
-  else if (sc.weno == WENO_OPTIMAL) launch_ssp_t<INTERP, UPW, WENO_OPTIMAL>(g, k, io, sp, st);
-  else launch_ssp_t<INTERP, UPW, WENO_JS>(g, k, io, sp, st);
-}
-}  // namespace
-
-void launch_pass(const Grid &g, const Scheme &sc, int dir, const PassBuffers &b, int mode, int stage, double ca,
-                 double cb, const double *dxg, hipStream_t st) {
-  PassConst k;
-  PassIO io;
-  pass_args(g, sc, b, dir, mode, stage, ca, cb, dxg, k, io);
   if (dir == 0) launch_d<0>(g, sc, k, io, st);
   else if (dir == 1) launch_d<1>(g, sc, k, io, st);
   else launch_d<2>(g, sc, k, io, st);
 }
-
-void launch_pass_z_affine(const Grid &g, const Scheme &sc, const PassBuffers &b, const double *A, const double *B,
-                          double *O1, double *O2, double *O3, double c1, double c2, double c3, int nout,
-                          const double *dxg, hipStream_t st) {
-  PassConst k;
-  PassIO io;
-  pass_args(g, sc, b, 2, OUT_STAGE, 0, 0.0, 0.0, dxg, k, io);
-  const SspIO sp{A, B, O1, O2, O3, c1, c2, c3, nout};
-  if (sc.interp == INTERP_CHAR) {
-    if (sc.upwind == UPWIND_ROE) launch_ssp_w<INTERP_CHAR, UPWIND_ROE>(g, sc, k, io, sp, st);
-    else launch_ssp_w<INTERP_CHAR, UPWIND_RUSANOV>(g, sc, k, io, sp, st);
-  } else {
-    if (sc.upwind == UPWIND_ROE) launch_ssp_w<INTERP_COMP, UPWIND_ROE>(g, sc, k, io, sp, st);
-    else launch_ssp_w<INTERP_COMP, UPWIND_RUSANOV>(g, sc, k, io, sp, st);
-  }
-}
-
 
 namespace {
 template <int INTERP, int UPW, int W>
@@ -1141,8 +1047,8 @@ unsigned ens_items_per_member(int dir, int shape, const int n[3], const int seg[
 }
 
 void launch_ens_pass(const Scheme &sc, int dir, int shape, const EnsMember *mem, int nmem, const unsigned *item0,
-                     unsigned nitems, unsigned grid, const double *U, double *R, double *u, double *S, double *acc,
-                     int stage, hipStream_t st) {
+                     unsigned nitems, unsigned grid, const double *U, double *R, const StageUpdate &upd,
+                     hipStream_t st) {
   EnsArgs a;
   a.mem = mem;
   a.nmem = nmem;
@@ -1154,11 +1060,7 @@ void launch_ens_pass(const Scheme &sc, int dir, int shape, const EnsMember *mem,
   a.eps34 = 0.75 * sc.eps;
   a.U = U;
   a.R = R;
-  a.u = u;
-  a.S = S;
-  a.acc = acc;
-  a.mode = OUT_STAGE;
-  a.stage = stage;
+  a.upd = upd;
   a.visc = sc.Re > 0;
   if (grid == 0 || grid > nitems) grid = nitems;
   if (sc.interp == INTERP_CHAR) {
@@ -1205,8 +1107,8 @@ void stage_launch_t(int weno, int rows, const EnsStageArgs &s, unsigned grid, in
 
 void launch_ens_stage(const Scheme &sc, int rows, const EnsMember *mem, int nmem, const unsigned *const item0[3],
                       const unsigned nitems[3], const unsigned *xgroups0, unsigned xg, unsigned grid, int cus,
-                      unsigned *ctr, unsigned spin_limit, const double *U, double *R, double *u, double *S,
-                      double *acc, int stage, hipStream_t st) {
+                      unsigned *ctr, unsigned spin_limit, const double *U, double *R, const StageUpdate &upd,
+                      hipStream_t st) {
   EnsStageArgs s;
   EnsArgs &a = s.a;
   a.mem = mem;
@@ -1219,11 +1121,7 @@ void launch_ens_stage(const Scheme &sc, int rows, const EnsMember *mem, int nmem
   a.eps34 = 0.75 * sc.eps;
   a.U = U;
   a.R = R;
-  a.u = u;
-  a.S = S;
-  a.acc = acc;
-  a.mode = OUT_STAGE;
-  a.stage = stage;
+  a.upd = upd;
   a.visc = sc.Re > 0;
   for (int d = 0; d < 3; d++) {
     s.item0[d] = item0[d];
