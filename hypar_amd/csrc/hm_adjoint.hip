@@ -26,6 +26,7 @@
 // of the branch the forward evaluation selects.
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <type_traits>
 
 #include "hm_device.h"
@@ -1077,7 +1078,7 @@ __device__ __forceinline__ void rhs_vjp_char_line(
 //  k_visc_vjp_tile   flux adjoints of every cell from its interior readers,
 //                    back through the flux onto Q (stored in QB) and onto the
 //                    gradients (stored in GB, already times dxinv), by tiles
-//                    of VTX x VTY columns marching through VKS z-planes: Q
+//                    of VTX x VTY columns marching through vks z-planes: Q
 //                    and the readers' adjoint weights of a plane sit in LDS
 //                    with a 2-cell halo in x and y, the z stencil in
 //                    registers, so each is read about once per tile;
@@ -1146,72 +1147,128 @@ __device__ __forceinline__ void visc_mu(const double *__restrict__ lam, const do
   for (int k = 0; k < 4; k++) m[k] = cb * l[k] + (nu_in ? ca * n[k] : 0.0);
 }
 
+// A plane of Q and of the readers' adjoint weights with a 2-cell halo in x and
+// y, and the tile's 1/dx and 1/dy, which are zero outside the grid: a reader
+// there does not count.  Two planes: the next one is staged while the slower
+// wavefronts still read this one, which leaves one barrier per plane.
+// A thread stages its own column from the window in its registers and 304 of
+// them one point of the halo, whose loads are in flight during the arithmetic
+// of the plane before.  (When every plane was loaded whole, twice over the
+// tile's halo, and waited for, in segments of 16 planes on any grid: 878 us for
+// eight grids of together 2.33e6 cells against 532 us now.)
+struct ViscVjpShared {
+  double q[2][4][VHY][VHX], m[2][4][VHY][VHX];
+  double dx[VHX], dy[VHY];
+};
+
 __device__ __forceinline__ void visc_vjp_tile(const double *__restrict__ Q, const double *__restrict__ lam,
                                               const double *__restrict__ nu_in, double ca, double cb,
                                               double *__restrict__ QB, double *__restrict__ GB, int nx, int ny,
-                                              int nz, const double *__restrict__ dxg, const ViscC &vc, int b,
-                                              double (&sQ)[4][VHY][VHX], double (&sM)[4][VHY][VHX]) {
+                                              int nz, const double *__restrict__ dxg, const ViscC &vc, int b, int vks,
+                                              ViscVjpShared &sh) {
   const size_t ncell = (size_t)nx * ny * nz;
   const size_t plane = (size_t)nx * ny;
   const int ntx = (nx + VTX - 1) / VTX, nty = (ny + VTY - 1) / VTY;
   const int tx = b % ntx, ty = (b / ntx) % nty, kz = b / (ntx * nty);
-  const int x0 = tx * VTX, y0 = ty * VTY, k0 = kz * VKS;
-  const int lx = threadIdx.x % VTX, ly = threadIdx.x / VTX;
+  const int x0 = tx * VTX, y0 = ty * VTY, k0 = kz * vks;
+  const int t = threadIdx.x, lx = t % VTX, ly = t / VTX;
   const int i = x0 + lx, j = y0 + ly;
   const bool own = i < nx && j < ny;
-  const int ic = own ? i : 0, jc = own ? j : 0;
-  const size_t col = (size_t)jc * nx + ic;
+  // columns past the grid hold the periodic copies, which tile columns next to
+  // the grid's last ones read: x0 + ox spans [x0 - 2, x0 + VTX + 1] and y0 + oy
+  // [y0 - 2, y0 + VTY + 1], which can exceed 2 nx and 2 ny.  The column is a
+  // byte offset of 32 bits, added to a wave-uniform plane address: with 64-bit
+  // lane offsets the compiler keeps one address per array and component in
+  // registers through the loop.  A plane of 2^29 columns, where the offset
+  // would overflow, makes u, lam and nu alone 322 GB (nz >= 5).
+  auto column = [&](int ox, int oy) {
+    return (unsigned)(((y0 + oy + 2 * ny) % ny) * (size_t)nx + (x0 + ox + 2 * nx) % nx) * 8u;
+  };
+  unsigned col = column(lx, ly);
+  // 304 threads also stage a point of the halo: rows -2, -1, VTY, VTY+1 over
+  // the full width, then columns -2, -1, VTX, VTX+1
+  const bool halo = t < 4 * VHX + 4 * VTY;
+  int hx = t % VHX, hy = t / VHX;
+  if (hy >= 2) hy += VTY;
+  if (t >= 4 * VHX) {
+    const int u = t - 4 * VHX, r = u % 4;
+    hx = r < 2 ? r : VTX + r;
+    hy = 2 + u / 4;
+  }
+  unsigned hcol = halo ? column(hx - 2, hy - 2) : col;
   const double *dx = dxg + 3, *dy = dxg + (nx + 6) + 3, *dz = dxg + (nx + 6) + (ny + 6) + 3;
-  const int k1 = min(k0 + VKS, nz);
+  const int k1 = min(k0 + vks, nz);
+  if (t < VHX) sh.dx[t] = x0 + t >= 2 && x0 + t - 2 < nx ? dx[x0 + t - 2] : 0.0;
+  else if (t < VHX + VHY) {
+    const int r = y0 + t - VHX - 2;
+    sh.dy[t - VHX] = r >= 0 && r < ny ? dy[r] : 0.0;
+  }
   const int offs[4] = {-2, -1, 1, 2};
-  // window: Q and the weights m of this column at planes k-2..k+2
-  double q[5][4], m[5][4];
+  // Q and the readers' weights of a column; a missing nu_in reads lam's lines
+  // a second time, so that no branch holds the loads up
+  const double *nu = nu_in ? nu_in : lam;
+  auto at = [](const double *base, unsigned byte) { return *(const double *)((const char *)base + byte); };
+  auto load = [&](size_t pl, unsigned c, double (&qo)[4], double (&l)[4], double (&n)[4]) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      qo[v] = at(Q + v * ncell + pl, c);
+      l[v] = at(lam + (1 + v) * ncell + pl, c);
+      n[v] = at(nu + (1 + v) * ncell + pl, c);
+    }
+  };
+  auto weight = [&](double l, double n) { return cb * l + (nu_in ? ca * n : 0.0); };
+  auto put = [](double *base, unsigned byte, double x) { *(double *)((char *)base + byte) = x; };
+  // window: Q and the weights m of this column at planes k-2..k+2; l and n of
+  // plane k+2 and the halo point of plane k arrive unweighted
+  double q[5][4], m[5][4], l[4], n[4], hq[4] = {0, 0, 0, 0}, hl[4] = {0, 0, 0, 0}, hn[4] = {0, 0, 0, 0};
 #pragma unroll
   for (int s = 0; s < 4; s++) {
-    const size_t c = col + (size_t)wrapn(k0 - 2 + s, nz) * plane;
+    load((size_t)wrapn(k0 - 2 + s, nz) * plane, col, q[s], l, n);
 #pragma unroll
-    for (int v = 0; v < 4; v++) q[s + 1][v] = Q[(size_t)v * ncell + c];
-    visc_mu(lam, nu_in, ca, cb, ncell, c, m[s + 1]);
+    for (int v = 0; v < 4; v++) m[s][v] = weight(l[v], n[v]);
   }
+  load((size_t)wrapn(k0 + 2, nz) * plane, col, q[4], l, n);
+  if (halo) load((size_t)k0 * plane, hcol, hq, hl, hn);
+  int buf = 0;
   for (int k = k0; k < k1; k++) {
+    asm volatile("" : "+v"(col), "+v"(hcol));
+    auto &sq = sh.q[buf];
+    auto &sm = sh.m[buf];
 #pragma unroll
-    for (int s = 0; s < 4; s++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) { q[s][v] = q[s + 1][v]; m[s][v] = m[s + 1][v]; }
-    {
-      const size_t c = col + (size_t)wrapn(k + 2, nz) * plane;
-#pragma unroll
-      for (int v = 0; v < 4; v++) q[4][v] = Q[(size_t)v * ncell + c];
-      visc_mu(lam, nu_in, ca, cb, ncell, c, m[4]);
+    for (int v = 0; v < 4; v++) {
+      m[4][v] = weight(l[v], n[v]);
+      sq[v][ly + 2][lx + 2] = q[2][v];
+      sm[v][ly + 2][lx + 2] = m[2][v];
     }
-    // tile of plane k with halo
-    const size_t pk = (size_t)k * plane;
-    for (int c = threadIdx.x; c < VHX * VHY; c += VTX * VTY) {
-      const int hx = c % VHX, hy = c / VHX;
-      // x0 - 2 + hx spans [x0 - 2, x0 + VTX + 1] and y0 - 2 + hy spans
-      // [y0 - 2, y0 + VTY + 1], which can exceed 2 nx and 2 ny
-      const int gi = (x0 - 2 + hx + 2 * nx) % nx, gj = (y0 - 2 + hy + 2 * ny) % ny;
-      const size_t h = pk + (size_t)gj * nx + gi;
-      double mh[4];
-      visc_mu(lam, nu_in, ca, cb, ncell, h, mh);
+    if (halo)
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        sQ[v][hy][hx] = Q[(size_t)v * ncell + h];
-        sM[v][hy][hx] = mh[v];
+        sq[v][hy][hx] = hq[v];
+        sm[v][hy][hx] = weight(hl[v], hn[v]);
       }
-    }
     __syncthreads();
+    double qn[4] = {0, 0, 0, 0};
+    if (k + 1 < k1) {
+      load((size_t)wrapn(k + 3, nz) * plane, col, qn, l, n);
+      if (halo) load((size_t)(k + 1) * plane, hcol, hq, hl, hn);
+    }
     if (own) {
       double gr[4][3];
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        const double *r = &sQ[c][ly + 2][0];
-        gr[c][0] = d4c(r[lx], r[lx + 1], r[lx + 3], r[lx + 4]) * dx[i];
-        gr[c][1] = d4c(sQ[c][ly][lx + 2], sQ[c][ly + 1][lx + 2], sQ[c][ly + 3][lx + 2], sQ[c][ly + 4][lx + 2]) * dy[j];
+        const double *r = &sq[c][ly + 2][0];
+        gr[c][0] = d4c(r[lx], r[lx + 1], r[lx + 3], r[lx + 4]) * sh.dx[lx + 2];
+        gr[c][1] = d4c(sq[c][ly][lx + 2], sq[c][ly + 1][lx + 2], sq[c][ly + 3][lx + 2], sq[c][ly + 4][lx + 2]) * sh.dy[ly + 2];
         gr[c][2] = d4c(q[0][c], q[1][c], q[3][c], q[4][c]) * dz[k];
       }
       const double qc[4] = {q[2][0], q[2][1], q[2][2], q[2][3]};
       const double mu = pow076(qc[3]);
+      double zw[5];  // dz has ghost entries; a reader out there does not count
+#pragma unroll
+      for (int s = 0; s < 5; s++) {
+        const double w = dz[k - 2 + s];
+        zw[s] = (unsigned)(k - 2 + s) < (unsigned)nz ? w : 0.0;
+      }
       double qb[4] = {0, 0, 0, 0}, grb[4][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, mub = 0.0;
       // direction by direction: reader r = pos - s reads this cell's flux
       // with weight d4w(s) dxinv(r), inside the grid only
@@ -1221,29 +1278,37 @@ __device__ __forceinline__ void visc_vjp_tile(const double *__restrict__ Q, cons
 #pragma unroll
         for (int s = 0; s < 4; s++) {
           const int o = offs[s];
-          const int r = (d == 0 ? i : (d == 1 ? j : k)) - o;
-          if (r >= 0 && r < (d == 0 ? nx : (d == 1 ? ny : nz))) {
-            const double w = d4w(o) * (d == 0 ? dx[r] : (d == 1 ? dy[r] : dz[r]));
+          const double w = d4w(o) * (d == 0 ? sh.dx[lx + 2 - o]
+                                            : (d == 1 ? sh.dy[ly + 2 - o] : zw[2 - o]));
 #pragma unroll
-            for (int c = 0; c < 4; c++)
-              fb[c] += w * (d == 0 ? sM[c][ly + 2][lx + 2 - o] : (d == 1 ? sM[c][ly + 2 - o][lx + 2] : m[2 - o][c]));
-          }
+          for (int c = 0; c < 4; c++)
+            fb[c] += w * (d == 0 ? sm[c][ly + 2][lx + 2 - o] : (d == 1 ? sm[c][ly + 2 - o][lx + 2] : m[2 - o][c]));
         }
         if (d == 0) mub += visc_flux_vjp<0>(qc, gr, mu, vc, fb, qb, grb);
         else if (d == 1) mub += visc_flux_vjp<1>(qc, gr, mu, vc, fb, qb, grb);
         else mub += visc_flux_vjp<2>(qc, gr, mu, vc, fb, qb, grb);
+        __builtin_amdgcn_sched_barrier(0);  // the next direction's weights are read after this one's use
       }
       qb[3] += mub * (0.76 * mu * nr_rcp(qc[3]));
-      const size_t idx = pk + col;
-      const double dxe[3] = {dx[i], dy[j], dz[k]};
+      const size_t pl = (size_t)k * plane;
+      const double dxe[3] = {sh.dx[lx + 2], sh.dy[ly + 2], dz[k]};
 #pragma unroll
       for (int c = 0; c < 4; c++) {
-        QB[(size_t)c * ncell + idx] = qb[c];
+        put(QB + c * ncell + pl, col, qb[c]);
 #pragma unroll
-        for (int e = 0; e < 3; e++) GB[(size_t)(c * 3 + e) * ncell + idx] = grb[c][e] * dxe[e];
+        for (int e = 0; e < 3; e++) put(GB + (c * 3 + e) * ncell + pl, col, grb[c][e] * dxe[e]);
       }
     }
-    __syncthreads();
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        q[s][v] = q[s + 1][v];
+        m[s][v] = m[s + 1][v];
+      }
+      q[4][v] = qn[v];
+    }
+    buf ^= 1;
   }
 }
 
@@ -1369,13 +1434,16 @@ __global__ void __launch_bounds__(VJP_CHAR_LINE_MAX) __attribute__((amdgpu_waves
 __global__ void __launch_bounds__(VT) k_visc_vjp_tile(const double *__restrict__ Q, const double *__restrict__ lam,
                                                      const double *__restrict__ nu_in, double ca, double cb,
                                                      double *__restrict__ QB, double *__restrict__ GB, int nx, int ny,
-                                                     int nz, const double *__restrict__ dxg, ViscC vc) {
-  __shared__ double sQ[4][VHY][VHX], sM[4][VHY][VHX];
-  visc_vjp_tile(Q, lam, nu_in, ca, cb, QB, GB, nx, ny, nz, dxg, vc, blockIdx.x, sQ, sM);
+                                                     int nz, const double *__restrict__ dxg, ViscC vc, int vks) {
+  __shared__ ViscVjpShared sh;
+  visc_vjp_tile(Q, lam, nu_in, ca, cb, QB, GB, nx, ny, nz, dxg, vc, blockIdx.x, vks, sh);
 }
 
+// one wavefront per block: a grid has few lines, and their scattered loads
+// are spread over more CUs (x, 5280 lines of 48 cells: 15 us; 30 us at four
+// wavefronts)
 template <int DIR>
-__global__ void __launch_bounds__(256) k_visc_vjp_ghost(const double *__restrict__ Q, const double *__restrict__ lam,
+__global__ void __launch_bounds__(64) k_visc_vjp_ghost(const double *__restrict__ Q, const double *__restrict__ lam,
                                                         const double *__restrict__ nu_in, double ca, double cb,
                                                         double *__restrict__ QB, int nx, int ny, int nz,
                                                         const double *__restrict__ dxg, ViscC vc) {
@@ -1489,8 +1557,8 @@ __global__ void __launch_bounds__(256) k_ens_vjp_prims(EnsVjp a, size_t ncell) {
 
 // tiles of all members; tiles0 holds each member's first tile
 __global__ void __launch_bounds__(VT) k_ens_visc_vjp_tile(EnsVjp a, const unsigned *__restrict__ tiles0,
-                                                         unsigned ntiles) {
-  __shared__ double sQ[4][VHY][VHX], sM[4][VHY][VHX];
+                                                         unsigned ntiles, int vks) {
+  __shared__ ViscVjpShared sh;
   const unsigned item = blockIdx.x;  // one block per tile (a loop over tiles spills 12 B per lane)
   if (item >= ntiles) return;
   const int m = ens_find(tiles0, a.nmem, item);
@@ -1498,11 +1566,11 @@ __global__ void __launch_bounds__(VT) k_ens_visc_vjp_tile(EnsVjp a, const unsign
   const double *Q = a.work + 20 * M.off;
   double *QB = a.work + 20 * M.off + 4 * M.ncell, *GB = a.work + 20 * M.off + 8 * M.ncell;
   visc_vjp_tile(Q, a.lam + 5 * M.off, a.nu_in ? a.nu_in + 5 * M.off : nullptr, M.dt * a.A, M.dt * a.B, QB, GB,
-                M.n[0], M.n[1], M.n[2], M.dxg, a.vc, (int)(item - tiles0[m]), sQ, sM);
+                M.n[0], M.n[1], M.n[2], M.dxg, a.vc, (int)(item - tiles0[m]), vks, sh);
 }
 
 template <int DIR>
-__global__ void __launch_bounds__(256) k_ens_visc_vjp_ghost(EnsVjp a, const unsigned *__restrict__ first,
+__global__ void __launch_bounds__(64) k_ens_visc_vjp_ghost(EnsVjp a, const unsigned *__restrict__ first,
                                                             unsigned nitems) {
   const unsigned item = blockIdx.x * blockDim.x + threadIdx.x;
   if (item >= nitems) return;
@@ -1600,18 +1668,40 @@ void launch_rhs_vjp(const Grid &g, const Scheme &sc, const double *u, const doub
     double *Q = work;
     const ViscC vc = {sc.gamma, 1.0 / sc.Re, 1.0 / (sc.gamma - 1.0), 1.0 / sc.Pr};
     launch_prims(g, sc, u, Q, st);
-    hipLaunchKernelGGL(k_visc_vjp_tile, dim3(visc_tiles(g.n[0], g.n[1], g.n[2])), dim3(VT), 0, st, Q, lam, nu_in, ca,
-                       cb, QB, GB, g.n[0], g.n[1], g.n[2], dxg, vc);
-    const unsigned gx = (unsigned)((g.ncell / g.n[0] + 255) / 256), gy = (unsigned)((g.ncell / g.n[1] + 255) / 256),
-                   gz = (unsigned)((g.ncell / g.n[2] + 255) / 256);
-    hipLaunchKernelGGL(k_visc_vjp_ghost<0>, dim3(gx), dim3(256), 0, st, Q, lam, nu_in, ca, cb, QB, g.n[0], g.n[1],
+    hipLaunchKernelGGL(k_visc_vjp_tile, dim3(visc_tiles(g.n[0], g.n[1], g.n[2], g.vks)), dim3(VT), 0, st, Q, lam, nu_in,
+                       ca, cb, QB, GB, g.n[0], g.n[1], g.n[2], dxg, vc, g.vks);
+    const unsigned gx = (unsigned)((g.ncell / g.n[0] + 63) / 64), gy = (unsigned)((g.ncell / g.n[1] + 63) / 64),
+                   gz = (unsigned)((g.ncell / g.n[2] + 63) / 64);
+    hipLaunchKernelGGL(k_visc_vjp_ghost<0>, dim3(gx), dim3(64), 0, st, Q, lam, nu_in, ca, cb, QB, g.n[0], g.n[1],
                        g.n[2], dxg, vc);
-    hipLaunchKernelGGL(k_visc_vjp_ghost<1>, dim3(gy), dim3(256), 0, st, Q, lam, nu_in, ca, cb, QB, g.n[0], g.n[1],
+    hipLaunchKernelGGL(k_visc_vjp_ghost<1>, dim3(gy), dim3(64), 0, st, Q, lam, nu_in, ca, cb, QB, g.n[0], g.n[1],
                        g.n[2], dxg, vc);
-    hipLaunchKernelGGL(k_visc_vjp_ghost<2>, dim3(gz), dim3(256), 0, st, Q, lam, nu_in, ca, cb, QB, g.n[0], g.n[1],
+    hipLaunchKernelGGL(k_visc_vjp_ghost<2>, dim3(gz), dim3(64), 0, st, Q, lam, nu_in, ca, cb, QB, g.n[0], g.n[1],
                        g.n[2], dxg, vc);
   }
   launch_vjp_dir<0>(g, sc, u, lam, nu_in, ca, cb, nu, L, last, dxg, st, QB, GB);
+}
+
+// With W blocks on 256 CUs, one block each, and p + 2 plane times a block, the
+// length p with the least ceil(W/256) (p + 2); a shorter one has to win 3%.
+int visc_vjp_segment(int count, const int (*n)[3]) {
+  constexpr int CUS = 256;
+  int nmax = 0;
+  for (int m = 0; m < count; m++) nmax = n[m][2] > nmax ? n[m][2] : nmax;
+  int best = nmax;
+  double tbest = 0.0;
+  for (int parts = 1; parts <= nmax; parts++) {
+    const int p = (nmax + parts - 1) / parts;
+    if (parts > 1 && p == (nmax + parts - 2) / (parts - 1)) continue;
+    double blocks = 0.0;
+    for (int m = 0; m < count; m++) blocks += visc_tiles(n[m][0], n[m][1], n[m][2], p);
+    const double t = ceil(blocks / CUS) * (p + 2);
+    if (parts == 1 || t < 0.97 * tbest) {
+      tbest = t;
+      best = p;
+    }
+  }
+  return best;
 }
 
 bool ens_vjp_supported(const Scheme &sc, const int nmax[3]) {
@@ -1680,12 +1770,12 @@ void launch_ens_rhs_vjp(const Scheme &sc, const EnsVjpPlan &p, const double *u, 
   if (visc) {
     const unsigned nb = (unsigned)((p.ncell + 255) / 256);
     hipLaunchKernelGGL(k_ens_vjp_prims, dim3(nb), dim3(256), 0, st, a, p.ncell);
-    hipLaunchKernelGGL(k_ens_visc_vjp_tile, dim3(p.ntiles), dim3(VT), 0, st, a, p.tiles0, p.ntiles);
-    hipLaunchKernelGGL(k_ens_visc_vjp_ghost<0>, dim3((p.nlines[0] + 255) / 256), dim3(256), 0, st, a, p.lines0[0],
+    hipLaunchKernelGGL(k_ens_visc_vjp_tile, dim3(p.ntiles), dim3(VT), 0, st, a, p.tiles0, p.ntiles, p.vks);
+    hipLaunchKernelGGL(k_ens_visc_vjp_ghost<0>, dim3((p.nlines[0] + 63) / 64), dim3(64), 0, st, a, p.lines0[0],
                        p.nlines[0]);
-    hipLaunchKernelGGL(k_ens_visc_vjp_ghost<1>, dim3((p.nlines[1] + 255) / 256), dim3(256), 0, st, a, p.lines0[1],
+    hipLaunchKernelGGL(k_ens_visc_vjp_ghost<1>, dim3((p.nlines[1] + 63) / 64), dim3(64), 0, st, a, p.lines0[1],
                        p.nlines[1]);
-    hipLaunchKernelGGL(k_ens_visc_vjp_ghost<2>, dim3((p.nlines[2] + 255) / 256), dim3(256), 0, st, a, p.lines0[2],
+    hipLaunchKernelGGL(k_ens_visc_vjp_ghost<2>, dim3((p.nlines[2] + 63) / 64), dim3(64), 0, st, a, p.lines0[2],
                        p.nlines[2]);
   }
   // the x lines add the viscous share (QB, GB of a.work) before their own

@@ -276,6 +276,7 @@ hm_status hm_create(const hm_config *cfg, hm_solver **out) {
   s->g.seg[0] = s->g.n[0];
   for (int d = 1; d < 3; d++) hm::march_segments(1, &s->g.n, d, &s->g.seg[d]);
   s->g.pks = hm::visc_segment(1, &s->g.n);
+  s->g.vks = hm::visc_vjp_segment(1, &s->g.n);
   s->sc.interp = cfg->interp == HM_INTERP_CHARACTERISTIC ? hm::INTERP_CHAR : hm::INTERP_COMP;
   s->sc.upwind = cfg->upwind == HM_UPWIND_ROE ? hm::UPWIND_ROE : hm::UPWIND_RUSANOV;
   s->sc.gamma = cfg->gamma;
@@ -989,7 +990,7 @@ struct hm_ensemble {
   double *par = nullptr, *Q = nullptr;
   unsigned *ptiles0 = nullptr, *tiles0 = nullptr;
   unsigned nptiles = 0, ntiles = 0;
-  int pks = 1;  // planes per z segment of the viscous-term launch
+  int pks = 1, vks = 1;  // planes per z segment of the viscous-term launch and of its adjoint
   unsigned *item0[2][3] = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
   unsigned nitems[2][3] = {{0, 0, 0}, {0, 0, 0}};
   // x items of the one-launch-per-stage kernel (ENS_STAGE_XG line groups each)
@@ -1203,6 +1204,7 @@ hm_status hm_ensemble_create(const hm_config *members, int nmembers, hm_ensemble
       for (int m = 0; m < nmembers; m++) e->mem[m].seg[d] = d == 0 ? e->mem[m].n[0] : seg[m];
     }
     e->pks = hm::visc_segment(nmembers, (const int(*)[3])dims.data());
+    e->vks = hm::visc_vjp_segment(nmembers, (const int(*)[3])dims.data());
   }
   const size_t n5 = 5 * e->ncell;
   if (hipGetDevice(&e->device) != hipSuccess) {
@@ -1237,7 +1239,7 @@ hm_status hm_ensemble_create(const hm_config *members, int nmembers, hm_ensemble
     }
     for (int m = 0; m < nmembers; m++) {
       const int *n = e->mem[m].n;
-      pre[m + 1] = pre[m] + hm::visc_tiles(n[0], n[1], n[2]);
+      pre[m + 1] = pre[m] + hm::visc_tiles(n[0], n[1], n[2], e->vks);
     }
     e->ntiles = pre[nmembers];
     if (hipMalloc((void **)&e->tiles0, pre.size() * sizeof(unsigned)) != hipSuccess ||
@@ -1573,6 +1575,7 @@ static hm_status ens_reverse_sweep(hm_ensemble *e, double *lam) {
   }
   vp.tiles0 = e->tiles0;
   vp.ntiles = e->ntiles;
+  vp.vks = e->vks;
   const int nck = (N + K - 1) / K;
   double *cur = lam;
   for (int seg = nck - 1; seg >= 0; seg--) {

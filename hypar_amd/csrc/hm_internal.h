@@ -24,6 +24,7 @@ struct Grid {
   size_t ncell;
   int seg[3];  // cells per march segment of the y and z passes (march_segments)
   int pks;     // planes per segment of the viscous-term kernel (visc_segment)
+  int vks;     // planes per segment of its adjoint (visc_vjp_segment)
 };
 
 struct Scheme {
@@ -124,16 +125,16 @@ void launch_pass(const Grid &g, const Scheme &sc, int dir, const PassBuffers &b,
 // primitive variables (u, v, w, T) of u into Q
 void launch_prims(const Grid &g, const Scheme &sc, const double *u, double *Q, hipStream_t st);
 
-// tiles of the viscous kernels (hm_kernels.hip, hm_adjoint.hip): a block
-// owns VTX x VTY (x, y) columns and marches through VKS z-planes
-constexpr int VTX = 64, VTY = 8, VKS = 16;
+// tiles of the viscous adjoint kernel (hm_adjoint.hip): a block owns VTX x VTY
+// (x, y) columns and marches through a z segment of vks planes
+constexpr int VTX = 64, VTY = 8;
 constexpr int VT = VTX * VTY;  // threads of a viscous block
 constexpr int VHX = VTX + 4, VHY = VTY + 4;
-
-// tiles (x, y, z-segment) of a grid
-__host__ __device__ inline unsigned visc_tiles(int nx, int ny, int nz) {
-  return (unsigned)(((nx + VTX - 1) / VTX) * ((ny + VTY - 1) / VTY) * ((nz + VKS - 1) / VKS));
+__host__ __device__ inline unsigned visc_tiles(int nx, int ny, int nz, int vks) {
+  return (unsigned)(((nx + VTX - 1) / VTX) * ((ny + VTY - 1) / VTY) * ((nz + vks - 1) / vks));
 }
+// segment length of that kernel over `count` grids that run together
+int visc_vjp_segment(int count, const int (*n)[3]);
 
 // tiles of the viscous-term kernel (hm_kernels.hip): a block owns PTX x PTY
 // (x, y) columns and marches through a z segment of pks planes
@@ -220,6 +221,7 @@ struct EnsVjpPlan {
   int nmax[3];
   const unsigned *tiles0;  // viscous members: each member's first viscous tile (nmem + 1 entries)
   unsigned ntiles;
+  int vks;                 // planes per tile
 };
 bool ens_vjp_supported(const Scheme &sc, const int nmax[3]);
 int ens_vjp_threads(int nmax);                 // block size of the line VJPs along a direction

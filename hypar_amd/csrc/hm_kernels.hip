@@ -540,10 +540,10 @@ static ViscParams visc_params(const Scheme &sc) {
 }
 
 // A segment of p planes marches p + 4 and starts on 4 more, and a CU holds one
-// block, so with W blocks on 256 CUs one grid takes ceil(W/256) (p + 6) plane
-// times; an ensemble, whose blocks differ in length, its total over 256 and
-// half the longest.  The length with the least such time is taken; a shorter
-// one has to win 3%.
+// block, so W blocks on 256 CUs take ceil(W/256) (p + 6) plane times.  The
+// length with the least such time is taken; a shorter one has to win 3%.  (For
+// grids that run together, total work over 256 plus half a block chose segments
+// too long: 463 us against 349 for the eight of 2.33e6 cells.)
 int visc_segment(int count, const int (*n)[3]) {
   constexpr int CUS = 256;
   int nmax = 0;
@@ -553,13 +553,9 @@ int visc_segment(int count, const int (*n)[3]) {
   for (int parts = 1; parts <= nmax; parts++) {
     const int p = (nmax + parts - 1) / parts;
     if (parts > 1 && p == (nmax + parts - 2) / (parts - 1)) continue;
-    double blocks = 0.0, work = 0.0;
-    for (int m = 0; m < count; m++) {
-      const double b = par_tiles(n[m][0], n[m][1], n[m][2], p);
-      blocks += b;
-      work += b * ((n[m][2] < p ? n[m][2] : p) + 6);
-    }
-    const double t = count == 1 ? ceil(blocks / CUS) * (p + 6) : fmax(work / CUS + 0.5 * (p + 6), p + 6);
+    double blocks = 0.0;
+    for (int m = 0; m < count; m++) blocks += par_tiles(n[m][0], n[m][1], n[m][2], p);
+    const double t = ceil(blocks / CUS) * (p + 6);
     if (parts == 1 || t < 0.97 * tbest) {
       tbest = t;
       best = p;
