@@ -76,7 +76,7 @@ size_t auto_tape_budget(size_t held_bytes) {
 struct hm_solver {
   hm_solver() : g(), sc(), device(0), stream(nullptr), dxg(nullptr), R(nullptr), par(nullptr), Q(nullptr),
                 S{nullptr, nullptr, nullptr},
-                part(nullptr), part_host(nullptr), npart(0), tmp(nullptr), tmp_elems(0),
+                part_host(nullptr), npart(0), tmp(nullptr), tmp_elems(0),
                 tape_nsteps(0), tape_every(0), tape_dt(0.0) {
     for (int i = 0; i < TAPE_SETS; i++) tape_holds[i] = -1;
   }
@@ -89,8 +89,7 @@ struct hm_solver {
   double *par;        // viscous term, 4*ncell (viscous runs only)
   double *Q;          // primitive variables u, v, w, T, 4*ncell (viscous only)
   double *S[3];       // RK stage states
-  double *part;       // reduction partials (device)
-  double *part_host;  // reduction partials (pinned host)
+  double *part_host;  // reduction partials: pinned host memory that the kernels write
   unsigned npart;
   double *tmp;        // layout-conversion staging
   size_t tmp_elems;
@@ -239,7 +238,7 @@ const char *hm_version(void) { return "hypar-mi355x 0.1 (gfx950, fp64)"; }
 void hm_destroy(hm_solver *s) {
   if (!s) return;
   hm::drop_bindings(s);
-  double *bufs[] = {s->dxg, s->R, s->par, s->Q, s->S[0], s->S[1], s->S[2], s->part, s->tmp};
+  double *bufs[] = {s->dxg, s->R, s->par, s->Q, s->S[0], s->S[1], s->S[2], s->tmp};
   for (double *b : bufs)
     if (b) (void)hipFree(b);
   if (s->part_host) (void)hipHostFree(s->part_host);
@@ -313,8 +312,7 @@ hm_status hm_create(const hm_config *cfg, hm_solver **out) {
   if ((st = dmalloc(&s->S[0], n5)) != HM_OK) goto bad;
   if ((st = dmalloc(&s->S[1], n5)) != HM_OK) goto bad;
   if ((st = dmalloc(&s->S[2], n5)) != HM_OK) goto bad;
-  s->npart = hm::reduction_blocks(n5);
-  if ((st = dmalloc(&s->part, s->npart)) != HM_OK) goto bad;
+  s->npart = 5 * hm::reduction_blocks(s->g.ncell);  // at least reduction_blocks(n5)
   if (hipHostMalloc((void **)&s->part_host, s->npart * sizeof(double), hipHostMallocDefault) != hipSuccess) {
     st = fail(HM_ERR_NOMEM, "hm_create: pinned host allocation failed");
     goto bad;
@@ -446,9 +444,8 @@ hm_status hm_cfl(hm_solver *s, const double *u, double dt, double *cfl) {
   if (st != HM_OK) return st;
   if (!cfl) return fail(HM_ERR_ARG, "hm_cfl: cfl is NULL");
   unsigned nb = hm::reduction_blocks(s->g.ncell);
-  hm::launch_cfl(s->g, s->sc, u, s->part, nb, s->dxg, dt, s->stream);
+  hm::launch_cfl(s->g, s->sc, u, s->part_host, nb, s->dxg, dt, s->stream);
   if ((st = check_launch("hm_cfl")) != HM_OK) return st;
-  HM_HIP(hipMemcpyAsync(s->part_host, s->part, nb * sizeof(double), hipMemcpyDeviceToHost, s->stream));
   HM_HIP(hipStreamSynchronize(s->stream));
   double m = 0.0;
   for (unsigned i = 0; i < nb; i++) m = s->part_host[i] > m ? s->part_host[i] : m;
@@ -462,16 +459,15 @@ hm_status hm_volume_integral(hm_solver *s, const double *u, double *out) {
   if (st != HM_OK) return st;
   if (!out) return fail(HM_ERR_ARG, "hm_volume_integral: out is NULL");
   unsigned nb = hm::reduction_blocks(s->g.ncell);
-  if (5 * nb > s->npart) nb = s->npart / 5 > 0 ? s->npart / 5 : 1;
-  hm::launch_volint(s->g, u, s->part, nb, s->dxg, s->stream);
+  hm::launch_volint(s->g, u, s->part_host, nb, s->dxg, s->stream);
   if ((st = check_launch("hm_volume_integral")) != HM_OK) return st;
-  HM_HIP(hipMemcpyAsync(s->part_host, s->part, 5 * nb * sizeof(double), hipMemcpyDeviceToHost, s->stream));
   HM_HIP(hipStreamSynchronize(s->stream));
+  double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  for (unsigned b = 0; b < nb; b++)
+    for (int v = 0; v < 5; v++) sum[v] += s->part_host[(size_t)b * 5 + v];
   for (int v = 0; v < 5; v++) {
-    double sum = 0.0;
-    for (unsigned b = 0; b < nb; b++) sum += s->part_host[(size_t)v * nb + b];
-    out[v] = sum;
-    if (!std::isfinite(sum)) return fail(HM_ERR_NONFINITE, "hm_volume_integral: state holds NaN/Inf");
+    out[v] = sum[v];
+    if (!std::isfinite(sum[v])) return fail(HM_ERR_NONFINITE, "hm_volume_integral: state holds NaN/Inf");
   }
   return HM_OK;
 }
@@ -483,9 +479,8 @@ hm_status hm_step_norm(hm_solver *s, const double *a, const double *b, double *n
   if (!norm) return fail(HM_ERR_ARG, "hm_step_norm: norm is NULL");
   const size_t n5 = 5 * s->g.ncell;
   unsigned nb = hm::reduction_blocks(n5);
-  hm::launch_sqdiff(a, b, s->part, nb, n5, s->stream);
+  hm::launch_sqdiff(a, b, s->part_host, nb, n5, s->stream);
   if ((st = check_launch("hm_step_norm")) != HM_OK) return st;
-  HM_HIP(hipMemcpyAsync(s->part_host, s->part, nb * sizeof(double), hipMemcpyDeviceToHost, s->stream));
   HM_HIP(hipStreamSynchronize(s->stream));
   double sum = 0.0;
   for (unsigned i = 0; i < nb; i++) sum += s->part_host[i];

@@ -68,7 +68,7 @@ void launch_visc_par(const Grid &g, const Scheme &sc, const double *Q, double *p
 // par as a five-variable array with a zero mass component
 void launch_par_out(const Grid &g, const double *par, double *out, hipStream_t st);
 unsigned reduction_blocks(size_t n);
-// volume integral partials: part[v*nb + block], 5*nb entries
+// volume integral partials: part[5*block + v], 5*nb entries
 void launch_volint(const Grid &g, const double *u, double *part, unsigned nb, const double *dxg, hipStream_t st);
 void launch_cfl(const Grid &g, const Scheme &sc, const double *u, double *part, unsigned nb,
                 const double *dxg, double dt, hipStream_t st);

@@ -433,8 +433,19 @@ __global__ void __launch_bounds__(256) k_par_out(const double *__restrict__ par,
 }
 
 // ---------------------------------------------------------------------------
-// reductions: CFL max and squared-difference sum
+// reductions: CFL max, squared-difference sum, volume integrals
+//
+// Bound by the reads of the states.  512 blocks of 1024 threads fill the 256
+// CUs and leave 512 partials (five of each for the integrals), few enough for
+// the host to fold: the kernels write them into pinned host memory, without a
+// copy.  At 128^3: k_cfl 17.4 us (84 MB, 4.8 TB/s; 20.1 before), k_volint 14.7
+// (22.0 before, on 409 blocks of 256), k_sqdiff 25.3 for 168 MB; the three calls
+// 123 -> 109 us, the rest of it launches and waits.  (A last block that folds on
+// the GPU costs each block a release to memory behind its XCD's cache: 45 us
+// over 2048 blocks.)
 // ---------------------------------------------------------------------------
+constexpr int RED_THREADS = 1024, RED_WAVES = RED_THREADS / 64;
+
 __device__ __forceinline__ double wave_max(double v) {
   for (int off = 32; off > 0; off >>= 1) v = fmax(v, __shfl_down(v, off, 64));
   return v;
@@ -444,25 +455,47 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// The cells t, t + T, t + 2T, ... of thread t of a launch of T threads, as
+// (i, j, k): T < 2^20, so the divisions are of 32 bits and once a thread, and
+// a step is additions with a carry instead of three 64-bit remainders a cell.
+struct CellWalk {
+  int i, j, k, si, sj, sk, nx, ny;
+  __device__ __forceinline__ CellWalk(int nx_, int ny_) : nx(nx_), ny(ny_) {
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x, T = gridDim.x * blockDim.x;
+    const unsigned r = t / (unsigned)nx, R = T / (unsigned)nx;
+    i = (int)(t - r * nx);
+    k = (int)(r / (unsigned)ny);
+    j = (int)(r - (unsigned)k * ny);
+    si = (int)(T - R * nx);
+    sk = (int)(R / (unsigned)ny);
+    sj = (int)(R - (unsigned)sk * ny);
+  }
+  __device__ __forceinline__ void step() {
+    i += si;
+    j += sj;
+    k += sk;
+    if (i >= nx) { i -= nx; j++; }
+    if (j >= ny) { j -= ny; k++; }
+  }
+};
+
 // per-block partial maxima of the local CFL; NaN propagates as +Inf flag
-__global__ void __launch_bounds__(256) k_cfl(const double *__restrict__ u, double *__restrict__ part,
+__global__ void __launch_bounds__(RED_THREADS) k_cfl(const double *__restrict__ u, double *__restrict__ part,
                                              int nx, int ny, int nz, const double *__restrict__ dxg,
                                              double gamma, double dt) {
   const size_t ncell = (size_t)nx * ny * nz;
-  __shared__ double red[4];
+  __shared__ double red[RED_WAVES];
   double m = 0.0;
+  CellWalk cell(nx, ny);
   for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < ncell;
-       idx += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(idx % nx);
-    const int j = (int)((idx / nx) % ny);
-    const int k = (int)(idx / ((size_t)nx * ny));
+       idx += (size_t)gridDim.x * blockDim.x, cell.step()) {
     double s[NV];
     for (int v = 0; v < NV; v++) s[v] = u[(size_t)v * ncell + idx];
     Prim q = flowvar(s, gamma);
     const double c = sqrt(gamma * q.P / q.rho);
-    const double lx = (fabs(q.vx) + c) * dt * dxg[3 + i];
-    const double ly = (fabs(q.vy) + c) * dt * dxg[(nx + 6) + 3 + j];
-    const double lz = (fabs(q.vz) + c) * dt * dxg[(nx + 6) + (ny + 6) + 3 + k];
+    const double lx = (fabs(q.vx) + c) * dt * dxg[3 + cell.i];
+    const double ly = (fabs(q.vy) + c) * dt * dxg[(nx + 6) + 3 + cell.j];
+    const double lz = (fabs(q.vz) + c) * dt * dxg[(nx + 6) + (ny + 6) + 3 + cell.k];
     double l = fmax(fmax(lx, ly), lz);
     if (!(l == l) || l > 1.0e300) l = __builtin_inf();
     m = fmax(m, l);
@@ -473,14 +506,14 @@ __global__ void __launch_bounds__(256) k_cfl(const double *__restrict__ u, doubl
   __syncthreads();
   if (threadIdx.x == 0) {
     double r = red[0];
-    for (int q = 1; q < (int)(blockDim.x >> 6); q++) r = fmax(r, red[q]);
+    for (int q = 1; q < RED_WAVES; q++) r = fmax(r, red[q]);
     part[blockIdx.x] = r;
   }
 }
 
-__global__ void __launch_bounds__(256) k_sqdiff(const double *__restrict__ a, const double *__restrict__ b,
+__global__ void __launch_bounds__(RED_THREADS) k_sqdiff(const double *__restrict__ a, const double *__restrict__ b,
                                                 double *__restrict__ part, size_t n) {
-  __shared__ double red[4];
+  __shared__ double red[RED_WAVES];
   double s = 0.0;
   for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
        idx += (size_t)gridDim.x * blockDim.x) {
@@ -493,7 +526,7 @@ __global__ void __launch_bounds__(256) k_sqdiff(const double *__restrict__ a, co
   __syncthreads();
   if (threadIdx.x == 0) {
     double r = 0.0;
-    for (int q = 0; q < (int)(blockDim.x >> 6); q++) r += red[q];
+    for (int q = 0; q < RED_WAVES; q++) r += red[q];
     part[blockIdx.x] = r;
   }
 }
@@ -595,21 +628,19 @@ void launch_par_out(const Grid &g, const double *par, double *out, hipStream_t s
 // Volume integral of every conserved variable: sum of u dV over the
 // interior cells with dV = 1/dxinv_x 1/dxinv_y 1/dxinv_z
 // (src/HyParFunctions/VolumeIntegral.c:14-50); one partial per block and
-// variable, part[v*gridDim.x + block].
-__global__ void __launch_bounds__(256) k_volint(const double *__restrict__ u, double *__restrict__ part, int nx,
+// variable, part[5*block + v].
+__global__ void __launch_bounds__(RED_THREADS) k_volint(const double *__restrict__ u, double *__restrict__ part, int nx,
                                                 int ny, int nz, const double *__restrict__ dxg) {
   const size_t ncell = (size_t)nx * ny * nz;
-  __shared__ double red[NV][4];
+  __shared__ double red[NV][RED_WAVES];
   double acc[NV] = {0, 0, 0, 0, 0};
+  CellWalk cell(nx, ny);
   for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < ncell;
-       idx += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(idx % nx);
-    const int j = (int)((idx / nx) % ny);
-    const int k = (int)(idx / ((size_t)nx * ny));
+       idx += (size_t)gridDim.x * blockDim.x, cell.step()) {
     double dV = 1.0;
-    dV *= 1.0 / dxg[3 + i];
-    dV *= 1.0 / dxg[(nx + 6) + 3 + j];
-    dV *= 1.0 / dxg[(nx + 6) + (ny + 6) + 3 + k];
+    dV *= 1.0 / dxg[3 + cell.i];
+    dV *= 1.0 / dxg[(nx + 6) + 3 + cell.j];
+    dV *= 1.0 / dxg[(nx + 6) + (ny + 6) + 3 + cell.k];
 #pragma unroll
     for (int v = 0; v < NV; v++) acc[v] += u[(size_t)v * ncell + idx] * dV;
   }
@@ -622,28 +653,28 @@ __global__ void __launch_bounds__(256) k_volint(const double *__restrict__ u, do
   __syncthreads();
   if (threadIdx.x < NV) {
     double r = 0.0;
-    for (int q = 0; q < (int)(blockDim.x >> 6); q++) r += red[threadIdx.x][q];
-    part[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = r;
+    for (int q = 0; q < RED_WAVES; q++) r += red[threadIdx.x][q];
+    part[(size_t)blockIdx.x * NV + threadIdx.x] = r;
   }
 }
 
 unsigned reduction_blocks(size_t n) {
-  unsigned b = nblocks(n, 256);
-  return b > 2048 ? 2048 : (b == 0 ? 1 : b);
+  unsigned b = nblocks(n, RED_THREADS);
+  return b > 512 ? 512 : (b == 0 ? 1 : b);
 }
 
 void launch_volint(const Grid &g, const double *u, double *part, unsigned nb, const double *dxg, hipStream_t st) {
-  hipLaunchKernelGGL(k_volint, dim3(nb), dim3(256), 0, st, u, part, g.n[0], g.n[1], g.n[2], dxg);
+  hipLaunchKernelGGL(k_volint, dim3(nb), dim3(RED_THREADS), 0, st, u, part, g.n[0], g.n[1], g.n[2], dxg);
 }
 
 void launch_cfl(const Grid &g, const Scheme &sc, const double *u, double *part, unsigned nb,
                 const double *dxg, double dt, hipStream_t st) {
-  hipLaunchKernelGGL(k_cfl, dim3(nb), dim3(256), 0, st, u, part, g.n[0], g.n[1], g.n[2], dxg, sc.gamma, dt);
+  hipLaunchKernelGGL(k_cfl, dim3(nb), dim3(RED_THREADS), 0, st, u, part, g.n[0], g.n[1], g.n[2], dxg, sc.gamma, dt);
 }
 
 void launch_sqdiff(const double *a, const double *b, double *part, unsigned nb, size_t n,
                    hipStream_t st) {
-  hipLaunchKernelGGL(k_sqdiff, dim3(nb), dim3(256), 0, st, a, b, part, n);
+  hipLaunchKernelGGL(k_sqdiff, dim3(nb), dim3(RED_THREADS), 0, st, a, b, part, n);
 }
 
 void launch_aos_to_soa(const Grid &g, const double *aos, double *soa, int ghosts, hipStream_t st) {
