@@ -462,12 +462,12 @@ hm_status hm_volume_integral(hm_solver *s, const double *u, double *out) {
   hm::launch_volint(s->g, u, s->part_host, nb, s->dxg, s->stream);
   if ((st = check_launch("hm_volume_integral")) != HM_OK) return st;
   HM_HIP(hipStreamSynchronize(s->stream));
-  double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  long double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // the fold of the partials adds no rounding of its own
   for (unsigned b = 0; b < nb; b++)
     for (int v = 0; v < 5; v++) sum[v] += s->part_host[(size_t)b * 5 + v];
   for (int v = 0; v < 5; v++) {
-    out[v] = sum[v];
-    if (!std::isfinite(sum[v])) return fail(HM_ERR_NONFINITE, "hm_volume_integral: state holds NaN/Inf");
+    out[v] = (double)sum[v];
+    if (!std::isfinite(out[v])) return fail(HM_ERR_NONFINITE, "hm_volume_integral: state holds NaN/Inf");
   }
   return HM_OK;
 }
@@ -482,9 +482,9 @@ hm_status hm_step_norm(hm_solver *s, const double *a, const double *b, double *n
   hm::launch_sqdiff(a, b, s->part_host, nb, n5, s->stream);
   if ((st = check_launch("hm_step_norm")) != HM_OK) return st;
   HM_HIP(hipStreamSynchronize(s->stream));
-  double sum = 0.0;
+  long double sum = 0.0;
   for (unsigned i = 0; i < nb; i++) sum += s->part_host[i];
-  *norm = std::sqrt(sum / (double)s->g.ncell);
+  *norm = std::sqrt((double)sum / (double)s->g.ncell);
   if (!std::isfinite(*norm)) return fail(HM_ERR_NONFINITE, "hm_step_norm: NaN/Inf");
   return HM_OK;
 }
@@ -861,8 +861,8 @@ static hm_status adjoint_reverse_sweep(hm_solver *s, double *lam) {
       s->tape_holds[o] = seg;
       if (overlap) {
         // a recomputation writes the solver's step buffers (primitive
-        // variables, viscous terms, right-hand side, accumulator, the last
-        // step's scratch): the second stream's next one starts after this one
+        // variables, viscous terms, right-hand side, the last step's
+        // scratch): the second stream's next one starts after this one
         HM_HIP(hipEventRecord(s->ev_start, main));
         HM_HIP(hipStreamWaitEvent(s->aux, s->ev_start, 0));
       }
@@ -944,7 +944,7 @@ hm_status hm_profile_kernels(hm_solver *s, const double *u, int reps, double *ms
     hm::launch_prims(s->g, s->sc, u, s->Q, s->stream);
     hm::launch_visc_par(s->g, s->sc, s->Q, s->par, s->dxg, s->stream);
   }
-  // the passes as stage 1 of an RK4 step runs them: the z pass reads u and
+  // the passes as RK4's second and third stage run them: the z pass reads u and
   // writes the next stage state (and Q); u is not written
   const hm::PassBuffers b = {u, s->R, s->par, s->Q, {hm::UPD_MIX, 0.0, 0.0, u, nullptr, nullptr, s->S[1]}};
   for (int d = 0; d < 3 && st == HM_OK; d++)
