@@ -26,25 +26,25 @@ sys.path.insert(0, ROOT)
 METRIC = "NS3D WENO5-RK4 FP64 cell-updates/s at 256³; adjoint/forward time ratio"
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-# algorithmic HBM bytes per cell-update of a fused 3N RK4 step (5 FP64
-# variables = 40 B per array; stage 1 reads u, writes acc and U2 = 120 B;
-# stages 2-3 read U_s, u, acc, write acc, U_{s+1} = 200 B each; stage 4
-# reads U4, acc, writes u = 120 B).  Halo re-reads, metrics and every
+# algorithmic HBM bytes per cell-update of a fused RK4 step that keeps only
+# its stage states (5 FP64 variables = 40 B per array; stage 1 reads u, writes
+# U2 = 80 B; stages 2-3 read U_s, u, write U_{s+1} = 120 B each; stage 4 reads
+# U4, U2, U3, u, writes u = 200 B).  Halo re-reads, metrics and every
 # intermediate (the rhs accumulator between passes, the viscous fluxes and
 # primitive variables) count zero.
-STEP_BYTES_PER_CELL_UPDATE = 640
+STEP_BYTES_PER_CELL_UPDATE = 520
 # one launch of a stage kernel processes one stage of every cell: its share
-# of the step's algorithmic bytes is a quarter of 640 B per cell
+# of the step's algorithmic bytes is a quarter of 520 B per cell
 STAGE_BYTES_PER_CELL = STEP_BYTES_PER_CELL_UPDATE // 4
 # operand bytes per cell one launch of each kernel reads and writes in this
 # implementation (not the algorithmic figure; reported beside it), as
 # (inviscid, viscous extra):
 #   pass_x     read U_s, write R
 #   pass_y     read U_s and R, write R
-#   pass_z     read U_s, R, u, acc; write acc, U_{s+1}   (+ read par 32 B, write Q 32 B)
+#   pass_z     read U_s, R, u; write U_{s+1} (stages 2, 3)   (+ read par 32 B, write Q 32 B)
 #   visc_par   read Q (4 primitives), write par (4 components)
 #   prims      read u, write Q
-OPERAND_BYTES = {"pass_x": (80, 0), "pass_y": (120, 0), "pass_z": (240, 64), "visc_par": (64, 0),
+OPERAND_BYTES = {"pass_x": (80, 0), "pass_y": (120, 0), "pass_z": (160, 64), "visc_par": (64, 0),
                  "prims": (72, 0)}
 
 

@@ -1155,7 +1155,7 @@ __device__ __forceinline__ void visc_mu(const double *__restrict__ lam, const do
 // them one point of the halo, whose loads are in flight during the arithmetic
 // of the plane before.  (When every plane was loaded whole, twice over the
 // tile's halo, and waited for, in segments of 16 planes on any grid: 878 us for
-// eight grids of together 2.33e6 cells against 532 us now.)
+// eight grids of together 9.3e6 cells against 532 us now.)
 struct ViscVjpShared {
   double q[2][4][VHY][VHX], m[2][4][VHY][VHX];
   double dx[VHX], dy[VHY];

@@ -576,7 +576,7 @@ static ViscParams visc_params(const Scheme &sc) {
 // block, so W blocks on 256 CUs take ceil(W/256) (p + 6) plane times.  The
 // length with the least such time is taken; a shorter one has to win 3%.  (For
 // grids that run together, total work over 256 plus half a block chose segments
-// too long: 463 us against 349 for the eight of 2.33e6 cells.)
+// too long: 463 us against 349 for the eight of 9.3e6 cells.)
 int visc_segment(int count, const int (*n)[3]) {
   constexpr int CUS = 256;
   int nmax = 0;

@@ -6,7 +6,7 @@
 //   pass x:  R = dxinv (F_{i+1/2} - F_{i-1/2})
 //   pass y:  R = R + dyinv (G_{j+1/2} - G_{j-1/2})
 //   pass z:  r = -(R + dzinv (H_{k+1/2} - H_{k-1/2})) + par,
-//            then the RK4 stage update in 3N form (or r itself for hm_rhs)
+//            then the stage's update (or r itself for hm_rhs)
 // i.e. rhs = -hyp + par of TimeRHSFunctionExplicit.c:88-93 summed in the
 // reference's order, with the hyperbolic term of HyperbolicFunction.c:75-101
 // accumulated direction by direction and the parabolic term par of
@@ -53,13 +53,17 @@
 //    cells' fluxes passes L and R unchanged (L R = I).
 //
 // FP64 issue bounds these passes: a wave64 FP64 instruction takes a SIMD 4
-// cycles, and two waves per SIMD hide the rest to about 60%.  The forms above
-// take 946 FP64 (1050 VALU) instructions per interface of the characteristic
-// JS/Roe x pass and 744 (843) of the component-wise JS/Rusanov one, where
-// weights from second and one-sided differences, projected values and
+// cycles, and two waves per SIMD keep it busy 60-67% of the time (y), three
+// 73-81% (x); the z pass at 256^3 also moves 224 B per cell, at close to the
+// rate of a copy.
+// The forms above take 946 FP64 (1050 VALU) instructions per interface of the
+// characteristic JS/Roe x pass and 744 (843) of the component-wise JS/Rusanov
+// one (915 and 1016 of the former since the reciprocals take one cubic step),
+// where weights from second and one-sided differences, projected values and
 // Roe averages formed at each interface took 1356 (1474) and 1072 (1188):
 // 256^3 RK4 step 15.55 -> 13.54 ms, 201^3 SSPRK3/YC step 5.20 -> 4.18 ms,
-// 64-member Euler ensemble 18.7 -> 15.2 ms per step.
+// 64-member Euler ensemble 18.7 -> 15.2 ms per step by that alone.  At 256^3
+// the characteristic passes now take 0.72 (x), 0.76 (y) and 1.0 ms (z).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -702,8 +706,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(x_wave
   pass_x_body<INTERP, UPW, 4, W>(k, io, blockIdx.x, sh);
 }
 
-// at most 256 registers: two waves per SIMD (the characteristic passes sit
-// at the limit, and one register more would halve the occupancy)
+// at most 256 registers: two waves per SIMD, which is what the LDS allows.
+// Three, as blocks of 6 or 12 wavefronts with 6 or 12 rows per step, are slower:
+// six wavefronts sit 2, 2, 1, 1 on the SIMDs (256^3 characteristic step 11.8 ->
+// 14.1 ms), twelve wait for each other at every barrier (y 0.76 -> 0.83 ms).
 template <int DIR, int INTERP, int UPW, int W>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) k_pass_m(PassConst k, PassIO io) {
   __shared__ MShared<4, UPW> sh;

@@ -233,8 +233,8 @@ hm_status hm_tape_info(const hm_solver *s, int *sets, int *step_level, size_t *b
  * HyperbolicFunction_GPU.cu:517-576).  Launches each kernel of one RK stage
  * `reps` times on the solver's stream with state u and stores the mean
  * duration in milliseconds, measured with HIP events on that stream:
- * ms[0..2] the fused x, y, z passes of an RK stage (the z pass in its
- * stage-1 form, which reads u and the accumulator and writes the next stage
+ * ms[0..2] the fused x, y, z passes of an RK stage (the z pass in the form of
+ * RK4's second and third stage, which reads u and writes the next stage
  * state); ms[3] the viscous-term kernel and ms[4] the primitive-variable
  * kernel that hm_rk4 runs once per call (0 if inviscid).  u is not
  * modified. */

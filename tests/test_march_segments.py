@@ -2,7 +2,7 @@
 8 cells a line on).  Lines of every remainder of the 4-row march step, from
 the longest line that stays whole to lines of several segments, over one and
 several 64-column groups: the right-hand side and one SSPRK3 step (whose z
-pass is another kernel) against the oracle."""
+pass updates the state as well) against the oracle."""
 import dataclasses
 
 import pytest
