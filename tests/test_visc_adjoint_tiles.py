@@ -1,7 +1,9 @@
 """The viscous adjoint takes the grid in tiles of 64 x 8 columns and z segments
 whose length depends on the grid: sides one below, at and one above a tile,
 grids of one and of several segments, with both cotangents of a step's
-stages, against autograd through the FP64 reference."""
+stages, against autograd through the FP64 reference.  The ghost-layer kernels
+take the ten cells at a line's ends at once from 10 cells on: sides of 9, 10
+and 11 as well."""
 import pytest
 
 torch = pytest.importorskip("torch")
@@ -10,7 +12,7 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-12
 
 
-@pytest.mark.parametrize("dims", [(64, 8, 5), (63, 7, 6), (65, 9, 7), (66, 17, 40)])
+@pytest.mark.parametrize("dims", [(64, 8, 5), (63, 7, 6), (65, 9, 7), (66, 17, 40), (10, 9, 11)])
 def test_step_vjp_at_tile_edges(dims):
     from hypar_amd.solver import NS3D
     from oracle import torch_ref as T
