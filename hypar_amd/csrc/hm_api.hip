@@ -41,7 +41,7 @@ size_t tape_slots(const TapePlan &p, int nsteps, int every) {
   return (size_t)(p.step_level ? 1 : 4) * (size_t)std::min(nsteps, p.sets * every);
 }
 // every state the tape and the reverse sweep hold: the checkpoints, the
-// sets, 4 scratch states, and 3 stage states at step level
+// sets, 4 scratch states (the sweeps use three), and 3 stage states at step level
 size_t tape_total_states(const TapePlan &p, int nsteps, int every) {
   const size_t nck = (size_t)((nsteps + every - 1) / every);
   return nck + tape_slots(p, nsteps, every) + 4 + (p.step_level ? 3 : 0);
@@ -191,16 +191,18 @@ hm_status stage_launches(hm_solver *s, const double *U, const hm::StageUpdate &u
   return check_launch("Runge-Kutta stage passes");
 }
 
-// One RK4 step of u in place through the fused direction passes (TimeRK.c:126-195
-// with the "44" tableau).  Stage s reads Sx[s-1] (u for s = 0) and writes
-// Sx[s]; the last stage writes u from u and all three.
-hm_status rk4_step(hm_solver *s, double *u, double dt, double *const Sx[3]) {
-  for (int stage = 0; stage < 4; stage++) {
+// The first nstages stages, 3 or 4, of an RK4 step of u through the fused
+// direction passes (TimeRK.c:126-195 with the "44" tableau).  Stage s reads
+// Sx[s-1] (u for s = 0) and writes Sx[s]; the fourth writes u from u and all
+// three.
+hm_status rk4_stages(hm_solver *s, double *u, double dt, double *const Sx[3], int nstages) {
+  for (int stage = 0; stage < nstages; stage++) {
     hm_status st = stage_launches(s, stage == 0 ? u : Sx[stage - 1], rk4_update(stage, u, dt, Sx));
     if (st != HM_OK) return st;
   }
   return HM_OK;
 }
+hm_status rk4_step(hm_solver *s, double *u, double dt, double *const Sx[3]) { return rk4_stages(s, u, dt, Sx, 4); }
 
 // One SSPRK3 step of u in place (TimeRK.c:126-195 with the "ssprk3" tableau,
 // written through its stage states: see StageUpdate)
@@ -625,6 +627,14 @@ static hm_status rk4_step_store(hm_solver *s, double *u, double dt, double *cons
   return rk4_step(s, u, dt, U);
 }
 
+// The stage states U1, U2, U3 of the step from u, which is only read: what the
+// adjoint needs of a step whose result is not wanted.  The fourth stage, a
+// quarter of the step, would only form u_{n+1}.
+static hm_status rk4_stage_states(hm_solver *s, const double *u, double dt, double *const U[3]) {
+  if (s->sc.Re > 0) hm::launch_prims(s->g, s->sc, u, s->Q, s->stream);
+  return rk4_stages(s, const_cast<double *>(u), dt, U, 3);
+}
+
 // Step adjoint given the stage states U[0..3] (U[0] = u_n):
 // lam_out = lam + sum_s nu_s, nu_s = J(U_s)^T mu_s,
 // mu_s = dt b_s lam + dt a_{s+1,s} nu_{s+1} (formed inside the VJP kernels);
@@ -638,7 +648,7 @@ static hm_status vjp_work(hm_solver *s, double **w) {
   return st;
 }
 
-static hm_status rk4_step_vjp(hm_solver *s, double *const U[4], double dt, const double *lam, double *lam_out) {
+static hm_status rk4_step_vjp(hm_solver *s, const double *const U[4], double dt, const double *lam, double *lam_out) {
   const size_t n5 = 5 * s->g.ncell;
   hm_status st = ensure_buffers(s->vscratch, 3, n5);
   if (st != HM_OK) return st;
@@ -685,16 +695,12 @@ hm_status hm_rk4_vjp(hm_solver *s, const double *u_n, double dt, double *lam) {
   if ((st = check_state(s, lam, "hm_rk4_vjp: lam")) != HM_OK) return st;
   const size_t n5 = 5 * s->g.ncell;
   if ((st = ensure_buffers(s->stages, 4, n5)) != HM_OK) return st;
-  double *U[4] = {s->stages[0], s->stages[1], s->stages[2], s->stages[3]};
-  HM_HIP(hipMemcpyAsync(U[0], u_n, n5 * sizeof(double), hipMemcpyDeviceToDevice, s->stream));
-  // a throw-away copy advanced through the step yields the stage states
-  if ((st = ensure_buffers(s->vscratch, 4, n5)) != HM_OK) return st;
-  double *w = s->vscratch[3];
-  HM_HIP(hipMemcpyAsync(w, u_n, n5 * sizeof(double), hipMemcpyDeviceToDevice, s->stream));
-  double *const Us[3] = {U[1], U[2], U[3]};
-  if ((st = rk4_step_store(s, w, dt, Us)) != HM_OK) return st;
-  // U[0..3] are the first tape states: a recorded trajectory no longer finds
-  // the segments there and recomputes them
+  if ((st = ensure_buffers(s->vscratch, 3, n5)) != HM_OK) return st;
+  double *const Us[3] = {s->stages[1], s->stages[2], s->stages[3]};
+  const double *const U[4] = {u_n, Us[0], Us[1], Us[2]};
+  if ((st = rk4_stage_states(s, u_n, dt, Us)) != HM_OK) return st;
+  // the stage states are the first tape states: a recorded trajectory no
+  // longer finds the segments there and recomputes them
   for (int i = 0; i < TAPE_SETS; i++) s->tape_holds[i] = -1;
   double *L = s->vscratch[2];
   if ((st = rk4_step_vjp(s, U, dt, lam, L)) != HM_OK) return st;
@@ -756,7 +762,7 @@ hm_status hm_adjoint_forward(hm_solver *s, double *u, double dt, int nsteps, int
   if ((st = fit_buffers(s->ckpt, (size_t)nck, n5)) != HM_OK) return st;
   if ((st = fit_buffers(s->stages, tape_slots(plan, nsteps, every), n5)) != HM_OK) return st;
   if ((st = fit_buffers(s->sscratch, plan.step_level ? 3 : 0, n5)) != HM_OK) return st;
-  if ((st = ensure_buffers(s->vscratch, 4, n5)) != HM_OK) return st;
+  if ((st = ensure_buffers(s->vscratch, 3, n5)) != HM_OK) return st;
   // the last `sets` segments keep their states, one in each set: the
   // reverse sweep starts on them without recomputation
   const int nkeep = (nck >= plan.sets ? nck - plan.sets : 0) * every;
@@ -801,15 +807,15 @@ static hm_status recompute_segment(hm_solver *s, int seg, int n0, int n1, double
     }
     return HM_OK;
   }
-  if ((st = ensure_buffers(s->vscratch, 4, n5)) != HM_OK) return st;
   for (int n = n0; n < n1; n++) {
     double **U = S + (size_t)4 * (n - n0);
     // U[0] of the first step is the checkpoint; later steps find u_n in
     // their slot, advanced there by the step before
     if (n == n0) HM_HIP(hipMemcpyAsync(U[0], s->ckpt[seg], n5 * sizeof(double), hipMemcpyDeviceToDevice, s->stream));
-    double *next = n + 1 < n1 ? S[(size_t)4 * (n - n0 + 1)] : s->vscratch[3];
-    HM_HIP(hipMemcpyAsync(next, U[0], n5 * sizeof(double), hipMemcpyDeviceToDevice, s->stream));
     double *const Us[3] = {U[1], U[2], U[3]};
+    if (n + 1 == n1) return rk4_stage_states(s, U[0], dt, Us);
+    double *next = S[(size_t)4 * (n - n0 + 1)];
+    HM_HIP(hipMemcpyAsync(next, U[0], n5 * sizeof(double), hipMemcpyDeviceToDevice, s->stream));
     if ((st = rk4_step_store(s, next, dt, Us)) != HM_OK) return st;
   }
   return HM_OK;
@@ -824,7 +830,7 @@ static hm_status adjoint_reverse_sweep(hm_solver *s, double *lam) {
   const size_t n5 = 5 * s->g.ncell;
   if ((st = ensure_buffers(s->stages, tape_slots(plan, N, K), n5)) != HM_OK) return st;
   if ((st = ensure_buffers(s->sscratch, plan.step_level ? 3 : 0, n5)) != HM_OK) return st;
-  if ((st = ensure_buffers(s->vscratch, 4, n5)) != HM_OK) return st;
+  if ((st = ensure_buffers(s->vscratch, 3, n5)) != HM_OK) return st;
   // With two or more stage-level sets, a second stream recomputes the
   // segment before the current one while the solver's stream runs the
   // current one's adjoint.  With one set, or at step level (whose adjoint
@@ -861,8 +867,8 @@ static hm_status adjoint_reverse_sweep(hm_solver *s, double *lam) {
       s->tape_holds[o] = seg;
       if (overlap) {
         // a recomputation writes the solver's step buffers (primitive
-        // variables, viscous terms, right-hand side, the last step's
-        // scratch): the second stream's next one starts after this one
+        // variables, viscous terms, right-hand side): the second stream's next
+        // one starts after this one
         HM_HIP(hipEventRecord(s->ev_start, main));
         HM_HIP(hipStreamWaitEvent(s->aux, s->ev_start, 0));
       }
@@ -891,11 +897,9 @@ static hm_status adjoint_reverse_sweep(hm_solver *s, double *lam) {
       double *out = cur == lam ? s->vscratch[2] : lam;
       if (plan.step_level) {
         // the step's stage states, from its starting state
-        double *w = s->vscratch[3];
-        HM_HIP(hipMemcpyAsync(w, S[n - n0], n5 * sizeof(double), hipMemcpyDeviceToDevice, main));
         double *const Us[3] = {s->sscratch[0], s->sscratch[1], s->sscratch[2]};
-        if ((st = rk4_step_store(s, w, dt, Us)) != HM_OK) return st;
-        double *const U[4] = {S[n - n0], Us[0], Us[1], Us[2]};
+        if ((st = rk4_stage_states(s, S[n - n0], dt, Us)) != HM_OK) return st;
+        const double *const U[4] = {S[n - n0], Us[0], Us[1], Us[2]};
         if ((st = rk4_step_vjp(s, U, dt, cur, out)) != HM_OK) return st;
       } else if ((st = rk4_step_vjp(s, S + (size_t)4 * (n - n0), dt, cur, out)) != HM_OK) {
         return st;
@@ -1088,11 +1092,16 @@ hm_status ens_capture(hm_ensemble *e, double *u) {
 
 // one RK4 step of all members in place on u, keeping the stage states
 // U1, U2, U3 (eager launches; the adjoint's forward and recomputation)
-hm_status ens_step_store(hm_ensemble *e, double *u, double *const U[3]) {
+hm_status ens_stages(hm_ensemble *e, double *u, double *const U[3], int nstages) {
   hipStream_t st = e->stream;
   if (e->sc.Re > 0) hm::launch_ens_prims(e->sc, e->mem_dev, e->nmem, u, e->ncell, st);
-  for (int stage = 0; stage < 4; stage++) ens_stage_launches(e, stage, u, U, st);
+  for (int stage = 0; stage < nstages; stage++) ens_stage_launches(e, stage, u, U, st);
   return check_launch("hm_ensemble: step");
+}
+hm_status ens_step_store(hm_ensemble *e, double *u, double *const U[3]) { return ens_stages(e, u, U, 4); }
+// the stage states alone; u is only read (rk4_stage_states)
+hm_status ens_stage_states(hm_ensemble *e, const double *u, double *const U[3]) {
+  return ens_stages(e, const_cast<double *>(u), U, 3);
 }
 
 hm_status ens_check(const hm_ensemble *e, const void *u, const char *name) {
@@ -1513,7 +1522,7 @@ hm_status hm_ensemble_adjoint_forward(hm_ensemble *e, double *u, int nsteps, int
   if ((st = fit_buffers(e->ckpt, (size_t)nck, n5)) != HM_OK) return st;
   if ((st = fit_buffers(e->stages, tape_slots(plan, nsteps, every), n5)) != HM_OK) return st;
   if ((st = fit_buffers(e->sscratch, plan.step_level ? 3 : 0, n5)) != HM_OK) return st;
-  if ((st = ens_buffers(e->vscratch, 4, n5)) != HM_OK) return st;
+  if ((st = ens_buffers(e->vscratch, 3, n5)) != HM_OK) return st;
   // the last `sets` segments keep their states (segment seg in set seg % sets)
   const int nkeep = (nck >= plan.sets ? nck - plan.sets : 0) * every;
   for (int n = 0; n < nsteps; n++) {
@@ -1550,7 +1559,7 @@ static hm_status ens_reverse_sweep(hm_ensemble *e, double *lam) {
   const size_t n5 = 5 * e->ncell;
   if ((st = ens_buffers(e->stages, tape_slots(plan, N, K), n5)) != HM_OK) return st;
   if ((st = ens_buffers(e->sscratch, plan.step_level ? 3 : 0, n5)) != HM_OK) return st;
-  if ((st = ens_buffers(e->vscratch, 4, n5)) != HM_OK) return st;
+  if ((st = ens_buffers(e->vscratch, 3, n5)) != HM_OK) return st;
   double *work = nullptr;
   const size_t nw = hm::ens_vjp_work_size(e->sc, e->ncell);
   if (nw) {
@@ -1592,9 +1601,13 @@ static hm_status ens_reverse_sweep(hm_ensemble *e, double *lam) {
           double **U = S + (size_t)4 * (n - n0);
           if (n == n0)
             HM_HIP(hipMemcpyAsync(U[0], e->ckpt[seg], n5 * sizeof(double), hipMemcpyDeviceToDevice, e->stream));
-          double *next = n + 1 < n1 ? S[(size_t)4 * (n - n0 + 1)] : e->vscratch[3];
-          HM_HIP(hipMemcpyAsync(next, U[0], n5 * sizeof(double), hipMemcpyDeviceToDevice, e->stream));
           double *const Us[3] = {U[1], U[2], U[3]};
+          if (n + 1 == n1) {
+            if ((st = ens_stage_states(e, U[0], Us)) != HM_OK) return st;
+            break;
+          }
+          double *next = S[(size_t)4 * (n - n0 + 1)];
+          HM_HIP(hipMemcpyAsync(next, U[0], n5 * sizeof(double), hipMemcpyDeviceToDevice, e->stream));
           if ((st = ens_step_store(e, next, Us)) != HM_OK) return st;
         }
       }
@@ -1604,10 +1617,8 @@ static hm_status ens_reverse_sweep(hm_ensemble *e, double *lam) {
       double *Ust[4];
       if (plan.step_level) {
         // the step's stage states, from its starting state
-        double *w = e->vscratch[3];
-        HM_HIP(hipMemcpyAsync(w, S[n - n0], n5 * sizeof(double), hipMemcpyDeviceToDevice, e->stream));
         double *const Us[3] = {e->sscratch[0], e->sscratch[1], e->sscratch[2]};
-        if ((st = ens_step_store(e, w, Us)) != HM_OK) return st;
+        if ((st = ens_stage_states(e, S[n - n0], Us)) != HM_OK) return st;
         Ust[0] = S[n - n0];
         for (int i = 0; i < 3; i++) Ust[i + 1] = Us[i];
       } else {
