@@ -322,10 +322,12 @@ __device__ __forceinline__ void roe_speed_vjp(const double *uL, const double *uR
   roe_avg_vjp(uL, uR, gamma, gv, gH, ubL, ubR);
 }
 
-// Euler flux along DIR of a cell's state (navierstokes3d.h:118-139)
+// Euler flux along DIR of a cell's state (navierstokes3d.h:118-139).  As in
+// the forward passes a cell without mass has no velocity: its flux enters the
+// stencils of the interfaces around it and has to be finite.
 template <int DIR>
 __device__ __forceinline__ void vjp_flux(const double *u, double gamma, double f[NV]) {
-  const double ir = nr_rcp(u[0]);
+  const double ir = u[0] == 0.0 ? 0.0 : nr_rcp(u[0]);
   const double v[3] = {u[1] * ir, u[2] * ir, u[3] * ir};
   const double P = (gamma - 1.0) * (u[4] - 0.5 * u[0] * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]));
   f[0] = u[1 + DIR];
