@@ -128,7 +128,9 @@ __device__ __forceinline__ int wrapi(int p, int n) {
 
 // Stencil of d/dx_d at the ghost position of slot s (0..3 for the positions
 // -2, -1, n, n+1): 12 times the weights of the five points from offset
-// ghost_first(slot) on (periodic copies).
+// ghost_first(slot) on (periodic copies).  The weighted values are summed
+// before the sum is scaled by dxinv/12: scaled weights are rounded, so that
+// equal values no longer cancel.
 __device__ __forceinline__ int ghost_first(int slot) { return slot == 0 ? -1 : (slot == 3 ? -3 : -2); }
 __device__ __forceinline__ double ghost_weight(int slot, int k) {
   const double lo[5] = {-3, -10, 18, -6, 1}, hi[5] = {-1, 6, -18, 10, 3}, mid[5] = {1, -8, 0, 8, -1};
@@ -260,10 +262,12 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
         for (int k = 0; k < 5; k++) {
           double r[4];
           ldq(col, q + o0 + k, r);
-          const double w = ghost_weight(slot, k) * (r12 * dza[3 + q]);
+          const double w = ghost_weight(slot, k);
 #pragma unroll
           for (int v = 0; v < 4; v++) d[v] += w * r[v];
         }
+#pragma unroll
+        for (int v = 0; v < 4; v++) d[v] *= r12 * dza[3 + q];
         ghost_flux<2>(fzq, qv, d, mu, vp);
       }
     } else {
@@ -297,10 +301,12 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
         double d[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int k = 0; k < 5; k++) {
-          const double w = ghost_weight(slot, k) * (r12 * dxa[3 + i]);
+          const double w = ghost_weight(slot, k);
 #pragma unroll
           for (int v = 0; v < 4; v++) d[v] += w * sq(v, o0 + k, 0);
         }
+#pragma unroll
+        for (int v = 0; v < 4; v++) d[v] *= r12 * dxa[3 + i];
         ghost_flux<0>(fv, qv, d, mu, vp);
 #pragma unroll
         for (int v = 0; v < 4; v++) sh.fx[buf][v][oy][ox + 2] = fv[v];
@@ -310,10 +316,12 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
         double d[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int k = 0; k < 5; k++) {
-          const double w = ghost_weight(slot, k) * (r12 * dya[3 + j]);
+          const double w = ghost_weight(slot, k);
 #pragma unroll
           for (int v = 0; v < 4; v++) d[v] += w * sq(v, 0, o0 + k);
         }
+#pragma unroll
+        for (int v = 0; v < 4; v++) d[v] *= r12 * dya[3 + j];
         ghost_flux<1>(fv, qv, d, mu, vp);
 #pragma unroll
         for (int v = 0; v < 4; v++) sh.fy[buf][v][oy + 2][ox] = fv[v];
