@@ -60,6 +60,10 @@ __device__ __forceinline__ double nr_rcp(double d) {
   return __builtin_fma(r, __builtin_fma(e, e, e), r);
 }
 
+// 1/d with a division's values where the refinement has none: infinite at
+// zero, zero at infinity, both with d's sign
+__device__ __forceinline__ double rcp_all(double d) { return __builtin_amdgcn_div_fixup(nr_rcp(d), d, 1.0); }
+
 // 1/sqrt(d), d > 0 and normal, from the hardware estimate r: with
 // e = 1 - d r^2 (at most 1.1e-7, measured), r + r e (1/2 + 3/8 e) leaves an
 // error of 5/16 e^3.
@@ -126,9 +130,11 @@ __device__ __forceinline__ double pow076(double T) {
 }
 
 // primitive variables u, v, w, T = gamma P / rho of the viscous term
-// (NavierStokes3DParabolicFunction.c:85-108)
+// (NavierStokes3DParabolicFunction.c:85-108), u, v, w zero without mass.  A
+// density that is neither zero nor infinite has to be a normal number below
+// 2^1022.
 __device__ __forceinline__ void visc_prims(const double *u, double gamma, double q[4]) {
-  const double ir = nr_rcp(u[0]);
+  const double ir = rcp_all(u[0]);
   const double iv = u[0] == 0.0 ? 0.0 : ir;
   q[0] = u[1] * iv;
   q[1] = u[2] * iv;
