@@ -197,7 +197,9 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
   const bool wantx = kind != 1 && iny && i < nx + 2, wanty = kind != 0 && inx && j < ny + 2;
   const bool regular = inx && iny && (wantx || wanty);
   const double r12 = 1.0 / 12.0;
-  const double dxi = regular ? dxa[3 + i] * r12 : 0.0, dyi = regular ? dya[3 + j] * r12 : 0.0;
+  // also for the ghost positions: read in the march, they cost the border tiles
+  // 1 us a plane (256^3: 515 us against 430, 128^3: 76 against 71)
+  const double dxi = i < nx + 2 ? dxa[3 + i] * r12 : 0.0, dyi = j < ny + 2 ? dya[3 + j] * r12 : 0.0;
 
   // a further point of the staged plane, beyond those of the block's threads:
   // rows y0-4, y0-3, y0+TY+2, y0+TY+3, columns alike, and the 16 points
@@ -306,7 +308,7 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
           for (int v = 0; v < 4; v++) d[v] += w * sq(v, o0 + k, 0);
         }
 #pragma unroll
-        for (int v = 0; v < 4; v++) d[v] *= r12 * dxa[3 + i];
+        for (int v = 0; v < 4; v++) d[v] *= dxi;
         ghost_flux<0>(fv, qv, d, mu, vp);
 #pragma unroll
         for (int v = 0; v < 4; v++) sh.fx[buf][v][oy][ox + 2] = fv[v];
@@ -321,7 +323,7 @@ __device__ __forceinline__ void visc_par_tile(const double *__restrict__ Q, doub
           for (int v = 0; v < 4; v++) d[v] += w * sq(v, 0, o0 + k);
         }
 #pragma unroll
-        for (int v = 0; v < 4; v++) d[v] *= r12 * dya[3 + j];
+        for (int v = 0; v < 4; v++) d[v] *= dyi;
         ghost_flux<1>(fv, qv, d, mu, vp);
 #pragma unroll
         for (int v = 0; v < 4; v++) sh.fy[buf][v][oy + 2][ox] = fv[v];
