@@ -1,11 +1,14 @@
-"""The reciprocals, roots and primitive variables of hm_device.h, compiled for
+"""The reciprocals, roots and the viscosity law of hm_device.h, compiled for
 the CPU with the hardware's estimates replaced by ones that are off by the
 most that was measured of them, and without contraction of a*b + c: what the
 source writes, the result may rest on, and nothing else.
 
 Bounds (u = 2^-53): a reciprocal ends in one rounding, and its e + e^2 of 4.7e-8
 adds 4.7e-8 u.  An inverse root's e = 1 - (d r) r carries the rounding of d r
-(u, halved by the series) and ends in one: 1.5 u."""
+(u, halved by the series) and ends in one: 1.5 u.  T^0.76 ends in the rounding
+of 1 + q g (u for results over 1, u/2 of 0.707 below), after q g's own (u/4,
+of 0.34) and g's (u/4 times ln 2): at most 1.7 u in all; 2 u = 2^-52 are
+allowed."""
 import ctypes
 import os
 import subprocess
@@ -51,6 +54,7 @@ void off(double x) { g_off = x; }
 void rcp(const double *x, double *y, int n) { for (int i = 0; i < n; i++) y[i] = hm::nr_rcp(x[i]); }
 void rsq(const double *x, double *y, int n) { for (int i = 0; i < n; i++) y[i] = hm::nr_rsq(x[i]); }
 void root(const double *x, double *y, int n) { for (int i = 0; i < n; i++) y[i] = hm::nr_sqrt(x[i]); }
+void pow76(const double *x, double *y, int n) { for (int i = 0; i < n; i++) y[i] = hm::pow076(x[i]); }
 void prims(const double *u, double gamma, double *q) { hm::visc_prims(u, gamma, q); }
 }
 """
@@ -103,6 +107,25 @@ def test_reciprocal_and_roots(dev):
     assert _error(dev("rsq", x), 1 / np.sqrt(X)) <= 1.51 * U
     assert _error(dev("root", x), np.sqrt(X)) <= 1.01 * U
     assert dev("root", np.zeros(1))[0] == 0.0
+
+
+@pytest.mark.parametrize("lo,hi", [(-1, 1), (-44, 44), (-1022, 1023.99), (-1074, -1022)])
+def test_viscosity_law(dev, lo, hi):
+    x = _arguments(lo, hi)
+    # both sides of the interval's ends sqrt(1/2) 2^k
+    k = np.arange(int(np.ceil(lo)) + 1, int(hi))
+    edge = np.sqrt(0.5) * np.exp2(k.astype(float))
+    x = np.concatenate([x, edge, np.nextafter(edge, np.inf), np.nextafter(edge, 0), np.exp2(k.astype(float))])
+    x = x[x > 0]
+    exact = np.exp(np.longdouble(0.76) * np.log(x.astype(np.longdouble)))
+    # the reference's own error: the logarithm's rounding, magnified by its size
+    slack = 2.0 ** -64 * 0.76 * max(abs(lo), abs(hi)) + 2.0 ** -63
+    assert _error(dev("pow76", x), exact) <= 2 * U + slack
+
+
+def test_viscosity_law_special_values(dev):
+    y = dev("pow76", [0.0, np.inf, np.nan, -1.0, -np.inf])
+    assert y[0] == 0.0 and y[1] == np.inf and np.isnan(y[2:]).all()
 
 
 @pytest.mark.parametrize("rho", [1.0, -2.0, 0.0, -0.0, np.inf, -np.inf, np.nan])
