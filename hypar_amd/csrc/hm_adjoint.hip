@@ -113,8 +113,9 @@ __device__ __forceinline__ LineSlot line_slot(size_t item, int n, size_t nlines)
 //            through the mapping and the JS normalisation
 //  * optimal (no_limiting): the constant weights 0.1, 0.6, 0.3
 // (sum a_k h_k = 0 takes the cross terms out.)  One reciprocal of
-// A l_1 l_2 l_3 gives 1/A and the 1/(l_k A); the mapped weights take a second
-// one for the mapping.
+// A l_1 l_2 l_3 gives 1/A and 1/(l_1 l_2 l_3); the mapped weights take a second
+// one for the mapping.  The reciprocal itself, l^-7 or l^-9, is as large as
+// 1e280 for an epsilon of 1e-40 in a uniform region: ob multiplies 1/A alone.
 struct W5Side {
   double c, w1, w2, w3, g1, g2, g3, gt;
 };
@@ -176,16 +177,18 @@ __device__ __forceinline__ W5Side w5_side(double l1, double l2, double l3, doubl
   const double q = nr_rcp(A * P);
   const double inv = q * P;
   r.c = (a1 * p1 + a2 * p2 + a3 * p3) * inv;
-  const double oi = ob * inv, k = (-2.0 * ob) * (W == WENO_JS ? q : t2 * q);
+  const double oi = ob * inv, k = -2.0 * (W == WENO_JS ? q * A : t2 * (q * A));
   r.w1 = a1 * oi;
   r.w2 = a2 * oi;
   r.w3 = a3 * oi;
-  const double h1 = s1 * (p1 - r.c), h2 = s2 * (p2 - 6.0 * r.c), h3 = s3 * (p3 - 3.0 * r.c);
+  const double h1 = (W == WENO_JS ? r.w1 : s1 * oi) * (p1 - r.c);
+  const double h2 = (W == WENO_JS ? r.w2 : s2 * oi) * (p2 - 6.0 * r.c);
+  const double h3 = (W == WENO_JS ? r.w3 : s3 * oi) * (p3 - 3.0 * r.c);
   r.g1 = k * (q1 * h1);
   r.g2 = k * (q2 * h2);
   r.g3 = k * (q3 * h3);
   if (W != WENO_JS) {
-    const double gt = 2.0 * t * oi * (h1 + h2 + h3);
+    const double gt = 2.0 * t * (h1 + h2 + h3);
     if (W == WENO_Z) {
       r.g3 += gt;
       r.g1 -= gt;
