@@ -40,8 +40,10 @@ namespace {
 size_t tape_slots(const TapePlan &p, int nsteps, int every) {
   return (size_t)(p.step_level ? 1 : 4) * (size_t)std::min(nsteps, p.sets * every);
 }
-// every state the tape and the reverse sweep hold: the checkpoints, the
-// sets, 4 scratch states (the sweeps use three), and 3 stage states at step level
+// The states a schedule is charged for: the checkpoints, the sets, 4 scratch
+// states, and 3 stage states at step level.  The sweeps hold three of the
+// scratch states; the fourth stays in the count so that a budget in bytes
+// keeps the schedule it was set for.
 size_t tape_total_states(const TapePlan &p, int nsteps, int every) {
   const size_t nck = (size_t)((nsteps + every - 1) / every);
   return nck + tape_slots(p, nsteps, every) + 4 + (p.step_level ? 3 : 0);
@@ -694,9 +696,9 @@ hm_status hm_rk4_vjp(hm_solver *s, const double *u_n, double dt, double *lam) {
   if ((st = check_state(s, u_n, "hm_rk4_vjp: u_n")) != HM_OK) return st;
   if ((st = check_state(s, lam, "hm_rk4_vjp: lam")) != HM_OK) return st;
   const size_t n5 = 5 * s->g.ncell;
-  if ((st = ensure_buffers(s->stages, 4, n5)) != HM_OK) return st;
+  if ((st = ensure_buffers(s->stages, 3, n5)) != HM_OK) return st;
   if ((st = ensure_buffers(s->vscratch, 3, n5)) != HM_OK) return st;
-  double *const Us[3] = {s->stages[1], s->stages[2], s->stages[3]};
+  double *const Us[3] = {s->stages[0], s->stages[1], s->stages[2]};
   const double *const U[4] = {u_n, Us[0], Us[1], Us[2]};
   if ((st = rk4_stage_states(s, u_n, dt, Us)) != HM_OK) return st;
   // the stage states are the first tape states: a recorded trajectory no

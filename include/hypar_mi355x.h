@@ -220,12 +220,13 @@ hm_status hm_adjoint_forward(hm_solver *s, double *u, double dt, int nsteps, int
  * the same, bit for bit, whatever the schedule. */
 hm_status hm_adjoint_reverse(hm_solver *s, double *lam);
 /* Bytes the tape of the next forward sweep may hold: checkpoints, sets,
- * scratch states and viscous work space.  0 (the default) takes the
+ * four scratch states and viscous work space.  0 (the default) takes the
  * device's free memory plus what the tape already holds, less a reserve of
  * 2 GiB or 2% of the device, whichever is larger. */
 hm_status hm_set_tape_budget(hm_solver *s, size_t bytes);
 /* The schedule of the recorded trajectory: sets (1..3), step_level (0/1)
- * and the bytes it holds (any pointer may be NULL). */
+ * and the bytes it is charged for, the least budget that gives it (any
+ * pointer may be NULL).  The sweeps hold one scratch state less. */
 hm_status hm_tape_info(const hm_solver *s, int *sets, int *step_level, size_t *bytes);
 
 /* Kernel timing for roofline reports (no counterpart in the reference; the
