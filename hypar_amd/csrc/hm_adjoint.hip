@@ -450,12 +450,7 @@ __device__ __forceinline__ void l_row_vjp(const RoeAdj &s, double gm1, int k, co
   }
 }
 
-// |l| with Harten's entropy fix, as the passes form it, and its derivative
-__device__ __forceinline__ double vjp_harten(double l) {
-  const double delta = 0.000001, delta2 = delta * delta, inv2d = 0.5 / delta;
-  const double al = fabs(l);
-  return al < delta ? (l * l + delta2) * inv2d : al;
-}
+// derivative of harten
 __device__ __forceinline__ double harten_d(double l) {
   const double delta = 0.000001;
   return fmin(fmax(l * (1.0 / delta), -1.0), 1.0);
@@ -632,14 +627,14 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
     const double sumb = g[0] + s.v[0] * g[1] + s.v[1] * g[2] + s.v[2] * g[3];
     const double difb = g[1 + DIR] + s.vn * eb;
     double lg[5];  // (R^T lambda_F)_k |lambda_k|
-    lg[0] = (sumb + s.ek * eb) * vjp_harten(s.vn);
-    lg[1] = (sumb + s.h0 * eb - s.a * difb) * vjp_harten(s.vn - s.a);
-    lg[2] = (sumb + s.h0 * eb + s.a * difb) * vjp_harten(s.vn + s.a);
+    lg[0] = (sumb + s.ek * eb) * harten(s.vn);
+    lg[1] = (sumb + s.h0 * eb - s.a * difb) * harten(s.vn - s.a);
+    lg[2] = (sumb + s.h0 * eb + s.a * difb) * harten(s.vn + s.a);
     if (DIR == 0) { lg[3] = -g[2] - s.v[1] * eb; lg[4] = g[3] + s.v[2] * eb; }
     else if (DIR == 1) { lg[3] = g[1] + s.v[0] * eb; lg[4] = -g[3] - s.v[2] * eb; }
     else { lg[3] = -g[1] - s.v[0] * eb; lg[4] = g[2] + s.v[1] * eb; }
-    lg[3] *= vjp_harten(s.vn);
-    lg[4] *= vjp_harten(s.vn);
+    lg[3] *= harten(s.vn);
+    lg[4] *= harten(s.vn);
 #pragma unroll 1
     for (int k = 0; k < 5; k++) {
       double row[NV];
@@ -724,9 +719,9 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
       if (DIR == 0) { lgk[3] = -ld[2] - s.v[1] * eb; lgk[4] = ld[3] + s.v[2] * eb; }
       else if (DIR == 1) { lgk[3] = ld[1] + s.v[0] * eb; lgk[4] = -ld[3] - s.v[2] * eb; }
       else { lgk[3] = -ld[1] - s.v[0] * eb; lgk[4] = ld[2] + s.v[1] * eb; }
-      lam_k[0] = lam_k[3] = lam_k[4] = vjp_harten(s.vn);
-      lam_k[1] = vjp_harten(s.vn - s.a);
-      lam_k[2] = vjp_harten(s.vn + s.a);
+      lam_k[0] = lam_k[3] = lam_k[4] = harten(s.vn);
+      lam_k[1] = harten(s.vn - s.a);
+      lam_k[2] = harten(s.vn + s.a);
       double gv[3] = {0, 0, 0}, ab = 0.0;
       // rows of L: p_k = l_k . du, g_k = |lambda_k| p_k
 #pragma unroll
@@ -886,9 +881,9 @@ __device__ __forceinline__ void rhs_vjp_char_line(
       lk[0] = lk[1] = lk[2] = fmax(m01, m12);
       sel = m01 >= m12 ? (aL >= aR ? 0 : 1) : (aR >= aA ? 1 : 2);
     } else {
-      lk[0] = vjp_harten(s.vn);
-      lk[1] = vjp_harten(s.vn - s.a);
-      lk[2] = vjp_harten(s.vn + s.a);
+      lk[0] = harten(s.vn);
+      lk[1] = harten(s.vn - s.a);
+      lk[2] = harten(s.vn + s.a);
     }
   }
   // the two shear fields (one row of L each: CA or CB times (x_J - v_J x_0))
@@ -1602,12 +1597,6 @@ __global__ void __launch_bounds__(64) k_ens_visc_vjp_ghost(EnsVjp a, const unsig
                            M.dt * a.B, QB, M.n[0], M.n[1], M.n[2], M.dxg, a.vc, item - first[m]);
 }
 
-// y = a*x + b*y
-__global__ void k_axpby(const double *__restrict__ x, double a, double *__restrict__ y, double b, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    y[i] = (a == 0.0 ? 0.0 : a * x[i]) + b * y[i];  // x unread when a == 0
-}
-
 // ---------------------------------------------------------------------------
 bool vjp_supported(const Grid &g, const Scheme &sc) {
   const int lmax = sc.interp == INTERP_CHAR ? VJP_CHAR_LINE_MAX : VJP_LINE_MAX;
@@ -1702,27 +1691,8 @@ void launch_rhs_vjp(const Grid &g, const Scheme &sc, const double *u, const doub
   launch_vjp_dir<0>(g, sc, u, lam, nu_in, ca, cb, nu, L, last, dxg, st, QB, GB);
 }
 
-// With W blocks on 256 CUs, one block each, and p + 2 plane times a block, the
-// length p with the least ceil(W/256) (p + 2); a shorter one has to win 3%.
-int visc_vjp_segment(int count, const int (*n)[3]) {
-  constexpr int CUS = 256;
-  int nmax = 0;
-  for (int m = 0; m < count; m++) nmax = n[m][2] > nmax ? n[m][2] : nmax;
-  int best = nmax;
-  double tbest = 0.0;
-  for (int parts = 1; parts <= nmax; parts++) {
-    const int p = (nmax + parts - 1) / parts;
-    if (parts > 1 && p == (nmax + parts - 2) / (parts - 1)) continue;
-    double blocks = 0.0;
-    for (int m = 0; m < count; m++) blocks += visc_tiles(n[m][0], n[m][1], n[m][2], p);
-    const double t = ceil(blocks / CUS) * (p + 2);
-    if (parts == 1 || t < 0.97 * tbest) {
-      tbest = t;
-      best = p;
-    }
-  }
-  return best;
-}
+// a segment of p planes takes p + 2 plane times
+int visc_vjp_segment(int count, const int (*n)[3]) { return plane_segment(count, n, 2, visc_tiles); }
 
 bool ens_vjp_supported(const Scheme &sc, const int nmax[3]) {
   Grid g;
@@ -1801,12 +1771,6 @@ void launch_ens_rhs_vjp(const Scheme &sc, const EnsVjpPlan &p, const double *u, 
   // the x lines add the viscous share (QB, GB of a.work) before their own
   a.mode = L ? (set_L ? VJP_ADD_LSET : VJP_ADD_L) : VJP_ADD;
   launch_ens_vjp_dir<0>(sc, p, a, st);
-}
-
-void launch_axpby(const double *x, double a, double *y, double b, size_t n, hipStream_t st) {
-  size_t nb = (n + 255) / 256;
-  if (nb > 65536) nb = 65536;
-  hipLaunchKernelGGL(k_axpby, dim3((unsigned)nb), dim3(256), 0, st, x, a, y, b, n);
 }
 
 }  // namespace hm

@@ -263,6 +263,13 @@ __device__ __forceinline__ double harten_abs(double l) {
   return al < delta ? (l * l + delta2) / (2 * delta) : al;
 }
 
+// the same without the division, in the fused passes and the adjoint
+__device__ __forceinline__ double harten(double l) {
+  const double delta = 0.000001, delta2 = delta * delta, inv2d = 0.5 / delta;
+  const double al = fabs(l);
+  return al < delta ? (l * l + delta2) * inv2d : al;
+}
+
 // WENO5 interpolant.  (m3,m2,m1,p1,p2) are the stencil values the
 // smoothness indicators use, (g3,g2,g1,q1,q2) the values that are
 // interpolated (they differ only for the solution, whose weights come from u

@@ -146,6 +146,31 @@ __host__ __device__ inline unsigned par_tiles(int nx, int ny, int nz, int pks) {
 // segment length of the viscous-term kernel over `count` grids that run together
 int visc_segment(int count, const int (*n)[3]);
 
+// The z segment of these two kernels, whose blocks march p planes of a tile in
+// p + start plane times, one block on each of the 256 CUs: W blocks take
+// ceil(W/256) (p + start).  The length with the least such time is taken; a
+// shorter one has to win 3%.
+template <class Tiles>
+int plane_segment(int count, const int (*n)[3], int start, Tiles tiles) {
+  constexpr int CUS = 256;
+  int nmax = 0;
+  for (int m = 0; m < count; m++) nmax = n[m][2] > nmax ? n[m][2] : nmax;
+  int best = nmax;
+  double tbest = 0.0;
+  for (int parts = 1; parts <= nmax; parts++) {
+    const int p = (nmax + parts - 1) / parts;
+    if (parts > 1 && p == (nmax + parts - 2) / (parts - 1)) continue;
+    double blocks = 0.0;
+    for (int m = 0; m < count; m++) blocks += tiles(n[m][0], n[m][1], n[m][2], p);
+    const double t = std::ceil(blocks / CUS) * (p + start);
+    if (parts == 1 || t < 0.97 * tbest) {
+      tbest = t;
+      best = p;
+    }
+  }
+  return best;
+}
+
 // batched ensemble passes (hm_pass.hip): members of one scheme
 struct EnsMember {
   int n[3];
@@ -203,7 +228,6 @@ size_t vjp_work_size(const Grid &g, const Scheme &sc);
 void launch_rhs_vjp(const Grid &g, const Scheme &sc, const double *u, const double *lam, const double *nu_in,
                     double ca, double cb, double *nu, double *L, bool set_L, const double *dxg, double *work,
                     hipStream_t st);
-void launch_axpby(const double *x, double a, double *y, double b, size_t n, hipStream_t st);
 
 // the same for all members of an ensemble at once: member m's stage
 // coefficients are dt_m*A and dt_m*B; lines0[d] lists each member's first

@@ -582,30 +582,10 @@ static ViscParams visc_params(const Scheme &sc) {
   return vp;
 }
 
-// A segment of p planes marches p + 4 and starts on 4 more, and a CU holds one
-// block, so W blocks on 256 CUs take ceil(W/256) (p + 6) plane times.  The
-// length with the least such time is taken; a shorter one has to win 3%.  (For
-// grids that run together, total work over 256 plus half a block chose segments
-// too long: 463 us against 349 for the eight of 9.3e6 cells.)
-int visc_segment(int count, const int (*n)[3]) {
-  constexpr int CUS = 256;
-  int nmax = 0;
-  for (int m = 0; m < count; m++) nmax = n[m][2] > nmax ? n[m][2] : nmax;
-  int best = nmax;
-  double tbest = 0.0;
-  for (int parts = 1; parts <= nmax; parts++) {
-    const int p = (nmax + parts - 1) / parts;
-    if (parts > 1 && p == (nmax + parts - 2) / (parts - 1)) continue;
-    double blocks = 0.0;
-    for (int m = 0; m < count; m++) blocks += par_tiles(n[m][0], n[m][1], n[m][2], p);
-    const double t = ceil(blocks / CUS) * (p + 6);
-    if (parts == 1 || t < 0.97 * tbest) {
-      tbest = t;
-      best = p;
-    }
-  }
-  return best;
-}
+// A segment of p planes marches p + 4 and starts on 4 more.  (For grids that run
+// together, total work over 256 plus half a block chose segments too long: 463
+// us against 349 for the eight of 9.3e6 cells.)
+int visc_segment(int count, const int (*n)[3]) { return plane_segment(count, n, 6, par_tiles); }
 
 void launch_visc_par(const Grid &g, const Scheme &sc, const double *Q, double *par, const double *dxg,
                      hipStream_t st) {

@@ -85,7 +85,7 @@ struct PassConst {
   int n[3];
   int seg;    // cells per march segment along the pass direction (y, z passes)
   size_t ncell;
-  double gamma, gm1, inv_gm1, eps34;  // eps34 = 3/4 of the WENO epsilon
+  double gamma, gm1, eps34;  // eps34 = 3/4 of the WENO epsilon
   const double *dxg;  // ghosted dxinv x|y|z
 };
 
@@ -223,13 +223,6 @@ __device__ __forceinline__ RoeState roe_state(const LQ &L, const RQ &R, const Pa
   s.Lm0 = gek + avn;
   s.L40 = gek - avn;
   return s;
-}
-
-// |lambda| with Harten's entropy fix, delta = 1e-6 (NavierStokes3DUpwind.c:95-101)
-__device__ __forceinline__ double harten(double l) {
-  const double delta = 0.000001, delta2 = delta * delta, inv2d = 0.5 / delta;
-  const double al = fabs(l);
-  return al < delta ? (l * l + delta2) * inv2d : al;
 }
 
 // rows 0, d, 4 of L x (u-a wave in row d = DIR+1)
@@ -724,7 +717,7 @@ struct EnsArgs {
   int nmem;
   const unsigned *item0;   // first work item of each member, nmem + 1 entries
   unsigned nitems;
-  double gamma, gm1, inv_gm1, eps34;  // eps34 = 3/4 of the WENO epsilon
+  double gamma, gm1, eps34;  // eps34 = 3/4 of the WENO epsilon
   const double *U;         // stage states of all members (member m at 5*off)
   double *R;
   StageUpdate upd;
@@ -749,7 +742,6 @@ __device__ __forceinline__ void ens_setup(const EnsArgs &a, int m, int dir, Pass
   k.ncell = M.ncell;
   k.gamma = a.gamma;
   k.gm1 = a.gm1;
-  k.inv_gm1 = a.inv_gm1;
   k.eps34 = a.eps34;
   k.dxg = M.dxg;
   const size_t o = 5 * M.off;
@@ -1003,7 +995,6 @@ void launch_pass(const Grid &g, const Scheme &sc, int dir, const PassBuffers &b,
   k.ncell = g.ncell;
   k.gamma = sc.gamma;
   k.gm1 = sc.gamma - 1.0;
-  k.inv_gm1 = 1.0 / (sc.gamma - 1.0);
   k.eps34 = 0.75 * sc.eps;
   k.dxg = dxg;
   io.U = b.U;
@@ -1062,7 +1053,6 @@ void launch_ens_pass(const Scheme &sc, int dir, int shape, const EnsMember *mem,
   a.nitems = nitems;
   a.gamma = sc.gamma;
   a.gm1 = sc.gamma - 1.0;
-  a.inv_gm1 = 1.0 / (sc.gamma - 1.0);
   a.eps34 = 0.75 * sc.eps;
   a.U = U;
   a.R = R;
@@ -1123,7 +1113,6 @@ void launch_ens_stage(const Scheme &sc, int rows, const EnsMember *mem, int nmem
   a.nitems = 0;
   a.gamma = sc.gamma;
   a.gm1 = sc.gamma - 1.0;
-  a.inv_gm1 = 1.0 / (sc.gamma - 1.0);
   a.eps34 = 0.75 * sc.eps;
   a.U = U;
   a.R = R;
