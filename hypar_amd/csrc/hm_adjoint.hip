@@ -12,10 +12,10 @@
 // The interface-flux VJP spreads g over the 6 stencil cells as a flux-adjoint
 // part (later multiplied by the flux Jacobian transpose of the cell, once per
 // cell) and a direct solution-adjoint part (WENO of the solution, Rusanov
-// speed).  One workgroup owns one grid line along the direction: the line's
-// states, fluxes and modified energies live in LDS (sized to the line), each
-// thread is one interface, and each thread writes its six stencil
-// contributions to LDS slots that the owning cell then sums in a fixed
+// speed).  One workgroup owns one or several whole grid lines along the
+// direction: the lines' states and fluxes live in LDS (sized to the lines),
+// each thread is one interface, and each thread writes its six stencil
+// contributions to an LDS record that the owning cells then sum in a fixed
 // order, so the result is deterministic.
 //
 // Within an RK4 step the stage adjoint mu_s = dt b_s lam + dt a_{s+1,s}
@@ -456,12 +456,14 @@ __device__ __forceinline__ double harten_d(double l) {
   return fmin(fmax(l * (1.0 / delta), -1.0), 1.0);
 }
 
-// nu (+)= (d rhs_DIR / d u)^T mu along one direction, one workgroup per line,
-// with mu = cb*lam + ca*nu_in (nu_in may be null).  mode VJP_WRITE stores,
-// VJP_ADD accumulates into nu, VJP_ADD_L accumulates into nu and adds the
-// finished nu into L, VJP_ADD_LSET sets L = lam + the finished nu.  LDS (dynamic, 23 doubles per cell of the line):
-// state [5][n], cell flux [5][n], modified energy [n], stencil
-// contributions of the flux and solution adjoints [6][n] each.
+// nu (+)= (d rhs_DIR / d u)^T mu along one direction, one workgroup per group
+// of lines (LineSlot), with mu = cb*lam + ca*nu_in (nu_in may be null).  mode
+// VJP_WRITE stores, VJP_ADD accumulates into nu, VJP_ADD_L accumulates into nu
+// and adds the finished nu into L, VJP_ADD_LSET sets L = lam + the finished nu.
+// LDS (dynamic, VJP_LDS = 24 doubles per cell of the lines): a record per cell
+// of its state [5] and flux [5], and one per interface of the stencil
+// contributions of the flux and solution adjoints [6] each, both of odd length
+// so that neighbouring records start in other banks.
 enum { VJP_WRITE = 0, VJP_ADD = 1, VJP_ADD_L = 2, VJP_ADD_LSET = 3 };
 
 // state, lam and (when given) nu_in of cell c, every load issued before any
@@ -803,7 +805,7 @@ __device__ __forceinline__ void rhs_vjp_line(const double *__restrict__ u, const
 // and I.
 // longest grid line a characteristic adjoint workgroup holds: at 512 cells
 // the block is 8 wavefronts, two per SIMD (the register budget the
-// two-wave hint sets for every block size) and 88 KiB of LDS
+// two-wave hint sets for every block size) and 120 KiB of LDS
 constexpr int VJP_CHAR_LINE_MAX = 512;
 constexpr int VJP_CHAR_CS = VJP_CS;
 constexpr int VJP_CHAR_EV = 3;                    // variables exchanged at once
@@ -811,7 +813,7 @@ constexpr int VJP_CHAR_ES = 6 * VJP_CHAR_EV + 1;  // doubles per exchange record
 constexpr int VJP_CHAR_LDS = VJP_CHAR_CS + VJP_CHAR_ES;  // doubles of LDS per cell of the line
 
 // nu (+)= (d hyp_DIR-part of rhs / d u)^T mu along one direction for the
-// characteristic scheme; one workgroup per line, one thread per interface,
+// characteristic scheme; one workgroup per group of lines, one thread per interface,
 // modes as k_rhs_vjp.  LDS (dynamic, VJP_CHAR_LDS doubles per cell of the
 // line), laid out as for the component-wise scheme: a record per cell of its
 // state and flux and one per interface of its adjoints on the six stencil
@@ -1364,7 +1366,7 @@ __device__ __forceinline__ void visc_vjp_ghost_line(const double *__restrict__ Q
       else if (slot == 2) fb[k] = d4w(1) * a[3][k] + d4w(2) * a[2][k];
       else fb[k] = d4w(2) * a[3][k];
     }
-    // the forward evaluation at this ghost position (k_visc_ghost_x, k_visc_ghost)
+    // the forward evaluation at this ghost position (ghost_flux of hm_kernels.hip)
     const double(*w)[4] = f + slot;  // positions gp-3 .. gp+3
     // stencil weights over positions gp-3 .. gp+3
     double w7[7] = {0, 0, 0, 0, 0, 0, 0};

@@ -69,8 +69,9 @@ __device__ __forceinline__ void visc_flux(double fv[4], const QT &q, const doubl
 }
 
 // Viscous term of the right-hand side (NavierStokes3DParabolicFunction.c:50-325):
-//   par = (dxinv Dx FVx + dyinv Dy FVy) + dzinv Dz FVz,
-// summed in the reference's order, with FVd the viscous flux along d of the
+//   par = dxinv Dx FVx + dyinv Dy FVy + dzinv Dz FVz,
+// the x and y terms added to each other first and the z fluxes one by one
+// around their sum (the reference adds the three terms), with FVd the viscous flux along d of the
 // primitive variables (u, v, w, T) and their gradient (4th-order central
 // differences with periodic neighbours, scaled by the point's dxinv;
 // FirstDerivativeFourthOrder.c:103) and Dd the same central difference of
@@ -108,8 +109,10 @@ __device__ __forceinline__ void visc_flux(double fv[4], const QT &q, const doubl
 //
 // LDS bandwidth (3000 cycles per plane and CU) and vector issue (3200) bound
 // it, hardly overlapped because the block's wavefronts go through them
-// together: 3.3 us per plane.  Tiles of 16 x 16, two blocks per CU, took 603 us
-// at 256^3, this one 437 us; a form with 512 threads, two barriers per plane
+// together: 3.3 us per plane.  Its 11 wavefronts allow a thread 168 registers,
+// of which k_visc_par spills 4 and k_ens_visc 2 (20 and 12 B of scratch a lane).
+// Tiles of 16 x 16, two blocks per CU, took 603 us
+// at 256^3, this one 430 us; a form with 512 threads, two barriers per plane
 // and the halo points evaluated after the columns by some of the threads, 497
 // us (before that, with log and exp, a flux ring and a buffer of x + y parts,
 // 670 us).  64^3 takes 21 us, 16x12x20 14 us (87 and 91 us with segments of 16
@@ -394,7 +397,7 @@ struct EnsViscArgs {
 
 __global__ void __launch_bounds__(PAR_THREADS) k_ens_visc(EnsViscArgs a) {
   __shared__ ViscParShared<PTX, PTY> sh;
-  const unsigned item = blockIdx.x;  // one block per item (a loop over items spills 8 B per lane)
+  const unsigned item = blockIdx.x;  // one block per item (a loop over items spills 13 registers)
   if (item >= a.nitems) return;
   int lo = 0, hi = a.nmem - 1;
   while (lo < hi) {

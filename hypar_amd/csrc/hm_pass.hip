@@ -12,16 +12,17 @@
 // accumulated direction by direction and the parabolic term par of
 // NavierStokes3DParabolicFunction.c:50-325.
 //
-// Each pass stages the cells of its pencils in LDS once, evaluates every
-// cell's flux and modified energy once, computes the interface fluxes
-// (WENO5-JS, component-wise or characteristic, with Roe or Rusanov
+// Each pass stages the cells of its pencils in LDS once, evaluates what
+// depends on one cell alone (its flux, the factors of the Roe average) once,
+// computes the interface fluxes (WENO5, component-wise or characteristic, with Roe or Rusanov
 // upwinding) from LDS, and differences them in LDS: interface fluxes never
 // reach HBM.
 //  * x pass: one wavefront per x-line, chunks of 64 interfaces along x.
 //  * y, z passes: a block owns 64 consecutive columns (x fastest) of the
 //    plane across y (z), which may span several x-rows of that plane, and
 //    marches along y (z) four rows per step, with a 9-row ring of cell data
-//    and a 5-row ring of interface fluxes in LDS.
+//    and a 5-row ring of interface fluxes in LDS; on grids with few columns
+//    it marches one segment of its lines (march_segments).
 // Output of cell c needs the interfaces c-1/2 and c+1/2; a step emits the
 // cells one row (lane) behind its interfaces, and the last cell of a line,
 // whose right interface is the periodic image of interface 0, is emitted
@@ -63,7 +64,7 @@
 // Roe averages formed at each interface took 1356 (1474) and 1072 (1188):
 // 256^3 RK4 step 15.55 -> 13.54 ms, 201^3 SSPRK3/YC step 5.20 -> 4.18 ms,
 // 64-member Euler ensemble 18.7 -> 15.2 ms per step by that alone.  At 256^3
-// the characteristic passes now take 0.72 (x), 0.76 (y) and 1.0 ms (z).
+// the characteristic passes now take 0.72 (x), 0.76 (y) and 0.92 ms (z).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1147,7 +1148,11 @@ void launch_ens_stage(const Scheme &sc, int rows, const EnsMember *mem, int nmem
 // a segment reach n + 5).  Measured, y / z pass, whole lines -> segments: 64^3
 // component-wise 45 / 60 -> 17 / 20 us, 128^3 106 / 159 -> 86 / 125 us, 201^3
 // 403 / 539 -> 340 / 456 us; 256^3 stays whole (666 / 866 us, 656-672 / 866-900
-// in segments of 47 to 127 cells).
+// in segments of 47 to 127 cells).  The formula's shape and its factors are a
+// fit to such sweeps, not derived.  MR is the four-row blocks'; the two-row
+// blocks an ensemble can choose take the same segments (64 members of 32 to 64
+// a side, step with whole lines -> segments and the present arithmetic: four
+// rows 4.58 -> 3.55 ms, two rows 5.40 -> 4.17 ms).
 void march_segments(int count, const int (*n)[3], int dir, int *seg) {
   constexpr int MR = 4, CUS = 256;
   int nmax = 0;
